@@ -701,10 +701,14 @@ struct Pipeline {
   DBuf<int32_t> pos, cnt, off, list, inv;
   // the fused evaluation's static data per window (patches up to 4 x 4):
   // rows w_0 v_0[k] and singular pairs (s_0, s_1) per (frame, bucket place)
+  // (FP64; the FP32 overlap-add of strips takes the patches by column, their
+  // leading vectors by patch and two figures per window, see launch_bins)
   DBuf<char> w0b, s01b;
-  uint32_t static_frames = 0;  // frame subset of the static data (0: every frame; see launch_static_rows)
+  DBuf<int2> recs;
+  DBuf<float> w0, v0;
+  DBuf<uint32_t> wstat;
   DBuf<int16_t> jobs_d;
-  uint32_t max_jobs = 0, gather_blocks = 0;
+  uint32_t max_jobs = 0, risk_blocks = 0;
   // learned-lambda probe: the patch subsample (sh_s: p_sel = its size) with
   // its three-variant factors and divergence factors, per-slot lambdas
   bool probe_on = false;
@@ -830,11 +834,16 @@ struct Pipeline {
     if (median) b += 8ull * sh.vol;                      // w64
     b += es * sh.vol * nvar;                             // SVD input variants
     b += 4ull * sh.nw * sh.p_all;                        // pos
-    b += 8ull * sh.nw * ((size_t)sh.n1 * sh.n1 + 1);     // bucket counts + offsets
-    b += 8ull * sh.nw * sh.p_sel;                        // bucket lists + inverse
+    if (strip_overlap(sh))
+      b += 4ull * sh.nw * (column_bins(sh) + 1);         // column offsets
+    else
+      b += 8ull * sh.nw * ((size_t)sh.n1 * sh.n1 + 1);   // bucket counts + offsets
+    b += 8ull * sh.nw * sh.p_sel;                        // bucket lists + inverse, or the column records
     b += 8ull * sh.vol * (optimize ? 2 : 1);             // 1/W, delta2/W
     b += es * sh.nw * (size_t)sh.p_sel * (fused_eval(sh) ? 1 : sh.m);  // B0 (or dr)
-    if (fused_eval(sh)) {
+    if (strip_overlap(sh)) {
+      b += 4ull * sh.p_sel * (sh.m + sh.nw);                 // leading vectors
+    } else if (fused_eval(sh)) {
       b += singular_pair_bytes(sh);                          // static singular pairs
       b += es * sh.nw * (size_t)sh.p_sel * sh.m;             // static rows
     }
@@ -885,23 +894,31 @@ struct Pipeline {
     const size_t es = sh.fp64 ? 8 : 4;
     uvar.alloc((size_t)NB * sh.vol * nvar * es);
     pos.alloc((size_t)NB * sh.nw * sh.p_all);
-    const size_t npos = (size_t)sh.n1 * sh.n1;
-    cnt.alloc((size_t)NB * sh.nw * npos);
-    off.alloc((size_t)NB * sh.nw * (npos + 1));
-    list.alloc((size_t)NB * sh.nw * sh.p_sel);
-    inv.alloc((size_t)NB * sh.nw * sh.p_sel);
+    if (strip_overlap(sh)) {
+      off.alloc((size_t)NB * sh.nw * (column_bins(sh) + 1));
+      recs.alloc((size_t)NB * sh.nw * sh.p_sel);
+      w0.alloc((size_t)NB * sh.p_sel * sh.m);
+      v0.alloc((size_t)NB * sh.nw * sh.p_sel);
+      wstat.alloc(2 * (size_t)NB);
+    } else {
+      const size_t npos = (size_t)sh.n1 * sh.n1;
+      cnt.alloc((size_t)NB * sh.nw * npos);
+      off.alloc((size_t)NB * sh.nw * (npos + 1));
+      list.alloc((size_t)NB * sh.nw * sh.p_sel);
+      inv.alloc((size_t)NB * sh.nw * sh.p_sel);
+    }
     invw.alloc((size_t)NB * sh.vol);
     if (optimize) dw.alloc((size_t)NB * sh.vol * (sh.fp64 ? sizeof(double) : sizeof(float)));
     B0.alloc((size_t)NB * sh.nw * sh.p_sel * (fused_eval(sh) ? 1 : sh.m) * es);
-    if (fused_eval(sh)) {
+    if (fused_eval(sh) && !strip_overlap(sh)) {
       w0b.alloc((size_t)NB * sh.nw * sh.p_sel * sh.m * es);
       s01b.alloc((size_t)NB * singular_pair_bytes(sh));
     }
     factors.alloc((size_t)NB * nvar * sh.p_sel * sh.fstride * es);
     if (optimize) divq.alloc((size_t)NB * nvar * sh.p_sel * 2 * ((sh.nw + 3) & ~3u) * es);
-    gather_blocks = pgsvt::gather_blocks(sh, 0);
+    risk_blocks = frame_blocks(0);
     partial.alloc((size_t)NB * eval_blocks(sh, 3));
-    partial_b.alloc((size_t)NB * gather_blocks * 5);
+    partial_b.alloc((size_t)NB * risk_blocks * 5);
     sums.alloc((size_t)NB * 6);
     partial_k.alloc((size_t)NB * eval_blocks(sh, 3));
     kept_d.alloc(NB);
@@ -951,8 +968,16 @@ struct Pipeline {
       });
     }
     prof->run("buckets_weights", (double)nb * sh.nw * sh.p_sel, [&] {
-      hipchk(launch_buckets(pos.p, sel_d.p, nb, sh, cnt.p, off.p, list.p, inv.p, s), "buckets");
-      hipchk(launch_weights(off.p, d2.p, nb, sh, d2neg, d2pos, invw.p, optimize ? dw.p : nullptr, s), "weights");
+      if (strip_overlap(sh)) {
+        hipchk(launch_fill32(wstat.p, 2 * (size_t)nb, 0, s), "clear window figures");
+        hipchk(launch_bins(pos.p, sel_d.p, nb, sh, off.p, recs.p, s), "bins");
+        hipchk(launch_cover(off.p, recs.p, d2.p, nb, sh, d2neg, d2pos, invw.p, optimize ? (float*)dw.p : nullptr,
+                            wstat.p, s),
+               "cover");
+      } else {
+        hipchk(launch_buckets(pos.p, sel_d.p, nb, sh, cnt.p, off.p, list.p, inv.p, s), "buckets");
+        hipchk(launch_weights(off.p, d2.p, nb, sh, d2neg, d2pos, invw.p, optimize ? dw.p : nullptr, s), "weights");
+      }
     });
     // units: matrices decomposed
     prof->run("svd_jacobi", (double)nb * nvar_run * sh.p_sel, [&] {
@@ -961,12 +986,15 @@ struct Pipeline {
                         stats.p, s, svd_mapping),
              "svd");
     });
-    if (fused_eval(sh)) {
+    if (strip_overlap(sh)) {
+      // units: patches
+      prof->run("leading_vectors", (double)nb * sh.p_sel, [&] {
+        hipchk(launch_lead((const float*)factors.p, nb, nvar, sh, w0.p, v0.p, wstat.p, s), "leading vectors");
+      });
+    } else if (fused_eval(sh)) {
       // units: bucket places (patch x frame) of the static rows and pairs
-      const uint32_t nf = (static_frames && static_frames < sh.nw) ? static_frames + 1 : sh.nw;
-      prof->run("static_rows", (double)nb * nf * sh.p_sel, [&] {
-        hipchk(launch_static_rows(factors.p, inv.p, meta_d.p, nb, nvar, sh, w0b.p, s01b.p, s, static_frames),
-               "static rows");
+      prof->run("static_rows", (double)nb * sh.nw * sh.p_sel, [&] {
+        hipchk(launch_static_rows(factors.p, inv.p, nb, nvar, sh, w0b.p, s01b.p, s), "static rows");
       });
     }
     if (optimize && nvar_run == 3) {
@@ -977,8 +1005,24 @@ struct Pipeline {
     }
   }
 
-  // what the gather reads (see GatherSrc)
-  GatherSrc gather_src() const {
+  // overlap-add of the slots listed in wl (device) after their evaluation
+  // (modes and nk as launch_gather; slot_lam: their lambdas, or null for
+  // the windows' own)
+  void overlap(const uint32_t* wl, uint32_t na, int mode, double* out, double* part, const double* slot_lam = nullptr,
+               uint32_t nk = 0) {
+    if (strip_overlap(sh)) {
+      OverlapSrc o;
+      o.factors = (const float*)factors.p;
+      o.dr = (const float*)B0.p;
+      o.w0 = w0.p;
+      o.v0 = v0.p;
+      o.recs = recs.p;
+      o.off = off.p;
+      o.wstat = wstat.p;
+      o.nvar_stored = nvar;
+      hipchk(launch_overlap(o, invw.p, u64.p, meta_d.p, wl, na, sh, mode, out, part, s, nk), "overlap-add");
+      return;
+    }
     GatherSrc g;
     g.B0 = B0.p;
     g.factors = factors.p;
@@ -988,7 +1032,12 @@ struct Pipeline {
     g.list = list.p;
     g.nvar_stored = nvar;
     g.exp_w = p.exponential_weighting;
-    return g;
+    g.slot_lam = slot_lam;
+    hipchk(launch_gather(g, off.p, invw.p, u64.p, meta_d.p, wl, na, sh, mode, out, part, s, nk), "gather");
+  }
+  // partial sums an overlap-add of mode 0 writes per slot
+  uint32_t frame_blocks(uint32_t nk) const {
+    return strip_overlap(sh) ? overlap_blocks(sh, 0, nk) : pgsvt::gather_blocks(sh, 0, nk);
   }
 
   // one lambda evaluation of the slots listed in wl (device), their lambdas
@@ -1039,7 +1088,7 @@ struct Pipeline {
                    const std::vector<uint32_t>& wins, const std::vector<double>& lam, std::vector<double>& risk) {
     const uint32_t nb = (uint32_t)ms.size(), nslot = 3 * (uint32_t)wins.size();
     const uint32_t nk = gather_frames(sh, kProbeFrames);
-    const uint32_t gblk = pgsvt::gather_blocks(sh, 0, nk), eblk = eval_blocks(sh_s, 3);
+    const uint32_t gblk = frame_blocks(nk), eblk = eval_blocks(sh_s, 3);
     const double fk = (double)sh.nw / nk, fp = (double)sh.p_sel / sh_s.p_sel;
     hipchk(hipMemcpyAsync(meta_d.p, ms.data(), nb * sizeof(WinMeta), hipMemcpyHostToDevice, s), "H2D meta");
     risk.assign(nslot, 0.0);
@@ -1051,10 +1100,7 @@ struct Pipeline {
       hipchk(hipMemcpyAsync(lam_s.p, lam.data() + c0, na * 8, hipMemcpyHostToDevice, s), "H2D probe lambdas");
       prof->run("probe_eval", (double)na * sh.vol, [&] {
         evaluate(wl_s.p, na, 1, lam_s.p, nullptr, nullptr);
-        GatherSrc gs = gather_src();
-        gs.slot_lam = lam_s.p;
-        hipchk(launch_gather(gs, off.p, invw.p, u64.p, meta_d.p, wl_s.p, na, sh, 0, nullptr, partial_b.p, s, nk),
-               "probe gather");
+        overlap(wl_s.p, na, 0, nullptr, partial_b.p, lam_s.p, nk);
         hipchk(launch_round_prep(factors_s.p, divq_s.p, meta_d.p, wl_s.p, na, 3, sh_s, p.exponential_weighting,
                                  lam_s.p, nullptr, partial_s.p, nullptr, s),
                "probe divergence");
@@ -1109,10 +1155,8 @@ struct Pipeline {
         "search_eval", (double)na * sh.vol, "eval_reconstruct", (double)na * 3 * sh.p_sel,
         [&] { evaluate(wl_d.p, na, 3, nullptr, partial.p, count ? partial_k.p : nullptr); }, "gather_risk",
         (double)na * sh.vol, [&] {
-          hipchk(launch_gather(gather_src(), off.p, invw.p, u64.p, meta_d.p, wl_d.p, na, sh, 0, nullptr, partial_b.p,
-                               s),
-                 "gather");
-          hipchk(launch_risk_reduce(partial.p, eval_blocks(sh, 3), partial_b.p, gather_blocks, na, sums.p, s,
+          overlap(wl_d.p, na, 0, nullptr, partial_b.p);
+          hipchk(launch_risk_reduce(partial.p, eval_blocks(sh, 3), partial_b.p, risk_blocks, na, sums.p, s,
                                     count ? partial_k.p : nullptr, count ? kept_d.p : nullptr),
                  "reduce");
         });
@@ -1139,8 +1183,7 @@ struct Pipeline {
     hipchk(hipMemcpyAsync(wl_d.p, lst.data(), nb * sizeof(uint32_t), hipMemcpyHostToDevice, s), "H2D list");
     prof->run("final_frame", (double)nb * sh.p_sel, [&] {
       evaluate(wl_d.p, nb, 1, nullptr, nullptr, nullptr);
-      hipchk(launch_gather(gather_src(), off.p, invw.p, u64.p, meta_d.p, wl_d.p, nb, sh, 1, Yout, nullptr, s),
-             "gather final");
+      overlap(wl_d.p, nb, 1, Yout, nullptr);
     });
     hipchk(hipStreamSynchronize(s), "finish sync");
     prof->flush();
@@ -1870,21 +1913,15 @@ int run_core(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf, co
         for (uint32_t c0 = 0; c0 < slots; c0 += C) {
           const uint32_t na = std::min(C, slots - c0);
           P.evaluate(wl_g.p + c0, na, 3, lam_g.p + c0, P.partial.p, nullptr);
-          GatherSrc gs = P.gather_src();
-          gs.slot_lam = lam_g.p + c0;
-          hipchk(launch_gather(gs, P.off.p, P.invw.p, P.u64.p, P.meta_d.p, wl_g.p + c0, na, P.sh, 0, nullptr,
-                               P.partial_b.p, P.s),
-                 "grid gather");
-          hipchk(launch_risk_reduce(P.partial.p, eval_blocks(P.sh, 3), P.partial_b.p, P.gather_blocks, na,
+          P.overlap(wl_g.p + c0, na, 0, nullptr, P.partial_b.p, lam_g.p + c0);
+          hipchk(launch_risk_reduce(P.partial.p, eval_blocks(P.sh, 3), P.partial_b.p, P.risk_blocks, na,
                                     sums_g.p + (size_t)c0 * 6, P.s),
                  "grid reduce");
         }
         hipchk(launch_grid_select(sums_g.p, noise_g.p, nb, G, OoN, P.eps2, lam_g.p, P.meta_d.p, risk_g.p, P.s),
                "grid select");
         P.evaluate(P.wl_d.p, nb, 1, nullptr, nullptr, nullptr);
-        hipchk(launch_gather(P.gather_src(), P.off.p, P.invw.p, P.u64.p, P.meta_d.p, P.wl_d.p, nb, P.sh, 1, P.Yout,
-                             nullptr, P.s),
-               "gather final");
+        P.overlap(P.wl_d.p, nb, 1, P.Yout, nullptr);
         const hipError_t ce = hipStreamEndCapture(P.s, &graph);
         P.prof->suspended = false;
         hipchk(ce, "end capture");
@@ -1904,9 +1941,6 @@ int run_core(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf, co
       }
       continue;
     }
-    // the learned path gathers only the probe's frames and the output
-    // frames: the static data of those frames suffice
-    P.static_frames = learned ? (probe ? gather_frames(P.sh, kProbeFrames) : 1u) : 0u;
     P.decompose(ms, learned ? 1 : P.nvar);
     if (probe) P.decompose_probe(nb);
     std::vector<WindowPrep> prep(nb);
@@ -2032,7 +2066,6 @@ int run_core(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf, co
         mf.push_back(ms[b]);
         pf.push_back(prep[b]);
       }
-      P.static_frames = 0;  // the search gathers every frame
       P.decompose(mf, 3);
       hipchk(hipStreamSynchronize(P.s), "fallback decompose sync");
       // SBPLX from the probe's estimate of the minimum, steps of the size of
@@ -2161,7 +2194,8 @@ int run_noalloc(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf,
   const uint32_t sr = (g.Nw + 3) & ~3u;
   sh.fstride = factor_stride(g.Nw, sh.m);
   const size_t npos = (size_t)sh.n1 * sh.n1, vol = sh.vol;
-  const uint32_t max_jobs = 2 * g.Nw, eblk = eval_blocks(sh, 3), gblk = pgsvt::gather_blocks(sh, 0);
+  const uint32_t max_jobs = 2 * g.Nw, eblk = eval_blocks(sh, 3);
+  const uint32_t gblk = strip_overlap(sh) ? overlap_blocks(sh, 0) : pgsvt::gather_blocks(sh, 0);
   const double vP = 0.5 + 0.5 * 1. / std::sqrt(1. * 1. + 4), vQ = 1 - vP;
   const double d2neg = -1 * std::sqrt(vQ / vP), d2pos = std::sqrt(vP / vQ), eps2 = 1e-2;
   // the layout: per call, then the window being processed
@@ -2171,11 +2205,17 @@ int run_noalloc(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf,
     double *fmax, *sums, *Xw, *Zw, *u64, *w64, *invw, *partial, *partial_b;
     WinMeta* meta;
     int16_t* jobs;
-    float *uvar, *dw, *B0, *factors, *divq, *w0;
+    float *uvar, *dw, *B0, *factors, *divq, *w0, *v0;
     int32_t *pos, *cnt, *off, *list, *inv;
-    char* s01;
+    int2* recs;
+    uint32_t* wstat;
   } L{};
-  auto carve = [&](Carve& c) {
+  // stated: the layout with position buckets and rows per bucket place
+  // (patches up to 4 x 4), by whose size the shapes this entry point takes
+  // are stated; the present one is smaller, and a shape is neither refused
+  // nor taken anew when a layout shrinks
+  auto carve = [&](Carve& c, bool stated) {
+    const bool strips = strip_overlap(sh) && !stated;
     L.d2 = optimize ? c.take<uint8_t>(vol) : nullptr;
     L.sel = c.take<uint32_t>(sh.p_sel);
     L.wl = c.take<uint32_t>(1);
@@ -2190,29 +2230,39 @@ int run_noalloc(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf,
     L.w64 = median ? c.take<double>(vol) : nullptr;
     L.uvar = c.take<float>((size_t)nvar * vol);
     L.pos = c.take<int32_t>((size_t)g.Nw * sh.p_all);
-    L.cnt = c.take<int32_t>((size_t)g.Nw * npos);
-    L.off = c.take<int32_t>((size_t)g.Nw * (npos + 1));
-    L.list = c.take<int32_t>((size_t)g.Nw * sh.p_sel);
-    L.inv = c.take<int32_t>((size_t)g.Nw * sh.p_sel);
+    if (strips) {
+      L.off = c.take<int32_t>((size_t)g.Nw * (column_bins(sh) + 1));
+      L.recs = c.take<int2>((size_t)g.Nw * sh.p_sel);
+      L.w0 = c.take<float>((size_t)sh.p_sel * sh.m);
+      L.v0 = c.take<float>((size_t)g.Nw * sh.p_sel);
+      L.wstat = c.take<uint32_t>(2);
+    } else {
+      L.cnt = c.take<int32_t>((size_t)g.Nw * npos);
+      L.off = c.take<int32_t>((size_t)g.Nw * (npos + 1));
+      L.list = c.take<int32_t>((size_t)g.Nw * sh.p_sel);
+      L.inv = c.take<int32_t>((size_t)g.Nw * sh.p_sel);
+    }
     L.invw = c.take<double>(vol);
     L.dw = optimize ? c.take<float>(vol) : nullptr;
     L.B0 = c.take<float>((size_t)g.Nw * sh.p_sel * (fused_eval(sh) ? 1 : sh.m));
-    L.s01 = fused_eval(sh) ? c.take<char>(singular_pair_bytes(sh)) : nullptr;
-    L.w0 = fused_eval(sh) ? c.take<float>((size_t)g.Nw * sh.p_sel * sh.m) : nullptr;
+    if (fused_eval(sh) && !strips) {
+      c.take<char>(singular_pair_bytes(sh));
+      c.take<float>((size_t)g.Nw * sh.p_sel * sh.m);
+    }
     L.factors = c.take<float>((size_t)nvar * sh.p_sel * sh.fstride);
     L.divq = optimize ? c.take<float>((size_t)nvar * sh.p_sel * 2 * sr) : nullptr;
     L.partial = c.take<double>(eblk);
     L.partial_b = c.take<double>((size_t)gblk * 5);
   };
   Carve count;
-  carve(count);
+  carve(count, true);
   if (count.used > kNoAllocScratch)
     return fail(PGSVT_E_ARG, "this shape needs " + std::to_string(count.used) + " bytes of device scratch per window; "
                              "the entry point without allocation has " + std::to_string(kNoAllocScratch));
   std::lock_guard<std::mutex> lock(g_scratch_mu);
   Carve at;
   at.base = scratch_address();
-  carve(at);
+  carve(at, false);
 
   const size_t dsz = dtype_size(dtype);
   const uint64_t seed = seed_of(p);
@@ -2225,15 +2275,29 @@ int run_noalloc(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf,
   hipchk(hipMemcpyAsync(L.wl, &zero, sizeof zero, hipMemcpyHostToDevice, s), "H2D list");
   if (optimize) hipchk(launch_delta2((int64_t)seed, vol, L.d2, s), "delta2");
   hipchk(hipStreamSynchronize(s), "setup sync");  // the host vectors above are local
-  GatherSrc gsrc;
-  gsrc.B0 = L.B0;
-  gsrc.factors = L.factors;
-  gsrc.dr = L.B0;
-  gsrc.S01 = L.s01;
-  gsrc.exp_w = p.exponential_weighting;
-  gsrc.W0 = L.w0;
-  gsrc.list = L.list;
-  gsrc.nvar_stored = nvar;
+  auto overlap = [&](int mode, double* out, double* part) {
+    if (strip_overlap(sh)) {
+      OverlapSrc o;
+      o.factors = L.factors;
+      o.dr = L.B0;
+      o.w0 = L.w0;
+      o.v0 = L.v0;
+      o.recs = L.recs;
+      o.off = L.off;
+      o.wstat = L.wstat;
+      o.nvar_stored = nvar;
+      hipchk(launch_overlap(o, L.invw, L.u64, L.meta, L.wl, 1, sh, mode, out, part, s), "overlap-add");
+      return;
+    }
+    GatherSrc g;
+    g.B0 = L.B0;
+    g.factors = L.factors;
+    g.dr = L.B0;
+    g.exp_w = p.exponential_weighting;
+    g.list = L.list;
+    g.nvar_stored = nvar;
+    hipchk(launch_gather(g, L.off, L.invw, L.u64, L.meta, L.wl, 1, sh, mode, out, part, s), "gather");
+  };
   std::vector<double> fmax(2 * g.Nw), sums(6), hw;
   int status = 0;
   std::string warn;
@@ -2270,13 +2334,19 @@ int run_noalloc(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf,
     hipchk(launch_fill_ref(L.meta, 1, sh, L.pos, s), "fill_ref");
     if (p.motion_estimation)
       hipchk(launch_arps(median ? L.w64 : L.u64, L.jobs, max_jobs, 1, sh, (int)p.motion_window, L.pos, s), "arps");
-    hipchk(launch_buckets(L.pos, L.sel, 1, sh, L.cnt, L.off, L.list, L.inv, s), "buckets");
-    hipchk(launch_weights(L.off, L.d2, 1, sh, d2neg, d2pos, L.invw, L.dw, s), "weights");
+    if (strip_overlap(sh)) {
+      hipchk(launch_fill32(L.wstat, 2, 0, s), "clear window figures");
+      hipchk(launch_bins(L.pos, L.sel, 1, sh, L.off, L.recs, s), "bins");
+      hipchk(launch_cover(L.off, L.recs, L.d2, 1, sh, d2neg, d2pos, L.invw, L.dw, L.wstat, s), "cover");
+    } else {
+      hipchk(launch_buckets(L.pos, L.sel, 1, sh, L.cnt, L.off, L.list, L.inv, s), "buckets");
+      hipchk(launch_weights(L.off, L.d2, 1, sh, d2neg, d2pos, L.invw, L.dw, s), "weights");
+    }
     hipchk(launch_fill32(L.stats, 1, 0, s), "clear stats");
     hipchk(launch_svd(L.uvar, L.pos, L.sel, 1, nvar, nvar, sh, L.factors, 30, 1e-6, L.stats, s,
                       g_svd_mapping.load() == 1 ? 1 : 0),
            "svd");
-    if (fused_eval(sh)) hipchk(launch_static_rows(L.factors, L.inv, L.meta, 1, nvar, sh, L.w0, L.s01, s), "static rows");
+    if (strip_overlap(sh)) hipchk(launch_lead(L.factors, 1, nvar, sh, L.w0, L.v0, L.wstat, s), "leading vectors");
     if (optimize) hipchk(launch_divq(L.factors, L.pos, L.sel, L.dw, 1, nvar, sh, L.divq, s), "divergence factors");
     double alpha = alpha0, mu = mu0, sigma = sigma0, lambda = lambda0;
     if (optimize) {
@@ -2313,7 +2383,7 @@ int run_noalloc(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf,
           hipchk(launch_evaluation(sh, L.factors, L.divq, L.meta, L.wl, 1, nvar, 3, p.exponential_weighting, L.inv,
                                    L.B0, L.partial, nullptr, nullptr, s),
                  "eval");
-          hipchk(launch_gather(gsrc, L.off, L.invw, L.u64, L.meta, L.wl, 1, sh, 0, nullptr, L.partial_b, s), "gather");
+          overlap(0, nullptr, L.partial_b);
           hipchk(launch_risk_reduce(L.partial, eblk, L.partial_b, gblk, 1, L.sums, s), "reduce");
           hipchk(hipMemcpyAsync(sums.data(), L.sums, 6 * sizeof(double), hipMemcpyDeviceToHost, s), "D2H sums");
           hipchk(hipStreamSynchronize(s), "risk sync");
@@ -2339,7 +2409,7 @@ int run_noalloc(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf,
     hipchk(launch_evaluation(sh, L.factors, nullptr, L.meta, L.wl, 1, nvar, 1, p.exponential_weighting, L.inv, L.B0,
                              nullptr, nullptr, nullptr, s),
            "eval final");
-    hipchk(launch_gather(gsrc, L.off, L.invw, L.u64, L.meta, L.wl, 1, sh, 1, Y, nullptr, s), "gather final");
+    overlap(1, Y, nullptr);
     hipchk(hipStreamSynchronize(s), "window sync");  // m and jobs are reused by the next window
     est[t + (size_t)nf * 0] = lambda;
     est[t + (size_t)nf * 1] = alpha;
@@ -2635,9 +2705,7 @@ int pgsvt_window_reconstruct(const void* X, int dtype, uint32_t n_rows, uint32_t
     DBuf<double> out;
     out.alloc(P.sh.vol);
     P.evaluate(P.wl_d.p, 1, 1, nullptr, nullptr, nullptr);
-    hipchk(launch_gather(P.gather_src(), P.off.p, P.invw.p, P.u64.p, P.meta_d.p, P.wl_d.p, 1, P.sh, 2, out.p,
-                         nullptr, P.s),
-           "gather");
+    P.overlap(P.wl_d.p, 1, 2, out.p, nullptr);
     hipchk(hipMemcpyAsync(vol, out.p, out.bytes(), hipMemcpyDeviceToHost, P.s), "D2H vol");
     hipchk(hipStreamSynchronize(P.s), "sync");
     return 0;

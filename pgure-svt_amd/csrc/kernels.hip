@@ -692,29 +692,23 @@ __global__ __launch_bounds__(256) void k_svd(const T* __restrict__ u32, const in
   }
 }
 
-// Static data of the fused evaluation (patches up to 4 x 4), from the U
+// Static data of the fused evaluation (patches up to 4 x 4 in FP64), from the U
 // variant's factors once the SVD is done: at the patch's bucket place
 // j_k = place[b][k][p] of every frame k, its rank-0 row w_0 v_0[k] into W0
 // [nb][nw][p_sel][m] and its two largest singular values (s_0, s_1) into
 // S01 [nb][nw][p_sel][2].  4 lanes per (patch, frame), frames fastest, so
 // a patch's 15 rows read its w_0 from one cache line and each row is one
-// line-sized store.  (Inside k_svd these stores would cost it a wave per
-// SIMD: its epilogue already holds X, 1/s^2 and the ranks.)  nk = 0: every
-// frame; nk > 0: only the frames a gather reads with that frame subset
-// (i (nw - 1) / (nk - 1), i < nk) and the window's output frame (mode 1).
+// line-sized store.
 template <int BS, class T>
 __global__ __launch_bounds__(256) void k_static_rows(const T* __restrict__ factors, const int32_t* __restrict__ place,
-                                                     const WinMeta* __restrict__ meta, uint32_t nvar_stored,
-                                                     uint32_t p_sel, uint32_t nw, uint32_t nk, uint32_t fstride,
-                                                     T* __restrict__ W0, T* __restrict__ S01) {
+                                                     uint32_t nvar_stored, uint32_t p_sel, uint32_t nw,
+                                                     uint32_t fstride, T* __restrict__ W0, T* __restrict__ S01) {
   constexpr int M = BS * BS, QL = (M + 3) / 4;  // row elements per lane
   const uint32_t b = blockIdx.y;
   const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t sub = t % 4, row = t / 4;
-  const uint32_t nf = nk ? nk + 1 : nw;  // frames written per patch
-  const uint32_t p = row / nf, i = row % nf;
+  const uint32_t p = row / nw, k = row % nw;
   if (p >= p_sel) return;
-  const uint32_t k = !nk ? i : (i == nk ? meta[b].ref : (nk > 1 ? i * (nw - 1) / (nk - 1) : nw / 2));
   const uint32_t SR = (nw + 3) & ~3u;
   const T* F = factors + ((size_t)b * nvar_stored * p_sel + p) * fstride;  // the U variant
   const T* FW = F + (size_t)nw * SR;
@@ -1284,15 +1278,13 @@ __global__ __launch_bounds__(256) void k_divq(const T* __restrict__ factors, con
 // The reconstruction of a patch is B = sum_r d_r w_r v_r^T (src/svt.hpp:
 // 135-146 with src/utils.hpp:96-106), d_r = g(s_r)/s_r, w_r = X v_r = s_r u_r;
 // factors are sorted by descending s and g(s)/s grows with s, so the kept
-// ranks (d_r > 0) are a prefix.  The gather forms d_0 and whether rank 1 is
-// kept itself, from the window's static singular pairs (s_0, s_1) that
-// k_svd writes at every bucket place; this thread writes, for a patch that
-// keeps rank 1, the factors d_r of its further kept ranks to dr
-// [slot][p][r], r >= 1, followed by a 0 when fewer than n ranks are kept.
-// The gather forms the patch's rows from d_0 and the static rows (w_0 v_0[k]
-// at every bucket place, written by k_svd) and, for further ranks, from dr
-// and w_r, v_r of the factors, as it stages them, so the reconstruction
-// itself is never written.  With PGURE (qdiv set) the thread also adds the
+// ranks (d_r > 0) are a prefix.  FP32: the thread writes them to dr
+// [slot][r][p], d_0 negative when rank 1 is kept too, followed by a 0 when
+// fewer than n are kept; the overlap-add forms the rows from them and the
+// leading vectors and factors.  FP64: the gather forms d_0 and whether rank
+// 1 is kept itself, from the static singular pairs at every bucket place;
+// the thread writes the further kept ranks to dr [slot][p][r], r >= 1.
+// Either way the reconstruction itself is never written.  With PGURE (qdiv set) the thread also adds the
 // patch's divergence sum sum_r (d1_r q1_r - 2 d0_r q0_r + d2_r q2_r)
 // (src/pgure.hpp:136, see k_divq) to the FP64 partial of its block.  The
 // singular values and divergence factors come from the rank-major planes of
@@ -1321,20 +1313,31 @@ __global__ __launch_bounds__(256) void k_round_prep(const T* __restrict__ factor
     return qdiv ? qdiv[(((size_t)b * nvar_stored + v) * 2 * SR + r) * p_sel + pa] : FW[n * M + r];
   };
   auto qval = [&](int v, int r) -> T { return qdiv[(((size_t)b * nvar_stored + v) * 2 * SR + SR + r) * p_sel + pa]; };
+  // FP32: one plane per rank, d_0 (negative where rank 1 is kept too) among
+  // them, for the overlap-add, which reads them by patch; FP64: by patch
+  constexpr bool PLANES = sizeof(T) == 4;
+  auto dr_at = [&](int r) -> size_t {
+    return PLANES ? ((size_t)slot * nw + r) * p_sel + p : ((size_t)slot * p_sel + p) * nw + r;
+  };
   double s4 = 0.0;
   int kr = 0;  // kept ranks of the evaluated variants (profiling)
   const int nvar_run = qdiv ? 3 : 1;
   for (int v = 0; v < nvar_run && valid; ++v) {
     const T s0 = sval(v, 0);
+    T first = T(0);
     int r = 0;
     for (; r < n; ++r) {
       const T sr = (r == 0) ? s0 : sval(v, r);
       const T d = shrink_factor(sr, s0, lam, exp_w);
       if (!(d > T(0))) break;
       if (qdiv) s4 = fma((v == 0 ? -2.0 : 1.0) * (double)d, (double)qval(v, r), s4);
-      if (v == 0 && dr && r > 0) dr[((size_t)slot * p_sel + p) * nw + r] = d;
+      if (r == 0) first = d;
+      if (v == 0 && dr && r > 0) dr[dr_at(r)] = d;
     }
-    if (v == 0 && dr && r > 1 && r < n) dr[((size_t)slot * p_sel + p) * nw + r] = T(0);  // end of the kept ranks
+    if (v == 0 && dr) {
+      if (r > 1 && r < n) dr[dr_at(r)] = T(0);  // end of the kept ranks
+      if (PLANES) dr[dr_at(0)] = r > 1 ? -first : first;
+    }
     kr += r;
   }
   if (!qdiv && !kept) return;  // uniform over the launch
@@ -1460,7 +1463,8 @@ __global__ __launch_bounds__(256) void k_gather_direct(const T* __restrict__ B0,
         ((sm[threadIdx.x][0] + sm[threadIdx.x][1]) + sm[threadIdx.x][2]) + sm[threadIdx.x][3];
 }
 
-// Tiled gather for patches up to 4 x 4, fused with the reconstruction.  A
+// Tiled gather for patches up to 4 x 4 in FP64 (FP32: overlap.hip), fused
+// with the reconstruction.  A
 // block covers a tile of TR x TC voxels of one frame k; the patches that can
 // cover the tile sit in one contiguous bucket range per patch column.  The
 // block forms those patches' rows for frame k, B[q][k] = d_0 (w_0[q] v_0[k])
@@ -1481,8 +1485,6 @@ __global__ __launch_bounds__(256) void k_gather_direct(const T* __restrict__ B0,
 //   mode 0: risk sums per block: sum Uhat^2, sum Uhat, sum Uhat U, sum U, sum U^2
 //   mode 1: final frame: Y(:,:,out) = uMax * Uhat(:,:,ref)
 //   mode 2: whole window volume of slot 0 into out
-// 5 waves per SIMD for the FP32 4 x 4 instance (at most 96 VGPRs): its
-// latency-bound staging needs the waves more than the registers
 // voxel tile of one gather block (rows x columns of a frame); 256 voxels.
 // 32 x 8: 32 voxels of a column are contiguous in the column-major frame
 // (16 x 16 stages fewer halo rows but measured 10 % slower)
@@ -1490,12 +1492,7 @@ constexpr int kTileRows = 32, kTileCols = 8;
 static_assert(kTileRows * kTileCols == 256, "one voxel per thread");
 
 template <int BS, class T>
-constexpr int gather_min_waves() {
-  return (BS == 4 && sizeof(T) == 4) ? 5 : 1;
-}
-
-template <int BS, class T>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(gather_min_waves<BS, T>()))) void k_gather_tile(
+__global__ __launch_bounds__(256) void k_gather_tile(
     const T* __restrict__ factors, const T* __restrict__ dr, const T* __restrict__ S01, const T* __restrict__ W0,
     const int32_t* __restrict__ list, const int32_t* __restrict__ off, const double* __restrict__ invw,
     const double* __restrict__ u64, const WinMeta* __restrict__ meta, const uint32_t* __restrict__ wl,
@@ -1593,17 +1590,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(gather_min_
     int32_t ids[NS];
     ST w0[NS];
     T s0[NS], s1[NS];
-    // 4 x 4 patches in FP32: the 4 lanes of a row are one quad; lanes 0, 2
-    // and 3 of the quad load the row's patch index, s_0 and s_1 (the loads
-    // in flight hold one register per row instead of three).  After the
-    // wait the slots go in pairs (s, s + 1): lanes 2 and 3 form d_0 =
-    // shrink(s_0, s_0) and shrink(s_1, s_0) of the first row, lanes 0 and 1
-    // those of the second (its s_0, s_1 moved down by DPP), in the same
-    // instructions, and the quad shares the index and the factors by DPP
-    // broadcasts.
-    constexpr bool QUAD = (QW == 4 && sizeof(T) == 4);
-    uint32_t sc[NS];
-    const int sub = (int)threadIdx.x & 3;
 #pragma unroll
     for (int sl = 0; sl < NS; ++sl) {
       const int R = lr0 + RPI * sl;
@@ -1619,50 +1605,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(gather_min_
       }
       const int32_t j = use ? sT[lc * NRW] + (R - base) : 0;
       w0[sl] = *reinterpret_cast<const ST*>(W0k + (size_t)j * M + q);
-      if constexpr (QUAD) {
-        const void* a = sub == 0 ? (const void*)(Lk + j) : (const void*)(Sk + 2 * (size_t)j + (sub - 2));
-        sc[sl] = (use && sub != 1) ? *reinterpret_cast<const uint32_t*>(a) : (sub == 0 ? 0xffffffffu : 0u);
-      } else {
-        ids[sl] = use ? Lk[j] : -1;
-        s0[sl] = Sk[2 * (size_t)j];
-        s1[sl] = Sk[2 * (size_t)j + 1];
-      }
+      ids[sl] = use ? Lk[j] : -1;
+      s0[sl] = Sk[2 * (size_t)j];
+      s1[sl] = Sk[2 * (size_t)j + 1];
     }
-    T dn0 = T(0), dn1 = T(0);  // the second row's factors of a pair (QUAD)
 #pragma unroll
     for (int sl = 0; sl < NS; ++sl) {
       {
-        T d0, d1;
-        if constexpr (QUAD) {  // every lane of the quad is active here
-          const int x = (int)sc[sl];
-          ids[sl] = __builtin_amdgcn_mov_dpp(x, 0x00, 0xF, 0xF, false);  // quad_perm [0,0,0,0]
-          if (sl % 2 == 1) {  // formed with the row before
-            d0 = dn0;
-            d1 = dn1;
-          } else {
-            // lanes 2, 3: this row's s_0, s_1; lanes 0, 1: the next row's
-            // (quad_perm [2,3,2,3]), or unused values for the last row
-            int v = x, sa = __builtin_amdgcn_mov_dpp(x, 0xAA, 0xF, 0xF, false);  // [2,2,2,2]
-            if (sl + 1 < NS) {
-              const int y = (int)sc[sl + 1];
-              const int yv = __builtin_amdgcn_mov_dpp(y, 0xEE, 0xF, 0xF, false);
-              const int ya = __builtin_amdgcn_mov_dpp(y, 0xAA, 0xF, 0xF, false);
-              v = sub < 2 ? yv : x;
-              sa = sub < 2 ? ya : sa;
-            }
-            const int d = __builtin_bit_cast(
-                int, shrink_factor(__builtin_bit_cast(T, v), __builtin_bit_cast(T, sa), lam, exp_w));
-            d0 = __builtin_bit_cast(T, __builtin_amdgcn_mov_dpp(d, 0xAA, 0xF, 0xF, false));  // [2,2,2,2]
-            d1 = __builtin_bit_cast(T, __builtin_amdgcn_mov_dpp(d, 0xFF, 0xF, 0xF, false));  // [3,3,3,3]
-            if (sl + 1 < NS) {
-              dn0 = __builtin_bit_cast(T, __builtin_amdgcn_mov_dpp(d, 0x00, 0xF, 0xF, false));
-              dn1 = __builtin_bit_cast(T, __builtin_amdgcn_mov_dpp(d, 0x55, 0xF, 0xF, false));  // [1,1,1,1]
-            }
-          }
-        } else {
-          d0 = shrink_factor(s0[sl], s0[sl], lam, exp_w);
-          d1 = shrink_factor(s1[sl], s0[sl], lam, exp_w);
-        }
+        const T d0 = shrink_factor(s0[sl], s0[sl], lam, exp_w), d1 = shrink_factor(s1[sl], s0[sl], lam, exp_w);
         if (ids[sl] >= 0) {
           const int32_t id = ids[sl];
           ST row;
@@ -1941,20 +1891,14 @@ hipError_t launch_svd(const void* uvar, const int32_t* pos, const uint32_t* sel,
   return hipErrorInvalidValue;
 }
 
-hipError_t launch_static_rows(const void* factors, const int32_t* place, const WinMeta* meta, uint32_t nb,
-                              uint32_t nvar_stored, const Shape& sh, void* W0, void* S01, hipStream_t s, uint32_t nk) {
-  if (!fused_eval(sh) || nvar_stored == 0) return hipErrorInvalidValue;
-  if (nk >= sh.nw) nk = 0;
-  const uint32_t nf = nk ? nk + 1 : sh.nw;
-  const dim3 grid((uint32_t)(((size_t)sh.p_sel * nf * 4 + 255) / 256), nb);
+hipError_t launch_static_rows(const void* factors, const int32_t* place, uint32_t nb, uint32_t nvar_stored,
+                              const Shape& sh, void* W0, void* S01, hipStream_t s) {
+  if (!fused_eval(sh) || !sh.fp64 || nvar_stored == 0) return hipErrorInvalidValue;
+  const dim3 grid((uint32_t)(((size_t)sh.p_sel * sh.nw * 4 + 255) / 256), nb);
 #define PG_SR(B)                                                                                                 \
   case B:                                                                                                      \
-    if (sh.fp64)                                                                                               \
-      hipLaunchKernelGGL((k_static_rows<B, double>), grid, dim3(256), 0, s, (const double*)factors, place, meta, \
-                         nvar_stored, sh.p_sel, sh.nw, nk, sh.fstride, (double*)W0, (double*)S01);              \
-    else                                                                                                       \
-      hipLaunchKernelGGL((k_static_rows<B, float>), grid, dim3(256), 0, s, (const float*)factors, place, meta,   \
-                         nvar_stored, sh.p_sel, sh.nw, nk, sh.fstride, (float*)W0, (float*)S01);                \
+    hipLaunchKernelGGL((k_static_rows<B, double>), grid, dim3(256), 0, s, (const double*)factors, place,         \
+                       nvar_stored, sh.p_sel, sh.nw, sh.fstride, (double*)W0, (double*)S01);                    \
     return hipGetLastError();
   switch (sh.bs) {
     PG_SR(2) PG_SR(3) PG_SR(4)
@@ -1964,6 +1908,8 @@ hipError_t launch_static_rows(const void* factors, const int32_t* place, const W
 }
 
 bool fused_eval(const Shape& sh) { return sh.bs <= 4; }
+
+bool strip_overlap(const Shape& sh) { return sh.bs <= 4 && !sh.fp64; }
 
 uint32_t factor_stride(uint32_t nw, uint32_t m) {
   const uint32_t sr = (nw + 3) & ~3u;
@@ -2117,18 +2063,11 @@ hipError_t launch_gather(const GatherSrc& src, const int32_t* off, const double*
   const uint32_t nkk = (mode == 1) ? 1 : gather_frames(sh, nk);
 #define PG_GT(B)                                                                                                 \
   case B:                                                                                                      \
-    if (sh.fp64)                                                                                               \
-      hipLaunchKernelGGL((k_gather_tile<B, double>), dim3(nblk, na), dim3(256), 0, s, (const double*)src.factors, \
-                         (const double*)src.dr, (const double*)src.S01, (const double*)src.W0,                 \
-                         src.list, off, invw, u64, meta, wl, src.slot_lam, src.exp_w,                            \
-                         sh.nr, sh.fs, sh.nw,                                                                  \
-                         sh.vol, sh.n1, sh.p_sel, sh.fstride, src.nvar_stored, mode, nkk, out, partial);       \
-    else                                                                                                       \
-      hipLaunchKernelGGL((k_gather_tile<B, float>), dim3(nblk, na), dim3(256), 0, s, (const float*)src.factors,  \
-                         (const float*)src.dr, (const float*)src.S01, (const float*)src.W0,                    \
-                         src.list, off, invw, u64, meta, wl, src.slot_lam, src.exp_w,                             \
-                         sh.nr, sh.fs, sh.nw,                                                                  \
-                         sh.vol, sh.n1, sh.p_sel, sh.fstride, src.nvar_stored, mode, nkk, out, partial);       \
+    if (!sh.fp64) return hipErrorInvalidValue; /* launch_overlap */                                            \
+    hipLaunchKernelGGL((k_gather_tile<B, double>), dim3(nblk, na), dim3(256), 0, s, (const double*)src.factors,  \
+                       (const double*)src.dr, (const double*)src.S01, (const double*)src.W0, src.list, off,     \
+                       invw, u64, meta, wl, src.slot_lam, src.exp_w, sh.nr, sh.fs, sh.nw, sh.vol, sh.n1,        \
+                       sh.p_sel, sh.fstride, src.nvar_stored, mode, nkk, out, partial);                         \
     break;
 #define PG_GA(B)                                                                                                 \
   case B:                                                                                                      \

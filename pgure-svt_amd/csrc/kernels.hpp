@@ -50,12 +50,9 @@ hipError_t launch_svd(const void* uvar, const int32_t* pos, const uint32_t* sel,
 // the static data of the fused evaluation (patches up to 4 x 4) from the U
 // variant's factors: w_0 v_0[k] into W0 [nb][nw][p_sel][m] and the singular
 // pairs (s_0, s_1) into S01 [nb][nw][p_sel][2], at the bucket places place
-// [nb][nw][p_sel] (the buckets' inverse); for every frame (nk = 0), or for
-// the frames that gathers with frame subset nk and the final frames
-// (meta[b].ref) read
-hipError_t launch_static_rows(const void* factors, const int32_t* place, const WinMeta* meta, uint32_t nb,
-                              uint32_t nvar_stored, const Shape& sh, void* W0, void* S01, hipStream_t s,
-                              uint32_t nk = 0);
+// [nb][nw][p_sel] (the buckets' inverse); FP64 only
+hipError_t launch_static_rows(const void* factors, const int32_t* place, uint32_t nb, uint32_t nvar_stored,
+                              const Shape& sh, void* W0, void* S01, hipStream_t s);
 uint32_t svd_lanes(uint32_t bs, uint32_t nw, int mapping);
 // position buckets of every (window, frame): cnt and off are [nb][nw][n1*n1
 // (+1)], list [nb][nw][p_sel]
@@ -81,9 +78,9 @@ hipError_t launch_eval(const void* factors, const WinMeta* meta, const uint32_t*
 hipError_t launch_divq(const void* factors, const int32_t* pos, const uint32_t* sel, const void* dw, uint32_t nb,
                        uint32_t nvar, const Shape& sh, void* divq, hipStream_t s);
 // Patches up to 4 x 4 evaluate lambda in two launches: launch_round_prep
-// (per patch that keeps rank 1: the factors d_r of its further kept ranks
-// into dr [na][p_sel][nw], ended by a 0; with PGURE (qdiv = divq) the
-// divergence sums into partial [na][eval_blocks]), then launch_gather,
+// (the factors d_r of the kept ranks into dr; with PGURE (qdiv = divq) the
+// divergence sums into partial [na][eval_blocks]), then launch_overlap, or
+// in FP64 (dr [na][p_sel][nw], of ranks after the first) launch_gather,
 // which forms d_0 and the patch rows from the window's static singular
 // pairs and rows (written by launch_static_rows: S01 [nb][nw][p_sel][2], W0
 // [nb][nw][p_sel][m] in bucket order; singular_pair_bytes per window), dr
@@ -132,6 +129,36 @@ uint32_t gather_blocks(const Shape& sh, int mode, uint32_t nk = 0);
 hipError_t launch_gather(const GatherSrc& src, const int32_t* off, const double* invw, const double* u64,
                          const WinMeta* meta, const uint32_t* wl, uint32_t na, const Shape& sh, int mode, double* out,
                          double* partial, hipStream_t s, uint32_t nk = 0);
+// The FP32 overlap-add of patches up to 4 x 4 (overlap.hip) needs neither
+// position buckets nor rows per bucket place: launch_bins sorts every
+// frame's patches by the column of their position (recs [nb][nw][p_sel] =
+// (position, patch), off [nb][nw][column_bins + 1]), launch_cover makes 1/W
+// and delta2/W from them, launch_lead lays the U variant's w_0 (w0
+// [nb][p_sel][m]) and v_0 (v0 [nb][nw][p_sel]) out by patch, and
+// launch_overlap adds the rows up, with d_r from launch_round_prep (dr
+// [na][nw][p_sel], by rank: d_0, negative where rank 1 is kept too, then
+// the further kept ranks, ended by a 0).  wstat [nb][2]: the window's
+// largest s_0 (bits of a float) and largest W; zeroed by the caller before
+// launch_cover and launch_lead raise them.  Modes and nk as launch_gather.
+bool strip_overlap(const Shape& sh);
+uint32_t column_bins(const Shape& sh);
+hipError_t launch_bins(const int32_t* pos, const uint32_t* sel, uint32_t nb, const Shape& sh, int32_t* off,
+                       int2* recs, hipStream_t s);
+hipError_t launch_cover(const int32_t* off, const int2* recs, const uint8_t* d2, uint32_t nb, const Shape& sh,
+                        double d2neg, double d2pos, double* invw, float* dw, uint32_t* wstat, hipStream_t s);
+hipError_t launch_lead(const float* factors, uint32_t nb, uint32_t nvar_stored, const Shape& sh, float* w0, float* v0,
+                       uint32_t* wstat, hipStream_t s);
+struct OverlapSrc {
+  const float *factors = nullptr, *dr = nullptr, *w0 = nullptr, *v0 = nullptr;
+  const int2* recs = nullptr;
+  const int32_t* off = nullptr;
+  const uint32_t* wstat = nullptr;
+  uint32_t nvar_stored = 1;
+};
+uint32_t overlap_blocks(const Shape& sh, int mode, uint32_t nk = 0);
+hipError_t launch_overlap(const OverlapSrc& src, const double* invw, const double* u64, const WinMeta* meta,
+                          const uint32_t* wl, uint32_t na, const Shape& sh, int mode, double* out, double* partial,
+                          hipStream_t s, uint32_t nk = 0);
 // sums [na][6] = (sum Uhat^2, sum U, sum U^2, sum Uhat U,
 // sum d2 (U2p - 2 Uhat + U2m), sum Uhat); with pk (the eval's kept-rank
 // counts), kept [na] = their sum per window
