@@ -718,6 +718,10 @@ struct Pipeline {
   DBuf<char> factors_s, divq_s;
   DBuf<double> partial_s, lam_s;
   DBuf<uint32_t> stats;
+  // learned path: set once the leaf statistics are queued on their stream.
+  // The SVD is launched after that: its workgroups fill the GPU, and the
+  // leaf kernels, if queued behind them, would start when they have drained
+  std::shared_future<void> leaves_queued;
 
   ~Pipeline() {
     // drain the streams before the member buffers go back to the caches
@@ -979,6 +983,7 @@ struct Pipeline {
         hipchk(launch_weights(off.p, d2.p, nb, sh, d2neg, d2pos, invw.p, optimize ? dw.p : nullptr, s), "weights");
       }
     });
+    if (leaves_queued.valid()) leaves_queued.wait();
     // units: matrices decomposed
     prof->run("svd_jacobi", (double)nb * nvar_run * sh.p_sel, [&] {
       // rotation threshold |c| > tol sqrt(ab): 1e-6 in FP32, 1e-12 in FP64;
@@ -1342,15 +1347,31 @@ ProbeFit probe_fit(const double* lam, const double* r) {
   return {b * b / (4 * a) / scale, std::exp(xs)};
 }
 
-// Leaf statistics of the noise estimator (src/noise.hpp:55-100) for frames
-// `frames` of the device cube Xd (n x n frames, FP64), normalised by scale,
-// on the GPU: the split tests of every block of the complete quadtree whose
-// size the F table holds (k_split_stats), the reference's recursion on the
-// host with those decisions, then the statistics of each distinct leaf
-// (k_leaf_stats), in the tree's order per frame.  Frames of at least 16 x 16
-// (smaller ones never split and stay on the host).
-std::vector<FrameLeaves> gpu_frame_leaves(const double* Xd, uint32_t n, const std::vector<uint32_t>& frames,
-                                          double scale, hipStream_t s) {
+// a future that one thread makes ready, once
+struct OnceFlag {
+  std::promise<void> p;
+  std::shared_future<void> future = p.get_future().share();
+  bool done = false;
+  void set() {
+    if (!done) p.set_value();
+    done = true;
+  }
+};
+
+// Leaf statistics of the noise estimator (src/noise.hpp:55-100) on the GPU:
+// item i is frame frames[i] of the device cube Xd (n x n frames, FP64) over
+// scales[i]; sink(i, leaves) receives them in item order.  Split tests of
+// every block of the complete quadtree whose size the F table holds
+// (k_split_stats; ordered: rounded as the host's), the reference's recursion
+// on the host with those decisions, then the statistics of each distinct
+// leaf (k_leaf_*), in the tree's order per item.  Items go in groups whose
+// normalised frames take up to kLeafScratch values.  Frames of at least 16 x
+// 16 (smaller ones never split and stay on the host).  queued: set when the
+// first group's leaf kernels are on the stream.
+void gpu_frame_leaves(const double* Xd, uint32_t n, const std::vector<uint32_t>& frames,
+                      const std::vector<double>& scales, bool ordered, hipStream_t s,
+                      const std::function<void(uint32_t, FrameLeaves&&)>& sink, OnceFlag* queued = nullptr) {
+  constexpr uint64_t kLeafScratch = (uint64_t)1 << 25;
   std::vector<uint32_t> cand;
   std::map<std::array<uint32_t, 3>, uint32_t> cand_at;
   std::function<void(uint32_t, uint32_t, uint32_t)> add = [&](uint32_t i, uint32_t j, uint32_t N) {
@@ -1364,80 +1385,88 @@ std::vector<FrameLeaves> gpu_frame_leaves(const double* Xd, uint32_t n, const st
     add(i + h, j + h, h);
   };
   add(0, 0, n);
-  const uint32_t nf = (uint32_t)frames.size(), nc = (uint32_t)(cand.size() / 3);
-  std::vector<double> stat((size_t)nf * nc);
+  const uint64_t fs = (uint64_t)n * n;
+  const uint32_t total = (uint32_t)frames.size(), nc = (uint32_t)(cand.size() / 3);
+  const uint32_t group = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(kLeafScratch / fs, total));
   DBuf<uint32_t> frames_d, cand_d, leaves_d;
-  DBuf<double> stat_d, out_d;
-  if (nc > 0) {
-    frames_d.alloc(nf);
-    cand_d.alloc(cand.size());
-    stat_d.alloc(stat.size());
-    hipchk(hipMemcpyAsync(frames_d.p, frames.data(), nf * 4, hipMemcpyHostToDevice, s), "H2D leaf frames");
-    hipchk(hipMemcpyAsync(cand_d.p, cand.data(), cand.size() * 4, hipMemcpyHostToDevice, s), "H2D split blocks");
-    hipchk(launch_split_stats(Xd, n, scale, frames_d.p, nf, cand_d.p, nc, stat_d.p, s), "split stats");
-    hipchk(hipMemcpyAsync(stat.data(), stat_d.p, stat.size() * 8, hipMemcpyDeviceToHost, s), "D2H split stats");
-    hipchk(hipStreamSynchronize(s), "split stats sync");
-  }
-  // the reference's recursion per frame; each distinct leaf evaluated once
-  std::vector<uint32_t> leaves;
-  std::vector<std::vector<uint32_t>> order(nf);
-  for (uint32_t fi = 0; fi < nf; ++fi) {
-    const auto tree = quadtree_leaves(n, [&](uint32_t i, uint32_t j, uint32_t N) {
-      const double thr = split_threshold(N);
-      return thr >= 0 && stat[(size_t)fi * nc + cand_at.at({i, j, N})] > thr;
-    });
-    std::map<std::array<uint32_t, 3>, uint32_t> seen;
-    for (const auto& nd : tree) {
-      auto it = seen.find(nd);
-      if (it == seen.end()) {
-        it = seen.emplace(nd, (uint32_t)(leaves.size() / 4)).first;
-        leaves.insert(leaves.end(), {frames[fi], nd[0], nd[1], nd[2]});
-      }
-      order[fi].push_back(it->second);
-    }
-  }
-  const uint32_t nl = (uint32_t)(leaves.size() / 4);
-  std::vector<double> stats((size_t)nl * 2);
-  // leaves above the kernel's register cache: values and Laplacians formed
-  // once, up to kLeafScratch elements in all (the rest form them per pass)
-  constexpr uint64_t kLeafScratch = (uint64_t)1 << 25;
-  std::vector<uint64_t> boff(nl, ~0ull);
-  std::vector<uint32_t> big;
-  uint64_t nbe = 0;
-  for (uint32_t k = 0; k < nl; ++k) {
-    const uint64_t N = (uint64_t)leaves[4 * k + 3] * leaves[4 * k + 3];
-    if (N > leaf_cache_elements() && nbe + N <= kLeafScratch) {
-      boff[k] = nbe;
-      big.push_back(k);
-      nbe += N;
-    }
-  }
-  DBuf<uint32_t> big_d;
   DBuf<uint64_t> boff_d;
-  DBuf<double> vals_d, laps_d;
-  leaves_d.alloc(leaves.size());
-  out_d.alloc(stats.size());
-  boff_d.alloc(nl);
-  hipchk(hipMemcpyAsync(leaves_d.p, leaves.data(), leaves.size() * 4, hipMemcpyHostToDevice, s), "H2D leaves");
-  hipchk(hipMemcpyAsync(boff_d.p, boff.data(), (size_t)nl * 8, hipMemcpyHostToDevice, s), "H2D leaf offsets");
-  if (!big.empty()) {
-    big_d.alloc(big.size());
-    vals_d.alloc(nbe);
-    laps_d.alloc(nbe);
-    hipchk(hipMemcpyAsync(big_d.p, big.data(), big.size() * 4, hipMemcpyHostToDevice, s), "H2D large leaves");
+  DBuf<double> scales_d, Z, stat_d, out_d, laps_d;
+  Z.alloc(group * fs);
+  frames_d.alloc(total);
+  scales_d.alloc(total);
+  hipchk(hipMemcpyAsync(frames_d.p, frames.data(), total * 4, hipMemcpyHostToDevice, s), "H2D leaf frames");
+  hipchk(hipMemcpyAsync(scales_d.p, scales.data(), total * 8, hipMemcpyHostToDevice, s), "H2D leaf scales");
+  if (nc > 0) {
+    cand_d.alloc(cand.size());
+    stat_d.alloc((size_t)group * nc);
+    hipchk(hipMemcpyAsync(cand_d.p, cand.data(), cand.size() * 4, hipMemcpyHostToDevice, s), "H2D split blocks");
   }
-  hipchk(launch_leaf_stats(Xd, n, scale, leaves_d.p, nl, big_d.p, (uint32_t)big.size(), boff_d.p, vals_d.p, laps_d.p,
-                           out_d.p, s),
-         "leaf stats");
-  hipchk(hipMemcpyAsync(stats.data(), out_d.p, stats.size() * 8, hipMemcpyDeviceToHost, s), "D2H leaf stats");
-  hipchk(hipStreamSynchronize(s), "leaf stats sync");
-  std::vector<FrameLeaves> out(nf);
-  for (uint32_t fi = 0; fi < nf; ++fi)
-    for (uint32_t k : order[fi]) {
-      out[fi].mean.push_back(stats[2 * (size_t)k]);
-      out[fi].var.push_back(stats[2 * (size_t)k + 1]);
+  for (uint32_t g0 = 0; g0 < total; g0 += group) {
+    const uint32_t ni = std::min(group, total - g0);
+    std::vector<double> stat((size_t)ni * nc);
+    hipchk(launch_normalise(Xd, (uint32_t)fs, frames_d.p + g0, scales_d.p + g0, ni, Z.p, s), "normalise");
+    if (nc > 0) {
+      hipchk(launch_split_stats(Z.p, n, ni, cand_d.p, nc, ordered, stat_d.p, s), "split stats");
+      hipchk(hipMemcpyAsync(stat.data(), stat_d.p, stat.size() * 8, hipMemcpyDeviceToHost, s), "D2H split stats");
     }
-  return out;
+    hipchk(hipStreamSynchronize(s), "split stats sync");
+    // the reference's recursion per item; each distinct leaf evaluated once,
+    // sorted by the kernel that takes it
+    std::vector<uint32_t> found[3];
+    std::vector<std::vector<std::pair<uint32_t, uint32_t>>> order(ni);  // (class, place in it)
+    for (uint32_t i = 0; i < ni; ++i) {
+      const auto tree = quadtree_leaves(n, [&](uint32_t r, uint32_t c, uint32_t N) {
+        const double thr = split_threshold(N);
+        return thr >= 0 && stat[(size_t)i * nc + cand_at.at({r, c, N})] > thr;
+      });
+      std::map<std::array<uint32_t, 3>, std::pair<uint32_t, uint32_t>> seen;
+      for (const auto& nd : tree) {
+        auto it = seen.find(nd);
+        if (it == seen.end()) {
+          const uint32_t cl = leaf_class(nd[2]);
+          it = seen.emplace(nd, std::make_pair(cl, (uint32_t)(found[cl].size() / 4))).first;
+          found[cl].insert(found[cl].end(), {i, nd[0], nd[1], nd[2]});
+        }
+        order[i].push_back(it->second);
+      }
+    }
+    std::vector<uint32_t> leaves;
+    uint32_t count[3], at[3];
+    for (int c = 0; c < 3; ++c) {
+      at[c] = (uint32_t)(leaves.size() / 4);
+      count[c] = (uint32_t)(found[c].size() / 4);
+      leaves.insert(leaves.end(), found[c].begin(), found[c].end());
+    }
+    const uint32_t nl = (uint32_t)(leaves.size() / 4);
+    std::vector<uint64_t> boff(count[2]);
+    uint64_t nbe = 0;
+    for (uint32_t k = 0; k < count[2]; ++k) {
+      boff[k] = nbe;
+      nbe += (uint64_t)found[2][4 * k + 3] * found[2][4 * k + 3];
+    }
+    std::vector<double> stats((size_t)nl * 2);
+    // (the buffers of the group before are free: its results were read)
+    if (leaves_d.n < leaves.size()) leaves_d.alloc(leaves.size());
+    if (out_d.n < stats.size()) out_d.alloc(stats.size());
+    if (boff_d.n < boff.size()) boff_d.alloc(boff.size());
+    if (laps_d.n < nbe) laps_d.alloc(nbe);
+    hipchk(hipMemcpyAsync(leaves_d.p, leaves.data(), leaves.size() * 4, hipMemcpyHostToDevice, s), "H2D leaves");
+    if (!boff.empty())
+      hipchk(hipMemcpyAsync(boff_d.p, boff.data(), boff.size() * 8, hipMemcpyHostToDevice, s), "H2D leaf offsets");
+    hipchk(launch_leaf_stats(Z.p, n, leaves_d.p, count, boff_d.p, laps_d.p, out_d.p, s), "leaf stats");
+    if (queued) queued->set();
+    hipchk(hipMemcpyAsync(stats.data(), out_d.p, stats.size() * 8, hipMemcpyDeviceToHost, s), "D2H leaf stats");
+    hipchk(hipStreamSynchronize(s), "leaf stats sync");
+    for (uint32_t i = 0; i < ni; ++i) {
+      FrameLeaves fl;
+      for (const auto& o : order[i]) {
+        const size_t k = at[o.first] + o.second;
+        fl.mean.push_back(stats[2 * k]);
+        fl.var.push_back(stats[2 * k + 1]);
+      }
+      sink(g0 + i, std::move(fl));
+    }
+  }
 }
 
 // Host threads for n_jobs (-1 = all): the CPUs this process may run on,
@@ -1561,6 +1590,23 @@ std::vector<uint32_t> feature_sample(uint32_t p_sel, uint32_t nsamp) {
 }
 
 constexpr uint32_t kFeatureSamples = 256;
+
+// Where the leaf statistics of the noise estimator are formed (the results
+// are the same bit for bit).  The host threads cost nothing while the GPU
+// decomposes: 110 ns a value and thread (distinct (frame, normalisation)
+// pairs x pixels; 256 x 256 x 100: 45 ms on 16 threads) against the
+// decomposition's 14 m n^2 + 8 n^3 flops a matrix at 27 TFLOP/s.  Where they
+// would end after it, or nothing runs beside them (the lambda grid's graph
+// waits for every estimate), the GPU forms them (512 x 512 x 40, windows of
+// 7: the call 101 ms with the host's, 90 with the GPU's; 128 x 128 x 30 over
+// a grid: 53.8 against 50.5).  Below 2^18 values the host is done first
+// (64 x 64 x 20: 3.7 against 4.4 ms).
+bool leaves_on_gpu_pay(uint64_t values, uint32_t threads, double matrices, const Shape& sh, bool waits) {
+  if (values < ((uint64_t)1 << 18)) return false;
+  const double host = 110e-9 * (double)values / threads;
+  const double gpu = matrices * (14.0 * sh.m * sh.nw * sh.nw + 8.0 * sh.nw * sh.nw * sh.nw) / 27e12;
+  return waits || host > gpu;
+}
 
 // What one call computes.  mode 0: the reference driver (PGURE search or the
 // fixed lambda); 1: lambda proposed by the learned network; 2: only the
@@ -1730,38 +1776,44 @@ int run_core(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf, co
   } leaf_joiner{leaf_thread};
   const double gmax = *std::max_element(P.fmaxX.begin(), P.fmaxX.end());
   if (P.optimize || learned) {
-    // learned lambda: the leaf statistics of every frame on the GPU (one
-    // scale for all); the reference path keeps the host's bit-exact ones
-    const bool leaves_on_gpu = learned && nr >= 16;
+    // the distinct (frame, normalisation) pairs of the windows
     std::map<std::pair<uint32_t, uint64_t>, uint32_t> key_of;
-    std::vector<std::function<void(PrepPool&)>> jobs;
+    std::vector<std::vector<uint32_t>> needs(count);
     for (uint32_t t = rs.tb; t < rs.te; ++t) {
       const WinMeta m = P.meta_of(t);
       const double scale = learned ? gmax : m.uMax;
       uint64_t sbits;
       std::memcpy(&sbits, &scale, 8);
-      std::vector<uint32_t> need;
       for (uint32_t k = 0; k < g.Nw; ++k) {
-        const auto key = std::make_pair(m.s0 + k, sbits);
-        auto it = key_of.find(key);
-        if (it == key_of.end()) {
-          const uint32_t id = (uint32_t)leaf_jobs.size();
+        const auto it = key_of.emplace(std::make_pair(m.s0 + k, sbits), (uint32_t)leaf_jobs.size());
+        if (it.second) {
           leaf_jobs.emplace_back(new LeafJob{m.s0 + k, scale, {}, {}});
-          LeafJob* J = leaf_jobs.back().get();
-          J->fu = J->pr.get_future().share();
-          if (!leaves_on_gpu)
-            jobs.push_back([J, &P, nr](PrepPool&) {
-              try {
-                std::vector<double> buf((size_t)nr * nr);
-                P.host_frame(J->frame, J->scale, buf.data());
-                J->pr.set_value(std::make_shared<const FrameLeaves>(frame_leaves(buf.data(), nr)));
-              } catch (...) {
-                J->pr.set_exception(std::current_exception());
-              }
-            });
-          it = key_of.emplace(key, id).first;
+          leaf_jobs.back()->fu = leaf_jobs.back()->pr.get_future().share();
         }
-        need.push_back(it->second);
+        needs[t - rs.tb].push_back(it.first->second);
+      }
+    }
+    const bool leaves_on_gpu =
+        nr >= 16 && (learned || leaves_on_gpu_pay((uint64_t)leaf_jobs.size() * P.sh.fs, thread_count(p.n_jobs),
+                                                  (double)count * P.nvar * P.sh.p_sel, P.sh, rs.mode == 3));
+    std::vector<std::function<void(PrepPool&)>> jobs;
+    uint32_t made = 0;  // leaf jobs in the list (host)
+    for (uint32_t t = rs.tb; t < rs.te; ++t) {
+      const WinMeta m = P.meta_of(t);
+      const std::vector<uint32_t>& need = needs[t - rs.tb];
+      for (uint32_t id : need) {
+        if (leaves_on_gpu || id < made) continue;
+        LeafJob* J = leaf_jobs[id].get();
+        made = id + 1;
+        jobs.push_back([J, &P, nr](PrepPool&) {
+          try {
+            std::vector<double> buf((size_t)nr * nr);
+            P.host_frame(J->frame, J->scale, buf.data());
+            J->pr.set_value(std::make_shared<const FrameLeaves>(frame_leaves(buf.data(), nr)));
+          } catch (...) {
+            J->pr.set_exception(std::current_exception());
+          }
+        });
       }
       const double ratio = gmax / m.uMax;
       jobs.push_back([t, need, ratio, learned, &leaf_jobs, &P, &p, &rs, g, nr, nc, lambda0, alpha0, mu0,
@@ -1803,27 +1855,30 @@ int run_core(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf, co
       int dev = 0;
       hipchk(hipGetDevice(&dev), "hipGetDevice");
       std::vector<uint32_t> frames;
-      for (const auto& J : leaf_jobs) frames.push_back(J->frame);
+      std::vector<double> scales;
+      for (const auto& J : leaf_jobs) {
+        frames.push_back(J->frame);
+        scales.push_back(J->scale);
+      }
       const double* Xd = P.Xd.p;
-      leaf_thread = std::thread([&leaf_jobs, frames, dev, nr, gmax, Xd]() {
+      auto queued = std::make_shared<OnceFlag>();
+      if (learned) P.leaves_queued = queued->future;
+      leaf_thread = std::thread([&leaf_jobs, frames, scales, dev, nr, learned, Xd, queued]() {
         size_t done = 0;
         try {
           hipchk(hipSetDevice(dev), "hipSetDevice");
-          hipStream_t s2 = nullptr;
-          hipchk(hipStreamCreateWithFlags(&s2, hipStreamNonBlocking), "hipStreamCreate");
-          struct StreamGuard {
-            hipStream_t s;
-            ~StreamGuard() {
-              (void)hipStreamSynchronize(s);
-              (void)hipStreamDestroy(s);
-            }
-          } guard{s2};
+          StreamOwner s2;
           HostTimer tl("noise_leaves_gpu");
-          std::vector<FrameLeaves> lv = gpu_frame_leaves(Xd, nr, frames, gmax, s2);
-          for (; done < leaf_jobs.size(); ++done)
-            leaf_jobs[done]->pr.set_value(std::make_shared<const FrameLeaves>(std::move(lv[done])));
+          gpu_frame_leaves(
+              Xd, nr, frames, scales, !learned, s2.s,
+              [&](uint32_t i, FrameLeaves&& lv) {
+                leaf_jobs[i]->pr.set_value(std::make_shared<const FrameLeaves>(std::move(lv)));
+                done = i + 1;
+              },
+              queued.get());
         } catch (...) {
           for (; done < leaf_jobs.size(); ++done) leaf_jobs[done]->pr.set_exception(std::current_exception());
+          queued->set();
         }
       });
     }
@@ -2769,7 +2824,7 @@ int pgsvt_frame_leaves(const double* frame, uint32_t n, int on_gpu, uint32_t cap
       DBuf<double> d;
       d.alloc((size_t)n * n);
       hipchk(hipMemcpyAsync(d.p, frame, (size_t)n * n * 8, hipMemcpyHostToDevice, s), "H2D frame");
-      fl = std::move(gpu_frame_leaves(d.p, n, {0u}, 1.0, s)[0]);
+      gpu_frame_leaves(d.p, n, {0u}, {1.0}, true, s, [&](uint32_t, FrameLeaves&& l) { fl = std::move(l); });
     } else {
       fl = frame_leaves(frame, n);
     }

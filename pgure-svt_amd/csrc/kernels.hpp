@@ -195,21 +195,21 @@ hipError_t launch_fill32(void* p, uint64_t n, uint32_t v, hipStream_t s);
 hipError_t launch_copy_rows(const void* src, void* dst, uint32_t rows, uint32_t width, uint32_t step,
                             size_t src_batch, size_t dst_batch, uint32_t nb, hipStream_t s);
 
-// Noise estimator's quadtree on the GPU (noise_gpu.hip).  Split tests of
-// blocks [nblocks][3] (row, column, size) of frames frames [nf] of the FP64
-// cube X (n x n frames) normalised by scale: stat [nf][nblocks] = the F
-// statistic of SplitBlockQ.  Leaf statistics of leaves [nleaves][4] (frame,
-// row, column, size): out [nleaves][2] = (robust mean, robust variance).
-// Leaves of more than leaf_cache_elements() elements: those listed in big
-// [nbig] have their values and Laplacians formed once into vals and laps
-// from element boff[leaf] (boff [nleaves]); the others (boff ~0) form them
-// again at every pass.
-hipError_t launch_split_stats(const double* X, uint32_t n, double scale, const uint32_t* frames, uint32_t nf,
-                              const uint32_t* blocks, uint32_t nblocks, double* stat, hipStream_t s);
-uint32_t leaf_cache_elements();
-hipError_t launch_leaf_stats(const double* X, uint32_t n, double scale, const uint32_t* leaves, uint32_t nleaves,
-                             const uint32_t* big, uint32_t nbig, const uint64_t* boff, double* vals, double* laps,
-                             double* out, hipStream_t s);
+// Noise estimator's quadtree on the GPU (noise_gpu.hip).  launch_normalise:
+// Z [items][fs] = frame frames[i] of the FP64 cube X over scales[i].  Split
+// tests of blocks [nblocks][3] (row, column, size) of every item: stat
+// [items][nblocks] = the F statistic of SplitBlockQ, with the host's order
+// of every sum (ordered) or workgroup sums.  Leaf statistics of leaves [][4]
+// (item, row, column, size), sorted by leaf_class of their size (count [3]
+// of each): out [][2] = (robust mean, robust variance), rounded as the
+// host's; boff: where in laps each leaf of class 2 keeps its Laplacians.
+hipError_t launch_normalise(const double* X, uint32_t fs, const uint32_t* frames, const double* scales,
+                            uint32_t items, double* Z, hipStream_t s);
+hipError_t launch_split_stats(const double* Z, uint32_t n, uint32_t items, const uint32_t* blocks, uint32_t nblocks,
+                              bool ordered, double* stat, hipStream_t s);
+uint32_t leaf_class(uint32_t s);
+hipError_t launch_leaf_stats(const double* Z, uint32_t n, const uint32_t* leaves, const uint32_t count[3],
+                             const uint64_t* boff, double* laps, double* out, hipStream_t s);
 // lambda grid: G candidates per window from the sampled patches' median
 // singular value; then risk of every candidate from the sums [nb*G][6] and
 // the argmin into meta[b].lambda (risk [nb*G] kept)
