@@ -95,7 +95,7 @@ int pgsvt_denoise_device(const void* X_dev, int dtype, uint32_t n_rows,
 /* pgsvt_denoise_device that allocates no device memory.  No reference
  * counterpart: it is for callers that cannot allocate (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  Windows
- * are processed one at a time in a statically sized device array of 64 MiB
+ * are processed one at a time in a statically sized device array of 66 MiB
  * that each device the library runs on holds until the process ends; a
  * shape whose window needs more returns PGSVT_E_ARG with the size in the
  * message (64 x 64 frames fit with PGURE, 128 x 128 with a fixed lambda at

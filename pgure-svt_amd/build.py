@@ -32,6 +32,7 @@ HOST = ["-x", "c++", "-pthread"]
 
 SOURCES = [
     ("kernels.hip", DEVICE),
+    ("svd.hip", DEVICE),
     ("overlap.hip", DEVICE),
     ("hotpixel.hip", DEVICE),
     ("mlp.hip", DEVICE),

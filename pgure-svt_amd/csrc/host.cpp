@@ -697,7 +697,7 @@ struct Pipeline {
   DBuf<char> divq;  // per (patch, variant) singular values and divergence factors (PGURE)
   // SVD input variants, factors and U reconstructions: FP32, or FP64 for
   // the precision study (sh.fp64); sized in bytes
-  DBuf<char> uvar, factors, B0;  // B0: reconstructed rows (patches above 4 x 4) or the factors d_r (dr)
+  DBuf<char> uvar, factors, B0, dr;  // B0: reconstructed rows (patches above 4 x 4); dr: the factors d_r
   DBuf<int32_t> pos, cnt, off, list, inv;
   // the fused evaluation's static data per window (patches up to 4 x 4):
   // rows w_0 v_0[k] and singular pairs (s_0, s_1) per (frame, bucket place)
@@ -831,6 +831,12 @@ struct Pipeline {
     return m;
   }
 
+  // what an evaluation writes: the factors d_r of the kept ranks, and (FP64:
+  // instead) rows of patches above 4 x 4
+  bool uses_dr() const { return strip_overlap(sh) || fused_eval(sh); }
+  bool uses_rows() const { return stored_rows(sh) || !uses_dr(); }
+  size_t values_per_place() const { return (uses_dr() ? 1 : 0) + (uses_rows() ? sh.m : 0); }
+
   size_t bytes_per_window() const {
     const size_t es = sh.fp64 ? 8 : 4;
     size_t b = 0;
@@ -844,9 +850,9 @@ struct Pipeline {
       b += 8ull * sh.nw * ((size_t)sh.n1 * sh.n1 + 1);   // bucket counts + offsets
     b += 8ull * sh.nw * sh.p_sel;                        // bucket lists + inverse, or the column records
     b += 8ull * sh.vol * (optimize ? 2 : 1);             // 1/W, delta2/W
-    b += es * sh.nw * (size_t)sh.p_sel * (fused_eval(sh) ? 1 : sh.m);  // B0 (or dr)
+    b += es * sh.nw * (size_t)sh.p_sel * values_per_place();  // dr, B0 or rows
     if (strip_overlap(sh)) {
-      b += 4ull * sh.p_sel * (sh.m + sh.nw);                 // leading vectors
+      b += 4ull * sh.p_sel * ((fused_eval(sh) ? sh.m : 0) + sh.nw);  // leading vectors
     } else if (fused_eval(sh)) {
       b += singular_pair_bytes(sh);                          // static singular pairs
       b += es * sh.nw * (size_t)sh.p_sel * sh.m;             // static rows
@@ -901,7 +907,7 @@ struct Pipeline {
     if (strip_overlap(sh)) {
       off.alloc((size_t)NB * sh.nw * (column_bins(sh) + 1));
       recs.alloc((size_t)NB * sh.nw * sh.p_sel);
-      w0.alloc((size_t)NB * sh.p_sel * sh.m);
+      if (fused_eval(sh)) w0.alloc((size_t)NB * sh.p_sel * sh.m);
       v0.alloc((size_t)NB * sh.nw * sh.p_sel);
       wstat.alloc(2 * (size_t)NB);
     } else {
@@ -913,7 +919,8 @@ struct Pipeline {
     }
     invw.alloc((size_t)NB * sh.vol);
     if (optimize) dw.alloc((size_t)NB * sh.vol * (sh.fp64 ? sizeof(double) : sizeof(float)));
-    B0.alloc((size_t)NB * sh.nw * sh.p_sel * (fused_eval(sh) ? 1 : sh.m) * es);
+    if (uses_dr()) dr.alloc((size_t)NB * sh.nw * sh.p_sel * es);
+    if (uses_rows()) B0.alloc((size_t)NB * sh.nw * sh.p_sel * sh.m * es);
     if (fused_eval(sh) && !strip_overlap(sh)) {
       w0b.alloc((size_t)NB * sh.nw * sh.p_sel * sh.m * es);
       s01b.alloc((size_t)NB * singular_pair_bytes(sh));
@@ -1018,7 +1025,8 @@ struct Pipeline {
     if (strip_overlap(sh)) {
       OverlapSrc o;
       o.factors = (const float*)factors.p;
-      o.dr = (const float*)B0.p;
+      o.dr = (const float*)dr.p;
+      o.rows = (const float*)B0.p;
       o.w0 = w0.p;
       o.v0 = v0.p;
       o.recs = recs.p;
@@ -1031,7 +1039,7 @@ struct Pipeline {
     GatherSrc g;
     g.B0 = B0.p;
     g.factors = factors.p;
-    g.dr = B0.p;
+    g.dr = dr.p;
     g.S01 = s01b.p;
     g.W0 = w0b.p;
     g.list = list.p;
@@ -1050,7 +1058,7 @@ struct Pipeline {
   void evaluate(const uint32_t* wl, uint32_t na, uint32_t nvar_run, const double* slot_lam, double* part,
                 double* kept) {
     hipchk(launch_evaluation(sh, factors.p, divq.p, meta_d.p, wl, na, nvar, nvar_run, p.exponential_weighting, inv.p,
-                             B0.p, part, slot_lam, kept, s),
+                             dr.p, B0.p, part, slot_lam, kept, s),
            "eval");
   }
 
@@ -1592,20 +1600,21 @@ std::vector<uint32_t> feature_sample(uint32_t p_sel, uint32_t nsamp) {
 constexpr uint32_t kFeatureSamples = 256;
 
 // Where the leaf statistics of the noise estimator are formed (the results
-// are the same bit for bit).  The host threads cost nothing while the GPU
-// decomposes: 110 ns a value and thread (distinct (frame, normalisation)
-// pairs x pixels; 256 x 256 x 100: 45 ms on 16 threads) against the
-// decomposition's 14 m n^2 + 8 n^3 flops a matrix at 27 TFLOP/s.  Where they
-// would end after it, or nothing runs beside them (the lambda grid's graph
-// waits for every estimate), the GPU forms them (512 x 512 x 40, windows of
-// 7: the call 101 ms with the host's, 90 with the GPU's; 128 x 128 x 30 over
-// a grid: 53.8 against 50.5).  Below 2^18 values the host is done first
-// (64 x 64 x 20: 3.7 against 4.4 ms).
+// are the same bit for bit).  The host threads cost the GPU nothing while it
+// decomposes: about 60 ns a value and thread (distinct (frame,
+// normalisation) pairs x pixels) against the decomposition's 0.85 ns a
+// matrix and its 14 m n^2 + 8 n^3 flops at 25 TFLOP/s (256 x 256 x 100: the
+// call takes 116 ms with the host's, 119 with the GPU's, whose leaves share
+// the SIMDs with the SVD).  Where they would end after it, or nothing runs
+// beside them (the lambda grid's graph waits for every estimate), the GPU
+// forms them (512 x 512 x 40, windows of 7: 101 ms with the host's, 91 with
+// the GPU's; 128 x 128 x 30 over a grid: 53.8 against 50.5).  Below 2^18
+// values the host is done first (64 x 64 x 20: 3.7 against 4.4 ms).
 bool leaves_on_gpu_pay(uint64_t values, uint32_t threads, double matrices, const Shape& sh, bool waits) {
   if (values < ((uint64_t)1 << 18)) return false;
-  const double host = 110e-9 * (double)values / threads;
-  const double gpu = matrices * (14.0 * sh.m * sh.nw * sh.nw + 8.0 * sh.nw * sh.nw * sh.nw) / 27e12;
-  return waits || host > gpu;
+  const double host = 60e-9 * (double)values / threads;
+  const double flops = 14.0 * sh.m * sh.nw * sh.nw + 8.0 * sh.nw * sh.nw * sh.nw;
+  return waits || host > matrices * (0.85e-9 + flops / 25e12);
 }
 
 // What one call computes.  mode 0: the reference driver (PGURE search or the
@@ -2181,8 +2190,10 @@ int guarded(F f) {
 // keeps the last call's contents.  The kernels, their launch shapes and the
 // order of every sum are those of pgsvt_denoise_device, so the results are
 // the same bit for bit.
-constexpr size_t kNoAllocScratch = 64ull << 20;
-static __device__ __align__(256) unsigned char scratch[kNoAllocScratch];
+// The array is larger than the size that bounds the shapes, for layouts that
+// need a little more than the one the bound is stated for.
+constexpr size_t kNoAllocScratch = 64ull << 20, kNoAllocArray = 66ull << 20;
+static __device__ __align__(256) unsigned char scratch[kNoAllocArray];
 
 std::mutex g_scratch_mu;
 std::map<int, unsigned char*> g_scratch_at;  // device -> address of its copy of `scratch`
@@ -2250,7 +2261,7 @@ int run_noalloc(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf,
   sh.fstride = factor_stride(g.Nw, sh.m);
   const size_t npos = (size_t)sh.n1 * sh.n1, vol = sh.vol;
   const uint32_t max_jobs = 2 * g.Nw, eblk = eval_blocks(sh, 3);
-  const uint32_t gblk = strip_overlap(sh) ? overlap_blocks(sh, 0) : pgsvt::gather_blocks(sh, 0);
+  const uint32_t gblk = overlap_blocks(sh, 0);
   const double vP = 0.5 + 0.5 * 1. / std::sqrt(1. * 1. + 4), vQ = 1 - vP;
   const double d2neg = -1 * std::sqrt(vQ / vP), d2pos = std::sqrt(vP / vQ), eps2 = 1e-2;
   // the layout: per call, then the window being processed
@@ -2260,17 +2271,15 @@ int run_noalloc(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf,
     double *fmax, *sums, *Xw, *Zw, *u64, *w64, *invw, *partial, *partial_b;
     WinMeta* meta;
     int16_t* jobs;
-    float *uvar, *dw, *B0, *factors, *divq, *w0, *v0;
-    int32_t *pos, *cnt, *off, *list, *inv;
+    float *uvar, *dw, *B0, *dr, *factors, *divq, *w0, *v0;
+    int32_t *pos, *off;
     int2* recs;
     uint32_t* wstat;
   } L{};
-  // stated: the layout with position buckets and rows per bucket place
-  // (patches up to 4 x 4), by whose size the shapes this entry point takes
-  // are stated; the present one is smaller, and a shape is neither refused
-  // nor taken anew when a layout shrinks
+  // stated: the layout with position buckets, by whose size the shapes this
+  // entry point takes are stated: a shape is neither refused nor taken anew
+  // when the layout changes
   auto carve = [&](Carve& c, bool stated) {
-    const bool strips = strip_overlap(sh) && !stated;
     L.d2 = optimize ? c.take<uint8_t>(vol) : nullptr;
     L.sel = c.take<uint32_t>(sh.p_sel);
     L.wl = c.take<uint32_t>(1);
@@ -2285,35 +2294,38 @@ int run_noalloc(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf,
     L.w64 = median ? c.take<double>(vol) : nullptr;
     L.uvar = c.take<float>((size_t)nvar * vol);
     L.pos = c.take<int32_t>((size_t)g.Nw * sh.p_all);
-    if (strips) {
+    if (!stated) {
       L.off = c.take<int32_t>((size_t)g.Nw * (column_bins(sh) + 1));
       L.recs = c.take<int2>((size_t)g.Nw * sh.p_sel);
-      L.w0 = c.take<float>((size_t)sh.p_sel * sh.m);
+      if (fused_eval(sh)) L.w0 = c.take<float>((size_t)sh.p_sel * sh.m);
       L.v0 = c.take<float>((size_t)g.Nw * sh.p_sel);
       L.wstat = c.take<uint32_t>(2);
     } else {
-      L.cnt = c.take<int32_t>((size_t)g.Nw * npos);
-      L.off = c.take<int32_t>((size_t)g.Nw * (npos + 1));
-      L.list = c.take<int32_t>((size_t)g.Nw * sh.p_sel);
-      L.inv = c.take<int32_t>((size_t)g.Nw * sh.p_sel);
+      c.take<int32_t>((size_t)g.Nw * npos);
+      c.take<int32_t>((size_t)g.Nw * (npos + 1));
+      c.take<int32_t>((size_t)g.Nw * sh.p_sel);
+      c.take<int32_t>((size_t)g.Nw * sh.p_sel);
     }
     L.invw = c.take<double>(vol);
     L.dw = optimize ? c.take<float>(vol) : nullptr;
-    L.B0 = c.take<float>((size_t)g.Nw * sh.p_sel * (fused_eval(sh) ? 1 : sh.m));
-    if (fused_eval(sh) && !strips) {
+    if (!fused_eval(sh)) L.B0 = c.take<float>((size_t)g.Nw * sh.p_sel * sh.m);
+    if (fused_eval(sh) || !stated) L.dr = c.take<float>((size_t)g.Nw * sh.p_sel);
+    if (fused_eval(sh) && stated) {
       c.take<char>(singular_pair_bytes(sh));
       c.take<float>((size_t)g.Nw * sh.p_sel * sh.m);
     }
     L.factors = c.take<float>((size_t)nvar * sh.p_sel * sh.fstride);
     L.divq = optimize ? c.take<float>((size_t)nvar * sh.p_sel * 2 * sr) : nullptr;
-    L.partial = c.take<double>(eblk);
-    L.partial_b = c.take<double>((size_t)gblk * 5);
+    L.partial = c.take<double>(!stated ? eblk : fused_eval(sh) ? (sh.p_sel + 255) / 256 : (sh.p_sel + 3) / 4);
+    L.partial_b = c.take<double>((size_t)(!stated ? gblk : pgsvt::gather_blocks(sh, 0)) * 5);
   };
-  Carve count;
+  Carve count, real;
   carve(count, true);
+  carve(real, false);
   if (count.used > kNoAllocScratch)
     return fail(PGSVT_E_ARG, "this shape needs " + std::to_string(count.used) + " bytes of device scratch per window; "
                              "the entry point without allocation has " + std::to_string(kNoAllocScratch));
+  if (real.used > kNoAllocArray) return fail(PGSVT_E_ARG, "the scratch array is too small for this shape's layout");
   std::lock_guard<std::mutex> lock(g_scratch_mu);
   Carve at;
   at.base = scratch_address();
@@ -2331,27 +2343,17 @@ int run_noalloc(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf,
   if (optimize) hipchk(launch_delta2((int64_t)seed, vol, L.d2, s), "delta2");
   hipchk(hipStreamSynchronize(s), "setup sync");  // the host vectors above are local
   auto overlap = [&](int mode, double* out, double* part) {
-    if (strip_overlap(sh)) {
-      OverlapSrc o;
-      o.factors = L.factors;
-      o.dr = L.B0;
-      o.w0 = L.w0;
-      o.v0 = L.v0;
-      o.recs = L.recs;
-      o.off = L.off;
-      o.wstat = L.wstat;
-      o.nvar_stored = nvar;
-      hipchk(launch_overlap(o, L.invw, L.u64, L.meta, L.wl, 1, sh, mode, out, part, s), "overlap-add");
-      return;
-    }
-    GatherSrc g;
-    g.B0 = L.B0;
-    g.factors = L.factors;
-    g.dr = L.B0;
-    g.exp_w = p.exponential_weighting;
-    g.list = L.list;
-    g.nvar_stored = nvar;
-    hipchk(launch_gather(g, L.off, L.invw, L.u64, L.meta, L.wl, 1, sh, mode, out, part, s), "gather");
+    OverlapSrc o;
+    o.factors = L.factors;
+    o.dr = L.dr;
+    o.rows = L.B0;
+    o.w0 = L.w0;
+    o.v0 = L.v0;
+    o.recs = L.recs;
+    o.off = L.off;
+    o.wstat = L.wstat;
+    o.nvar_stored = nvar;
+    hipchk(launch_overlap(o, L.invw, L.u64, L.meta, L.wl, 1, sh, mode, out, part, s), "overlap-add");
   };
   std::vector<double> fmax(2 * g.Nw), sums(6), hw;
   int status = 0;
@@ -2389,19 +2391,14 @@ int run_noalloc(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf,
     hipchk(launch_fill_ref(L.meta, 1, sh, L.pos, s), "fill_ref");
     if (p.motion_estimation)
       hipchk(launch_arps(median ? L.w64 : L.u64, L.jobs, max_jobs, 1, sh, (int)p.motion_window, L.pos, s), "arps");
-    if (strip_overlap(sh)) {
-      hipchk(launch_fill32(L.wstat, 2, 0, s), "clear window figures");
-      hipchk(launch_bins(L.pos, L.sel, 1, sh, L.off, L.recs, s), "bins");
-      hipchk(launch_cover(L.off, L.recs, L.d2, 1, sh, d2neg, d2pos, L.invw, L.dw, L.wstat, s), "cover");
-    } else {
-      hipchk(launch_buckets(L.pos, L.sel, 1, sh, L.cnt, L.off, L.list, L.inv, s), "buckets");
-      hipchk(launch_weights(L.off, L.d2, 1, sh, d2neg, d2pos, L.invw, L.dw, s), "weights");
-    }
+    hipchk(launch_fill32(L.wstat, 2, 0, s), "clear window figures");
+    hipchk(launch_bins(L.pos, L.sel, 1, sh, L.off, L.recs, s), "bins");
+    hipchk(launch_cover(L.off, L.recs, L.d2, 1, sh, d2neg, d2pos, L.invw, L.dw, L.wstat, s), "cover");
     hipchk(launch_fill32(L.stats, 1, 0, s), "clear stats");
     hipchk(launch_svd(L.uvar, L.pos, L.sel, 1, nvar, nvar, sh, L.factors, 30, 1e-6, L.stats, s,
                       g_svd_mapping.load() == 1 ? 1 : 0),
            "svd");
-    if (strip_overlap(sh)) hipchk(launch_lead(L.factors, 1, nvar, sh, L.w0, L.v0, L.wstat, s), "leading vectors");
+    hipchk(launch_lead(L.factors, 1, nvar, sh, L.w0, L.v0, L.wstat, s), "leading vectors");
     if (optimize) hipchk(launch_divq(L.factors, L.pos, L.sel, L.dw, 1, nvar, sh, L.divq, s), "divergence factors");
     double alpha = alpha0, mu = mu0, sigma = sigma0, lambda = lambda0;
     if (optimize) {
@@ -2435,8 +2432,8 @@ int run_noalloc(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf,
         if (!known) {
           m.lambda = l;
           hipchk(hipMemcpyAsync(L.meta, &m, sizeof m, hipMemcpyHostToDevice, s), "H2D meta");
-          hipchk(launch_evaluation(sh, L.factors, L.divq, L.meta, L.wl, 1, nvar, 3, p.exponential_weighting, L.inv,
-                                   L.B0, L.partial, nullptr, nullptr, s),
+          hipchk(launch_evaluation(sh, L.factors, L.divq, L.meta, L.wl, 1, nvar, 3, p.exponential_weighting, nullptr,
+                                   L.dr, L.B0, L.partial, nullptr, nullptr, s),
                  "eval");
           overlap(0, nullptr, L.partial_b);
           hipchk(launch_risk_reduce(L.partial, eblk, L.partial_b, gblk, 1, L.sums, s), "reduce");
@@ -2461,8 +2458,8 @@ int run_noalloc(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf,
     // the output frame at the window's lambda (Pipeline::finish)
     m.lambda = lambda;
     hipchk(hipMemcpyAsync(L.meta, &m, sizeof m, hipMemcpyHostToDevice, s), "H2D meta");
-    hipchk(launch_evaluation(sh, L.factors, nullptr, L.meta, L.wl, 1, nvar, 1, p.exponential_weighting, L.inv, L.B0,
-                             nullptr, nullptr, nullptr, s),
+    hipchk(launch_evaluation(sh, L.factors, nullptr, L.meta, L.wl, 1, nvar, 1, p.exponential_weighting, nullptr, L.dr,
+                             L.B0, nullptr, nullptr, nullptr, s),
            "eval final");
     overlap(1, Y, nullptr);
     hipchk(hipStreamSynchronize(s), "window sync");  // m and jobs are reused by the next window

@@ -19,6 +19,8 @@
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "lanes.hpp"
+#include "shapes.hpp"
 
 namespace pgsvt {
 
@@ -455,243 +457,6 @@ __device__ __forceinline__ T shrink_factor(T s, T s0, double lam, int exp_w) {
   return s > T(0) ? fmax(s - w, T(0)) / s : T(0);
 }
 
-// --------------------------------------------------- batched Jacobi SVD --
-// One-sided (Hestenes) Jacobi on the m x n Casorati matrix of each patch
-// (arma::svd_econ at src/svt.hpp:111).  Output per patch, sorted by
-// descending singular value: V^T (n x n), W^T = (X V)^T (n x m) and s (n).
-// A group of L lanes holds one matrix; lane l owns rows l, l + L, l + 2L ...
-// of X (R rows), so the rotation parameters, which every lane of the group
-// computes, are shared by R rows.  Column dot products
-// are a sum over the lane's rows, then a butterfly across the group (DPP
-// inside a 16-lane row, lane swaps for 32/64-lane groups).  Every lane ends
-// the butterfly with the bit-identical sum, so all lanes apply the same
-// rotation.  Column norms are carried through the sweep with the exact
-// Jacobi update (a -= t c, b += t c) and refreshed at the start of every
-// sweep, so a pair costs one butterfly.  V is not accumulated: after
-// convergence V = X^T W S^-2 (X reloaded), row by row.  Its error in a
-// reconstruction d_r w_r v_r^T stays at eps * s_max (that of v_r is
-// eps * s_max / s_r, times |w_r| = s_r); ranks with s_r <= eps * s_max get
-// v_r = 0, below that level too.
-template <int CTRL>
-__device__ __forceinline__ float dpp_f(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
-}
-
-// The empty asm statement on entry makes v an opaque, already rounded
-// value.  Without it the compiler contracts the caller's product into the
-// first butterfly add, fma(x_i, x_j, neighbour's rounded product), which
-// rounds differently in the two lanes of a pair: the lanes then hold
-// different sums and apply different rotations (seen as singular values
-// off by 1e-2 of s_max on near-degenerate column pairs).
-template <int L>
-__device__ __forceinline__ float group_sum(float v) {
-  asm volatile("" : "+v"(v));
-  if (L >= 2) v += dpp_f<0xB1>(v);   // quad_perm [1,0,3,2]
-  if (L >= 4) v += dpp_f<0x4E>(v);   // quad_perm [2,3,0,1]
-  if (L >= 8) v += dpp_f<0x141>(v);  // row_half_mirror
-  if (L >= 16) v += dpp_f<0x140>(v); // row_mirror
-  if (L >= 32) v += __shfl_xor(v, 16);
-  if (L >= 64) v += __shfl_xor(v, 32);
-  return v;
-}
-
-// FP64 (the divergence factors and the precision-study path): the same
-// DPP steps on both halves of the double; after each step the lanes that
-// are paired next hold equal partial sums, so the result is the one of
-// the lane-swap (xor) butterfly and bit-identical in every lane
-template <int CTRL>
-__device__ __forceinline__ double dpp_d(double v) {
-  const int2 h = __builtin_bit_cast(int2, v);
-  int2 o;
-  o.x = __builtin_amdgcn_update_dpp(0, h.x, CTRL, 0xF, 0xF, false);
-  o.y = __builtin_amdgcn_update_dpp(0, h.y, CTRL, 0xF, 0xF, false);
-  return __builtin_bit_cast(double, o);
-}
-template <int L>
-__device__ __forceinline__ double group_sum(double v) {
-  asm volatile("" : "+v"(v));
-  if (L >= 2) v += dpp_d<0xB1>(v);   // quad_perm [1,0,3,2]
-  if (L >= 4) v += dpp_d<0x4E>(v);   // quad_perm [2,3,0,1]
-  if (L >= 8) v += dpp_d<0x141>(v);  // row_half_mirror
-  if (L >= 16) v += dpp_d<0x140>(v); // row_mirror
-  if (L >= 32) v += __shfl_xor(v, 16);
-  if (L >= 64) v += __shfl_xor(v, 32);
-  return v;
-}
-
-// reciprocal, square root and reciprocal square root: the hardware
-// approximations in FP32, IEEE-correct operations in FP64
-__device__ __forceinline__ float rcp_(float x) { return __builtin_amdgcn_rcpf(x); }
-__device__ __forceinline__ double rcp_(double x) { return 1.0 / x; }
-__device__ __forceinline__ float sqrt_(float x) { return __builtin_amdgcn_sqrtf(x); }
-__device__ __forceinline__ double sqrt_(double x) { return sqrt(x); }
-__device__ __forceinline__ float rsq_(float x) { return __builtin_amdgcn_rsqf(x); }
-__device__ __forceinline__ double rsq_(double x) { return 1.0 / sqrt(x); }
-
-// RT: the window length n = nw is known at run time only (n <= N): the
-// matrix is held as N columns, the last N - n zero, and every loop stops at
-// n (uniform branches); the stored layout follows n.
-template <int BS, int N, int L, class T, bool RT = false>
-__global__ __launch_bounds__(256) void k_svd(const T* __restrict__ u32, const int32_t* __restrict__ pos,
-                                             const uint32_t* __restrict__ sel, uint32_t nvar, uint32_t nvar_stored,
-                                             uint32_t p_sel, uint32_t p_all, uint32_t nr, uint32_t fs, uint32_t nw,
-                                             uint32_t vol, uint32_t lim, uint32_t fstride, int max_sweeps, T tol2,
-                                             T* __restrict__ factors, uint32_t* __restrict__ stats) {
-  constexpr int M = BS * BS, R = (M + L - 1) / L, SRN = (N + 3) & ~3;
-  const int n = RT ? (int)nw : N;
-  const int SR = RT ? ((n + 3) & ~3) : SRN;
-  const uint32_t b = blockIdx.y;
-  const int lane = threadIdx.x % L;
-  const uint32_t g = (blockIdx.x * blockDim.x + threadIdx.x) / L;
-  const uint32_t var = g / p_sel, p = g % p_sel;
-  const bool valid = var < nvar;  // uniform per group
-  const uint32_t it = valid ? (p_sel == p_all ? p : sel[p]) : 0;  // step 1: identity selection
-
-  const T* U = u32 + ((size_t)b * nvar_stored + (valid ? var : 0)) * vol;
-  // the lane's rows of the Casorati matrix X (column k: frame k's patch)
-  auto load_x = [&](T (&y)[R][N]) {
-#pragma unroll
-    for (int k = 0; k < N; ++k) {
-      const bool kin = !RT || k < n;
-      const int32_t pk = (valid && kin) ? pos[((size_t)b * nw + k) * p_all + it] : 0;
-      const uint32_t row = min((uint32_t)(pk & 0xffff), lim), col = min((uint32_t)(pk >> 16), lim);
-#pragma unroll
-      for (int h = 0; h < R; ++h) {
-        const int q = lane + L * h;
-        y[h][k] = (valid && kin && q < M) ? U[(size_t)k * fs + (row + q % BS) + (size_t)nr * (col + q / BS)] : T(0);
-      }
-    }
-  };
-  T x[R][N];
-  load_x(x);
-
-  T a[N];
-  int sweep = 0;
-  for (; sweep < max_sweeps; ++sweep) {
-#pragma unroll
-    for (int k = 0; k < N; ++k) {
-      T t = x[0][k] * x[0][k];
-#pragma unroll
-      for (int h = 1; h < R; ++h) t = fma(x[h][k], x[h][k], t);
-      a[k] = group_sum<L>(t);
-    }
-    // sum of t^2 over the sweep: zero exactly when no pair rotated.  A
-    // floating-point chain (never reassociated) keeps this in one register.
-    T tsum = T(0);
-#pragma unroll
-    for (int i = 0; i < N - 1; ++i) {
-      if (RT && i + 1 >= n) break;
-#pragma unroll
-      for (int j = i + 1; j < N; ++j) {
-        if (RT && j >= n) break;
-        // rotation zeroing the (i, j) inner product: zeta = (b - a) / 2c,
-        // t = sign(zeta) / (|zeta| + sqrt(1 + zeta^2)), cs = 1/sqrt(1+t^2)
-        T cp = x[0][i] * x[0][j];
-#pragma unroll
-        for (int h = 1; h < R; ++h) cp = fma(x[h][i], x[h][j], cp);
-        const T c = group_sum<L>(cp);
-        const bool rot = c * c > tol2 * a[i] * a[j];
-        // Late in the iteration most pairs rotate in none of the wave's
-        // matrices; the update is then the identity (t = 0, cs = 1, sn = 0
-        // reproduce every value exactly) and is skipped for the whole wave.
-        if (!__any(rot)) continue;
-        const T zeta = (a[j] - a[i]) * rcp_(c + c);
-        const T den = fabs(zeta) + sqrt_(fma(zeta, zeta, T(1)));
-        const T t = rot ? copysign(rcp_(den), zeta) : T(0);
-        const T cs = rsq_(fma(t, t, T(1)));
-        const T sn = cs * t;
-#pragma unroll
-        for (int h = 0; h < R; ++h) {
-          const T xi = x[h][i], xj = x[h][j];
-          x[h][i] = cs * xi - sn * xj;
-          x[h][j] = sn * xi + cs * xj;
-        }
-        a[i] = fma(-t, c, a[i]);
-        a[j] = fma(t, c, a[j]);
-        tsum = fma(t, t, tsum);
-      }
-    }
-    if (!__any(tsum > T(0))) break;
-  }
-  if (stats && lane == 0 && valid) atomicMax(stats, (uint32_t)sweep + 1);
-  // final column norms (identical in every lane of the group)
-#pragma unroll
-  for (int k = 0; k < N; ++k) {
-    T t = x[0][k] * x[0][k];
-#pragma unroll
-    for (int h = 1; h < R; ++h) t = fma(x[h][k], x[h][k], t);
-    a[k] = group_sum<L>(t);
-  }
-  if (!valid) return;
-  // Store in descending singular-value order, transposed: row r of V^T is
-  // the right singular vector of the r-th largest singular value (row
-  // stride SR, padded with zeros), row r of W^T is the matching column of
-  // W = X V = U S (the rotated Casorati columns), then the sorted values.
-  // rank(l) counts the values that sort before column l (ties by index).
-  T* F = factors + (((size_t)b * nvar_stored + var) * p_sel + p) * fstride;
-  T* FW = F + n * SR;
-  T* FS = FW + n * M;
-  // ranks (< N <= 32) packed in bytes, four per register: the epilogue
-  // keeps X, 1/s^2 and the ranks live, and unpacked ranks would cost the
-  // kernel a wave per SIMD
-  uint32_t rk8[(N + 3) / 4];
-#pragma unroll
-  for (int i = 0; i < (N + 3) / 4; ++i) rk8[i] = 0u;
-  auto rank_of = [&](int l) -> int { return (int)((rk8[l / 4] >> (8 * (l % 4))) & 0xffu); };
-  T inv[N];
-  T amax = a[0];
-#pragma unroll
-  for (int k = 1; k < N; ++k) amax = fmax(amax, a[k]);
-  constexpr T eps = std::numeric_limits<T>::epsilon();
-#pragma unroll
-  for (int l = 0; l < N; ++l) {
-    // (RT: the zero columns past n rank after every real one)
-    uint32_t rl = 0;
-#pragma unroll
-    for (int m = 0; m < N; ++m) rl += (a[m] > a[l] || (a[m] == a[l] && m < l)) ? 1u : 0u;
-    rk8[l / 4] |= rl << (8 * (l % 4));
-    inv[l] = a[l] > eps * eps * amax ? T(1) / a[l] : T(0);
-    if (RT && l >= n) continue;
-#pragma unroll
-    for (int h = 0; h < R; ++h) {
-      const int q = lane + L * h;
-      if (q < M) FW[rl * M + q] = x[h][l];
-    }
-    if (lane == 0) FS[rl] = sqrt(a[l]);
-  }
-
-  // V^T, column by column: element k of v_l = X^T w_l / s_l^2 from column
-  // k of X (reloaded), stored by lane k % L
-#pragma unroll
-  for (int k = 0; k < SRN; ++k) {
-    if (RT && k >= SR) break;
-    if (k < n) {
-      const int32_t pk = pos[((size_t)b * nw + k) * p_all + it];
-      const uint32_t row = min((uint32_t)(pk & 0xffff), lim), col = min((uint32_t)(pk >> 16), lim);
-      T xk[R];
-#pragma unroll
-      for (int h = 0; h < R; ++h) {
-        const int q = lane + L * h;
-        xk[h] = q < M ? U[(size_t)k * fs + (row + q % BS) + (size_t)nr * (col + q / BS)] : T(0);
-      }
-#pragma unroll
-      for (int l = 0; l < N; ++l) {
-        if (RT && l >= n) break;  // uniform: the zero columns
-        T pv = xk[0] * x[0][l];
-#pragma unroll
-        for (int h = 1; h < R; ++h) pv = fma(xk[h], x[h][l], pv);
-        const T vk = group_sum<L>(pv) * inv[l];
-        const int rl = rank_of(l);
-        if (lane == k % L) F[rl * SR + k] = vk;
-      }
-    } else {
-#pragma unroll
-      for (int l = 0; l < N; ++l)
-        if ((!RT || l < n) && lane == k % L) F[rank_of(l) * SR + k] = T(0);
-    }
-  }
-}
-
 // Static data of the fused evaluation (patches up to 4 x 4 in FP64), from the U
 // variant's factors once the SVD is done: at the patch's bucket place
 // j_k = place[b][k][p] of every frame k, its rank-0 row w_0 v_0[k] into W0
@@ -979,7 +744,8 @@ __device__ __forceinline__ void block_count(double* out, int v) {
 //   B = U diag(g(s)) V^T = sum over kept ranks r of (g(s_r)/s_r) w_r v_r^T
 // with w_r = X v_r = s_r u_r, stored by the SVD.  Factors are sorted by
 // descending s and g(s)/s grows with s, so the kept ranks are a prefix and
-// only their rows are read.  Patches above 4 x 4: a group of L = 64 lanes
+// only their rows are read.  Patches above 4 x 4 in FP64 (FP32: k_round_prep
+// and the overlap-add): a group of L = 64 lanes
 // owns one patch, lane q one row of B; the U reconstruction's row of every
 // frame goes to its
 // bucket-sorted place in `B0` ([slot][frame][patch in bucket order][row])
@@ -1167,11 +933,10 @@ __device__ __forceinline__ V group_bcast(V v) {
 // w_r[q] t_q are formed in FP64 and stored with the variant's singular
 // values (zero-padded to sr): the search rounds read s and q of the three
 // variants from there.  L = 16: every row is loaded first; L = 64 (larger
-// patches, or windows above 16 frames): one rank at a time.  Patches up to
-// 4 x 4 (the fused evaluation) store rank-major planes divq
-// [nb][nvar][2][sr][p_sel] (s, then q), so that a round reads one coalesced
-// value per patch and kept rank; larger patches per-patch records divq
-// [nb][p_sel][nvar][2][sr].
+// patches, or windows above 16 frames): one rank at a time.  Stored as
+// rank-major planes divq [nb][nvar][2][sr][p_sel] (s, then q), so that a
+// round reads one coalesced value per patch and kept rank; FP64 patches
+// above 4 x 4 as per-patch records divq [nb][p_sel][nvar][2][sr].
 // RT: window length n = nw known at run time only (n <= N), as in k_svd.
 // Patches above 8 x 8 give each lane several rows of D (lane q rows q,
 // q + L, ...).
@@ -1259,7 +1024,7 @@ __global__ __launch_bounds__(256) void k_divq(const T* __restrict__ factors, con
     }
   }
   if (valid && lane < SR) {
-    if constexpr (BS <= 4) {
+    if constexpr (BS <= 4 || sizeof(T) == 4) {
       // rank-major planes [b][var][s | q][rank][patch] for the fused
       // evaluation: a search round reads only the ranks it keeps, one
       // coalesced value per patch
@@ -1274,14 +1039,16 @@ __global__ __launch_bounds__(256) void k_divq(const T* __restrict__ factors, con
   }
 }
 
-// Lambda evaluation for patches up to 4 x 4, per patch (one thread each).
+// Lambda evaluation per patch (one thread each; FP64: patches up to 4 x 4).
 // The reconstruction of a patch is B = sum_r d_r w_r v_r^T (src/svt.hpp:
 // 135-146 with src/utils.hpp:96-106), d_r = g(s_r)/s_r, w_r = X v_r = s_r u_r;
 // factors are sorted by descending s and g(s)/s grows with s, so the kept
 // ranks (d_r > 0) are a prefix.  FP32: the thread writes them to dr
-// [slot][r][p], d_0 negative when rank 1 is kept too, followed by a 0 when
-// fewer than n are kept; the overlap-add forms the rows from them and the
-// leading vectors and factors.  FP64: the gather forms d_0 and whether rank
+// [slot][r][p], followed by a 0 when fewer than n are kept; the overlap-add
+// forms the rows from them and the leading vectors and factors.  d_0 is
+// negative when rank 1 is kept too, and scaled by kStoredRow (a power of
+// two) when more than kInlineRanks are (patches above 4 x 4): k_rows then forms the patch's rows
+// of every frame once.  FP64: the gather forms d_0 and whether rank
 // 1 is kept itself, from the static singular pairs at every bucket place;
 // the thread writes the further kept ranks to dr [slot][p][r], r >= 1.
 // Either way the reconstruction itself is never written.  With PGURE (qdiv set) the thread also adds the
@@ -1336,7 +1103,7 @@ __global__ __launch_bounds__(256) void k_round_prep(const T* __restrict__ factor
     }
     if (v == 0 && dr) {
       if (r > 1 && r < n) dr[dr_at(r)] = T(0);  // end of the kept ranks
-      if (PLANES) dr[dr_at(0)] = r > 1 ? -first : first;
+      if (PLANES) dr[dr_at(0)] = BS > 4 && r > kInlineRanks ? -first * T(kStoredRow) : r > 1 ? -first : first;
     }
     kr += r;
   }
@@ -1348,6 +1115,83 @@ __global__ __launch_bounds__(256) void k_round_prep(const T* __restrict__ factor
     if (threadIdx.x == 0) partial[(size_t)slot * gridDim.x + blockIdx.x] = ((red[0] + red[1]) + red[2]) + red[3];
   }
   if (kept) block_count(kept + (size_t)slot * gridDim.x + blockIdx.x, kr);
+}
+
+// Rows of the patches that keep more than kInlineRanks ranks (d_0 marked by
+// k_round_prep), all frames, by patch: rows [slot][frame][p][row], read by
+// the overlap-add.  Inline, a patch's row of every frame would read each
+// kept rank's w_r again; here a wave holds them for all frames.  A wave
+// looks at 16 patches and works off those marked, lane q on row q of B
+// (rows q, q + 64, ... above 8 x 8), the chain of the inline form.
+// RT: window length n = nw at run time (n <= N).
+template <int BS, int N, bool RT = false>
+__global__ __launch_bounds__(256) void k_rows(const float* __restrict__ factors, const float* __restrict__ dr,
+                                              const uint32_t* __restrict__ wl, uint32_t nvar_stored, uint32_t p_sel,
+                                              uint32_t nw, uint32_t fstride, float* __restrict__ rows) {
+  constexpr int M = BS * BS, SRN = (N + 3) & ~3, RQ = (M + 63) / 64, NV = SRN / 4;
+  const int n = RT ? (int)nw : N;
+  const int SR = RT ? ((n + 3) & ~3) : SRN;
+  const uint32_t slot = blockIdx.y, b = wl[slot];
+  const int lane = (int)(threadIdx.x % 64);
+  const uint32_t p0 = (blockIdx.x * 4 + threadIdx.x / 64) * 16;
+  const float* D = dr + (size_t)slot * nw * p_sel;
+  const float first = (lane < 16 && p0 + lane < p_sel) ? D[p0 + lane] : 0.f;
+  uint64_t todo = __ballot(first < -2.f);
+  while (todo) {
+    const int l = __ffsll((unsigned long long)todo) - 1;
+    todo &= todo - 1;
+    const uint32_t p = p0 + (uint32_t)l;
+    const float* F = factors + ((size_t)b * nvar_stored * p_sel + p) * fstride;  // the U variant
+    const float* FW = F + n * SR;
+    float dl = lane < n ? D[(size_t)lane * p_sel + p] : 0.f;
+    if (lane == 0) dl = -dl * (1.f / kStoredRow);
+    // the kept ranks are a prefix, a 0 behind it
+    const int nkeep = __ffsll((unsigned long long)~__ballot(dl > 0.f)) - 1;
+    float bq[RQ][N];
+#pragma unroll
+    for (int h = 0; h < RQ; ++h)
+#pragma unroll
+      for (int k = 0; k < N; ++k) bq[h][k] = 0.f;
+    // rank loop, loads of rank r + 1 issued before the products of rank r
+    float wn[RQ];
+    float4 vn[NV];
+    auto fetch = [&](int r) {
+#pragma unroll
+      for (int h = 0; h < RQ; ++h) wn[h] = lane + 64 * h < M ? FW[r * M + lane + 64 * h] : 0.f;
+      const float4* vr = reinterpret_cast<const float4*>(F + r * SR);
+#pragma unroll
+      for (int j = 0; j < NV; ++j) vn[j] = vr[j];
+    };
+    fetch(0);
+    for (int r = 0; r < nkeep; ++r) {
+      const float d = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, dl), r));
+      float y[RQ];
+#pragma unroll
+      for (int h = 0; h < RQ; ++h) y[h] = d * wn[h];
+      float4 vc[NV];
+#pragma unroll
+      for (int j = 0; j < NV; ++j) vc[j] = vn[j];
+      if (r + 1 < nkeep) fetch(r + 1);
+#pragma unroll
+      for (int h = 0; h < RQ; ++h) {
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+          const float t[4] = {vc[j].x, vc[j].y, vc[j].z, vc[j].w};
+#pragma unroll
+          for (int z = 0; z < 4; ++z)
+            if (4 * j + z < N) bq[h][4 * j + z] = fmaf(y[h], t[z], bq[h][4 * j + z]);
+        }
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      if (RT && k >= n) break;
+      const size_t at = (((size_t)slot * nw + k) * p_sel + p) * M;
+#pragma unroll
+      for (int h = 0; h < RQ; ++h)
+        if (lane + 64 * h < M) rows[at + lane + 64 * h] = bq[h][k];
+    }
+  }
 }
 
 // ----------------------------------------------------------- gather --
@@ -1777,118 +1621,8 @@ __global__ __launch_bounds__(256) void k_risk_reduce(const double* __restrict__ 
   if (threadIdx.x < 6) sums[(size_t)slot * 6 + threadIdx.x] = sm[threadIdx.x][0];
 }
 
-// shape table of the instantiated SVD / evaluation kernels (patch size,
-// window frames, lanes per patch in the evaluation, lanes per matrix in the
-// SVD)
-#define PG_SHAPES(X) \
-  X(4, 3, 16, 4) X(4, 5, 16, 4) X(4, 7, 16, 4) X(4, 9, 16, 4) X(4, 11, 16, 4) X(4, 13, 16, 4) X(4, 15, 16, 4) \
-  X(2, 3, 16, 4) X(3, 3, 16, 4) X(3, 5, 16, 4) X(3, 7, 16, 4) X(3, 9, 16, 4) \
-  X(6, 7, 64, 16) X(6, 15, 64, 16) X(6, 31, 64, 32) X(8, 7, 64, 16) X(8, 15, 64, 16) X(8, 31, 64, 32)
-
-// second lanes-per-matrix mapping of the SVD for each shape, timed against
-// the first by the autotuner of the batched path
-#define PG_SVD_ALT(X) \
-  X(4, 3, 8) X(4, 5, 8) X(4, 7, 8) X(4, 9, 8) X(4, 11, 8) X(4, 13, 8) X(4, 15, 8) \
-  X(2, 3, 2) X(3, 3, 8) X(3, 5, 8) X(3, 7, 8) X(3, 9, 8) \
-  X(6, 7, 32) X(6, 15, 32) X(6, 31, 64) X(8, 7, 32) X(8, 15, 32) X(8, 31, 64)
-
-// Every other shape, FP32 only: the window length is known at run time
-// (the kernels' RT form) up to NM frames.  (patch size, NM, lanes per
-// matrix in the SVD, lanes per patch in the divergence factors and, for
-// patches above 4 x 4, the evaluation; patches up to 4 x 4 evaluate fused,
-// one thread per patch)
-#define PG_GENERIC(X) \
-  X(2, 16, 4, 16) X(3, 16, 4, 16) X(4, 16, 4, 16) \
-  X(5, 16, 16, 64) X(5, 32, 16, 64) X(6, 16, 16, 64) X(6, 32, 32, 64) X(7, 16, 16, 64) X(7, 32, 32, 64) \
-  X(8, 16, 32, 64) X(8, 32, 64, 64) X(16, 16, 64, 64)
-
-bool shape_exact(uint32_t bs, uint32_t nw) {
-#define PG_CHK(B, N, L, LS) \
-  if (bs == B && nw == N) return true;
-  PG_SHAPES(PG_CHK)
-#undef PG_CHK
-  return false;
-}
-
-// the generic family that runs a shape: its NM, or 0
-uint32_t shape_generic(uint32_t bs, uint32_t nw) {
-  if (nw < 1) return 0;
-#define PG_GCHK(B, NM, L, LE) \
-  if (bs == B && nw <= NM) return NM;
-  PG_GENERIC(PG_GCHK)
-#undef PG_GCHK
-  return 0;
-}
-
-uint32_t svd_lanes(uint32_t bs, uint32_t nw, int which) {
-#define PG_L1(B, N, LE, L) \
-  if (which == 0 && bs == B && nw == N) return L;
-  PG_SHAPES(PG_L1)
-#undef PG_L1
-#define PG_L2(B, N, L) \
-  if (which == 1 && bs == B && nw == N) return L;
-  PG_SVD_ALT(PG_L2)
-#undef PG_L2
-  return 0;
-}
-
 bool svd_shape_supported(uint32_t bs, uint32_t nw, bool fp64) {
   return shape_exact(bs, nw) || (!fp64 && shape_generic(bs, nw) != 0);
-}
-
-hipError_t launch_svd(const void* uvar, const int32_t* pos, const uint32_t* sel, uint32_t nb, uint32_t nvar,
-                      uint32_t nvar_stored, const Shape& sh, void* factors, int max_sweeps, double tol,
-                      uint32_t* stats, hipStream_t s, int mapping) {
-  if (nvar > nvar_stored) return hipErrorInvalidValue;
-  const uint32_t lim = sh.nr - sh.bs;
-  const uint32_t groups = nvar * sh.p_sel;
-#define PG_SVD_F32(B, N, L)                                                                                      \
-  {                                                                                                            \
-    const dim3 grid((groups * L + 255) / 256, nb);                                                             \
-    hipLaunchKernelGGL((k_svd<B, N, L, float>), grid, dim3(256), 0, s, (const float*)uvar, pos, sel, nvar,     \
-                       nvar_stored, sh.p_sel, sh.p_all, sh.nr, sh.fs, sh.nw, sh.vol, lim, sh.fstride, max_sweeps,            \
-                       (float)(tol * tol), (float*)factors, stats);                                                \
-    return hipGetLastError();                                                                                  \
-  }
-#define PG_SVD(B, N, LE, L)                                                                                      \
-  if (sh.bs == B && sh.nw == N && (sh.fp64 || mapping == 0)) {                                                 \
-    if (sh.fp64) {                                                                                             \
-      /* FP64: at least 16 lanes per matrix (fewer rows per lane fit the registers); the 64-row matrices     \
-         of patch 8 take 32 (15 frames) and 64 (31 frames) */                                                  \
-      constexpr int LD = (B == 8 && N == 31) ? 64 : (B == 8 && N == 15) ? 32 : (L < 16 ? 16 : L);            \
-      const dim3 grid((groups * LD + 255) / 256, nb);                                                          \
-      hipLaunchKernelGGL((k_svd<B, N, LD, double>), grid, dim3(256), 0, s, (const double*)uvar, pos, sel, nvar, \
-                         nvar_stored, sh.p_sel, sh.p_all, sh.nr, sh.fs, sh.nw, sh.vol, lim, sh.fstride, max_sweeps, tol * tol, \
-                         (double*)factors, stats);                                                               \
-      return hipGetLastError();                                                                                \
-    }                                                                                                          \
-    PG_SVD_F32(B, N, L)                                                                                        \
-  }
-  PG_SHAPES(PG_SVD)
-#undef PG_SVD
-#define PG_SVD2(B, N, L)                                                                                         \
-  if (sh.bs == B && sh.nw == N && mapping == 1) PG_SVD_F32(B, N, L)
-  PG_SVD_ALT(PG_SVD2)
-#undef PG_SVD2
-  // an exact shape without an alternative mapping: the primary one
-#define PG_SVD3(B, N, LE, L)                                                                                     \
-  if (sh.bs == B && sh.nw == N && !sh.fp64) PG_SVD_F32(B, N, L)
-  PG_SHAPES(PG_SVD3)
-#undef PG_SVD3
-#undef PG_SVD_F32
-  if (sh.fp64) return hipErrorInvalidValue;
-  const uint32_t nm = shape_generic(sh.bs, sh.nw);
-#define PG_SVDG(B, NM, L, LE)                                                                                    \
-  if (sh.bs == B && nm == NM) {                                                                                \
-    const dim3 grid((groups * L + 255) / 256, nb);                                                             \
-    hipLaunchKernelGGL((k_svd<B, NM, L, float, true>), grid, dim3(256), 0, s, (const float*)uvar, pos, sel,    \
-                       nvar, nvar_stored, sh.p_sel, sh.p_all, sh.nr, sh.fs, sh.nw, sh.vol, lim, sh.fstride, max_sweeps,      \
-                       (float)(tol * tol), (float*)factors, stats);                                                \
-    return hipGetLastError();                                                                                  \
-  }
-  PG_GENERIC(PG_SVDG)
-#undef PG_SVDG
-  return hipErrorInvalidValue;
 }
 
 hipError_t launch_static_rows(const void* factors, const int32_t* place, uint32_t nb, uint32_t nvar_stored,
@@ -1909,7 +1643,9 @@ hipError_t launch_static_rows(const void* factors, const int32_t* place, uint32_
 
 bool fused_eval(const Shape& sh) { return sh.bs <= 4; }
 
-bool strip_overlap(const Shape& sh) { return sh.bs <= 4 && !sh.fp64; }
+bool strip_overlap(const Shape& sh) { return !sh.fp64; }
+
+bool stored_rows(const Shape& sh) { return strip_overlap(sh) && sh.bs > 4; }
 
 uint32_t factor_stride(uint32_t nw, uint32_t m) {
   const uint32_t sr = (nw + 3) & ~3u;
@@ -1917,20 +1653,50 @@ uint32_t factor_stride(uint32_t nw, uint32_t m) {
 }
 
 uint32_t eval_blocks(const Shape& sh, uint32_t nvar_run) {
-  (void)nvar_run;  // one group (one thread with the fused gather) per patch either way
-  if (fused_eval(sh)) return (sh.p_sel + 255) / 256;
+  (void)nvar_run;  // one thread per patch, or one 64-lane group, either way
+  if (fused_eval(sh) || strip_overlap(sh)) return (sh.p_sel + 255) / 256;
   return (sh.p_sel + 3) / 4;  // one 64-lane group per patch
+}
+
+// the rows of the marked patches (see k_rows)
+static hipError_t launch_rows(const float* factors, const float* dr, const uint32_t* wl, uint32_t na,
+                              uint32_t nvar_stored, const Shape& sh, float* rows, hipStream_t s) {
+  const dim3 grid((sh.p_sel + 63) / 64, na);
+#define PG_RW(B, N, L, LS)                                                                                       \
+  if constexpr (B > 4) {                                                                                       \
+    if (sh.bs == B && sh.nw == N) {                                                                            \
+      hipLaunchKernelGGL((k_rows<B, N>), grid, dim3(256), 0, s, factors, dr, wl, nvar_stored, sh.p_sel, sh.nw,  \
+                         sh.fstride, rows);                                                                    \
+      return hipGetLastError();                                                                                \
+    }                                                                                                          \
+  }
+  PG_SHAPES(PG_RW)
+#undef PG_RW
+  const uint32_t nm = shape_generic(sh.bs, sh.nw);
+#define PG_RWG(B, NM, L, LE)                                                                                     \
+  if constexpr (B > 4) {                                                                                       \
+    if (sh.bs == B && nm == NM) {                                                                              \
+      hipLaunchKernelGGL((k_rows<B, NM, true>), grid, dim3(256), 0, s, factors, dr, wl, nvar_stored, sh.p_sel,  \
+                         sh.nw, sh.fstride, rows);                                                             \
+      return hipGetLastError();                                                                                \
+    }                                                                                                          \
+  }
+  PG_GENERIC(PG_RWG)
+#undef PG_RWG
+  return hipErrorInvalidValue;
 }
 
 hipError_t launch_evaluation(const Shape& sh, const void* factors, const void* divq, const WinMeta* meta,
                              const uint32_t* wl, uint32_t na, uint32_t nvar_stored, uint32_t nvar_run, int exp_w,
-                             const int32_t* inv, void* rows, double* partial, const double* slot_lam, double* kept,
-                             hipStream_t s) {
-  if (fused_eval(sh))
-    return launch_round_prep(factors, nvar_run == 3 ? divq : nullptr, meta, wl, na, nvar_stored, sh, exp_w,
-                             slot_lam, rows, nvar_run == 3 ? partial : nullptr, kept, s);
-  return launch_eval(factors, meta, wl, na, nvar_stored, nvar_run, sh, exp_w, divq, inv, rows, partial, s, slot_lam,
-                     kept);
+                             const int32_t* inv, void* dr, void* rows, double* partial, const double* slot_lam,
+                             double* kept, hipStream_t s) {
+  if (!fused_eval(sh) && !strip_overlap(sh))
+    return launch_eval(factors, meta, wl, na, nvar_stored, nvar_run, sh, exp_w, divq, inv, rows, partial, s, slot_lam,
+                       kept);
+  const hipError_t e = launch_round_prep(factors, nvar_run == 3 ? divq : nullptr, meta, wl, na, nvar_stored, sh, exp_w,
+                                         slot_lam, dr, nvar_run == 3 ? partial : nullptr, kept, s);
+  if (e != hipSuccess || !stored_rows(sh)) return e;
+  return launch_rows((const float*)factors, (const float*)dr, wl, na, nvar_stored, sh, (float*)rows, s);
 }
 
 size_t singular_pair_bytes(const Shape& sh) { return (size_t)sh.nw * sh.p_sel * 2 * (sh.fp64 ? 8 : 4); }
@@ -1941,30 +1707,28 @@ hipError_t launch_round_prep(const void* factors, const void* qdiv, const WinMet
   const uint32_t nblk = eval_blocks(sh, 1);
 #define PG_RP(B, N, L, LS)                                                                                       \
   if (sh.bs == B && sh.nw == N) {                                                                              \
-    if constexpr (B <= 4) {                                                                                    \
-      if (sh.fp64)                                                                                             \
-        hipLaunchKernelGGL((k_round_prep<B, N, double>), dim3(nblk, na), dim3(256), 0, s,                      \
-                           (const double*)factors, (const double*)qdiv, meta, wl, nvar_stored, sh.p_sel, sh.nw, \
-                           sh.fstride, exp_w, slot_lam, (double*)dr, partial, kept);                            \
-      else                                                                                                     \
-        hipLaunchKernelGGL((k_round_prep<B, N, float>), dim3(nblk, na), dim3(256), 0, s, (const float*)factors, \
-                           (const float*)qdiv, meta, wl, nvar_stored, sh.p_sel, sh.nw, sh.fstride, exp_w,       \
-                           slot_lam, (float*)dr, partial, kept);                                                \
-      return hipGetLastError();                                                                                \
-    }                                                                                                          \
+    if (!sh.fp64)                                                                                              \
+      hipLaunchKernelGGL((k_round_prep<B, N, float>), dim3(nblk, na), dim3(256), 0, s, (const float*)factors,   \
+                         (const float*)qdiv, meta, wl, nvar_stored, sh.p_sel, sh.nw, sh.fstride, exp_w,         \
+                         slot_lam, (float*)dr, partial, kept);                                                 \
+    else if constexpr (B <= 4)                                                                                 \
+      hipLaunchKernelGGL((k_round_prep<B, N, double>), dim3(nblk, na), dim3(256), 0, s,                        \
+                         (const double*)factors, (const double*)qdiv, meta, wl, nvar_stored, sh.p_sel, sh.nw,   \
+                         sh.fstride, exp_w, slot_lam, (double*)dr, partial, kept);                              \
+    else                                                                                                       \
+      return hipErrorInvalidValue;                                                                             \
+    return hipGetLastError();                                                                                  \
   }
   PG_SHAPES(PG_RP)
 #undef PG_RP
   if (sh.fp64) return hipErrorInvalidValue;
   const uint32_t nm = shape_generic(sh.bs, sh.nw);
 #define PG_RPG(B, NM, L, LE)                                                                                     \
-  if constexpr (B <= 4) {                                                                                      \
-    if (sh.bs == B && nm == NM) {                                                                              \
-      hipLaunchKernelGGL((k_round_prep<B, NM, float, true>), dim3(nblk, na), dim3(256), 0, s,                  \
-                         (const float*)factors, (const float*)qdiv, meta, wl, nvar_stored, sh.p_sel, sh.nw,     \
-                         sh.fstride, exp_w, slot_lam, (float*)dr, partial, kept);                               \
-      return hipGetLastError();                                                                                \
-    }                                                                                                          \
+  if (sh.bs == B && nm == NM) {                                                                                \
+    hipLaunchKernelGGL((k_round_prep<B, NM, float, true>), dim3(nblk, na), dim3(256), 0, s,                    \
+                       (const float*)factors, (const float*)qdiv, meta, wl, nvar_stored, sh.p_sel, sh.nw,       \
+                       sh.fstride, exp_w, slot_lam, (float*)dr, partial, kept);                                 \
+    return hipGetLastError();                                                                                  \
   }
   PG_GENERIC(PG_RPG)
 #undef PG_RPG
@@ -1977,35 +1741,18 @@ hipError_t launch_eval(const void* factors, const WinMeta* meta, const uint32_t*
                        double* kept) {
   if (nvar_run == 3 && !divq) return hipErrorInvalidValue;  // launch_divq after the SVD
   const uint32_t nblk = eval_blocks(sh, nvar_run);
+  if (!sh.fp64) return hipErrorInvalidValue;
 #define PG_EV(B, N, L, LS)                                                                                       \
-  if (sh.bs == B && sh.nw == N) {                                                                              \
-    if constexpr (L == 64) {                                                                                   \
-      if (sh.fp64)                                                                                             \
-        hipLaunchKernelGGL((k_eval<B, N, L, double>), dim3(nblk, na), dim3(256), 0, s, (const double*)factors,  \
-                           meta, wl, nvar_stored, nvar_run, sh.p_sel, sh.nw, sh.fstride, exp_w,                 \
-                           (const double*)divq, inv, (double*)B0, partial, slot_lam, kept);                    \
-      else                                                                                                     \
-        hipLaunchKernelGGL((k_eval<B, N, L, float>), dim3(nblk, na), dim3(256), 0, s, (const float*)factors,    \
-                           meta, wl, nvar_stored, nvar_run, sh.p_sel, sh.nw, sh.fstride, exp_w,                 \
-                           (const float*)divq, inv, (float*)B0, partial, slot_lam, kept);                      \
+  if constexpr (L == 64) {                                                                                     \
+    if (sh.bs == B && sh.nw == N) {                                                                            \
+      hipLaunchKernelGGL((k_eval<B, N, L, double>), dim3(nblk, na), dim3(256), 0, s, (const double*)factors,    \
+                         meta, wl, nvar_stored, nvar_run, sh.p_sel, sh.nw, sh.fstride, exp_w,                   \
+                         (const double*)divq, inv, (double*)B0, partial, slot_lam, kept);                      \
       return hipGetLastError();                                                                                \
     }                                                                                                          \
   }
   PG_SHAPES(PG_EV)
 #undef PG_EV
-  if (sh.fp64) return hipErrorInvalidValue;
-  const uint32_t nm = shape_generic(sh.bs, sh.nw);
-#define PG_EVG(B, NM, L, LE)                                                                                     \
-  if constexpr (LE == 64 && B > 4) {                                                                           \
-    if (sh.bs == B && nm == NM) {                                                                              \
-      hipLaunchKernelGGL((k_eval<B, NM, LE, float, true>), dim3(nblk, na), dim3(256), 0, s,                    \
-                         (const float*)factors, meta, wl, nvar_stored, nvar_run, sh.p_sel, sh.nw, sh.fstride,   \
-                         exp_w, (const float*)divq, inv, (float*)B0, partial, slot_lam, kept);                 \
-      return hipGetLastError();                                                                                \
-    }                                                                                                          \
-  }
-  PG_GENERIC(PG_EVG)
-#undef PG_EVG
   return hipErrorInvalidValue;
 }
 
@@ -2061,9 +1808,9 @@ hipError_t launch_gather(const GatherSrc& src, const int32_t* off, const double*
                          double* partial, hipStream_t s, uint32_t nk) {
   const uint32_t nblk = gather_blocks(sh, mode, nk);
   const uint32_t nkk = (mode == 1) ? 1 : gather_frames(sh, nk);
+  if (!sh.fp64) return hipErrorInvalidValue;  // launch_overlap
 #define PG_GT(B)                                                                                                 \
   case B:                                                                                                      \
-    if (!sh.fp64) return hipErrorInvalidValue; /* launch_overlap */                                            \
     hipLaunchKernelGGL((k_gather_tile<B, double>), dim3(nblk, na), dim3(256), 0, s, (const double*)src.factors,  \
                        (const double*)src.dr, (const double*)src.S01, (const double*)src.W0, src.list, off,     \
                        invw, u64, meta, wl, src.slot_lam, src.exp_w, sh.nr, sh.fs, sh.nw, sh.vol, sh.n1,        \
@@ -2071,18 +1818,12 @@ hipError_t launch_gather(const GatherSrc& src, const int32_t* off, const double*
     break;
 #define PG_GA(B)                                                                                                 \
   case B:                                                                                                      \
-    if (sh.fp64)                                                                                               \
-      hipLaunchKernelGGL((k_gather_direct<B, double>), dim3(nblk, na), dim3(256), 0, s, (const double*)src.B0,   \
-                         off, invw, u64, meta, wl, sh.nr, sh.fs, sh.nw, sh.vol, sh.n1, sh.p_sel, mode, out,      \
-                         partial);                                                                             \
-    else                                                                                                       \
-      hipLaunchKernelGGL((k_gather_direct<B, float>), dim3(nblk, na), dim3(256), 0, s, (const float*)src.B0,     \
-                         off, invw, u64, meta, wl, sh.nr, sh.fs, sh.nw, sh.vol, sh.n1, sh.p_sel, mode, out,      \
-                         partial);                                                                             \
+    hipLaunchKernelGGL((k_gather_direct<B, double>), dim3(nblk, na), dim3(256), 0, s, (const double*)src.B0, off, \
+                       invw, u64, meta, wl, sh.nr, sh.fs, sh.nw, sh.vol, sh.n1, sh.p_sel, mode, out, partial);   \
     break;
   switch (sh.bs) {
     PG_GT(2) PG_GT(3) PG_GT(4)
-    PG_GA(5) PG_GA(6) PG_GA(7) PG_GA(8) PG_GA(16)
+    PG_GA(6) PG_GA(8)
     default: return hipErrorInvalidValue;
   }
 #undef PG_GA

@@ -77,26 +77,26 @@ hipError_t launch_eval(const void* factors, const WinMeta* meta, const uint32_t*
 // its singular values (zero-padded) then its factors
 hipError_t launch_divq(const void* factors, const int32_t* pos, const uint32_t* sel, const void* dw, uint32_t nb,
                        uint32_t nvar, const Shape& sh, void* divq, hipStream_t s);
-// Patches up to 4 x 4 evaluate lambda in two launches: launch_round_prep
+// FP32, and patches up to 4 x 4 in FP64, evaluate lambda in two launches: launch_round_prep
 // (the factors d_r of the kept ranks into dr; with PGURE (qdiv = divq) the
 // divergence sums into partial [na][eval_blocks]), then launch_overlap, or
 // in FP64 (dr [na][p_sel][nw], of ranks after the first) launch_gather,
 // which forms d_0 and the patch rows from the window's static singular
 // pairs and rows (written by launch_static_rows: S01 [nb][nw][p_sel][2], W0
 // [nb][nw][p_sel][m] in bucket order; singular_pair_bytes per window), dr
-// and the factors as it gathers.  Larger patches: launch_eval writes the
-// rows to B0, launch_gather reads them.
+// and the factors as it gathers.  Larger FP64 patches:
+// launch_eval writes the rows to B0, launch_gather reads them.
 bool fused_eval(const Shape& sh);
 size_t singular_pair_bytes(const Shape& sh);
 hipError_t launch_round_prep(const void* factors, const void* qdiv, const WinMeta* meta, const uint32_t* wl,
                              uint32_t na, uint32_t nvar_stored, const Shape& sh, int exp_w, const double* slot_lam,
                              void* dr, double* partial, double* kept, hipStream_t s);
-// One lambda evaluation of the listed slots, either form: `rows` is dr
-// (fused) or B0.
+// One lambda evaluation of the listed slots, either form (dr unused by
+// launch_eval, rows = B0 by the fused FP64 form).
 hipError_t launch_evaluation(const Shape& sh, const void* factors, const void* divq, const WinMeta* meta,
                              const uint32_t* wl, uint32_t na, uint32_t nvar_stored, uint32_t nvar_run, int exp_w,
-                             const int32_t* inv, void* rows, double* partial, const double* slot_lam, double* kept,
-                             hipStream_t s);
+                             const int32_t* inv, void* dr, void* rows, double* partial, const double* slot_lam,
+                             double* kept, hipStream_t s);
 // what the gather reads: fused (bs <= 4) the factors, dr, the static
 // singular pairs and rows with the bucket lists, and the lambdas (slot_lam
 // per slot, or the windows' meta) with the weighting; otherwise the rows B0
@@ -129,18 +129,22 @@ uint32_t gather_blocks(const Shape& sh, int mode, uint32_t nk = 0);
 hipError_t launch_gather(const GatherSrc& src, const int32_t* off, const double* invw, const double* u64,
                          const WinMeta* meta, const uint32_t* wl, uint32_t na, const Shape& sh, int mode, double* out,
                          double* partial, hipStream_t s, uint32_t nk = 0);
-// The FP32 overlap-add of patches up to 4 x 4 (overlap.hip) needs neither
-// position buckets nor rows per bucket place: launch_bins sorts every
-// frame's patches by the column of their position (recs [nb][nw][p_sel] =
-// (position, patch), off [nb][nw][column_bins + 1]), launch_cover makes 1/W
-// and delta2/W from them, launch_lead lays the U variant's w_0 (w0
-// [nb][p_sel][m]) and v_0 (v0 [nb][nw][p_sel]) out by patch, and
-// launch_overlap adds the rows up, with d_r from launch_round_prep (dr
-// [na][nw][p_sel], by rank: d_0, negative where rank 1 is kept too, then
-// the further kept ranks, ended by a 0).  wstat [nb][2]: the window's
+// The FP32 overlap-add (overlap.hip) needs neither position buckets nor rows
+// per bucket place: launch_bins sorts every frame's patches by the column of
+// their position (recs [nb][nw][p_sel] = (position, patch), off
+// [nb][nw][column_bins + 1]), launch_cover makes 1/W and delta2/W from them,
+// launch_lead lays the U variant's v_0 (v0 [nb][nw][p_sel]) and, for patches
+// up to 4 x 4, w_0 (w0 [nb][p_sel][m]; null for larger ones) out by patch, and launch_overlap adds the rows up, with
+// d_r from launch_evaluation (dr [na][nw][p_sel], by rank, ended by a 0; d_0
+// negative where rank 1 is kept too) and, for patches above 4 x 4 that keep
+// more than kInlineRanks ranks (d_0 scaled by kStoredRow), their rows of
+// every frame (rows [na][nw][p_sel][m]).  wstat [nb][2]: the window's
 // largest s_0 (bits of a float) and largest W; zeroed by the caller before
 // launch_cover and launch_lead raise them.  Modes and nk as launch_gather.
+constexpr int kInlineRanks = 6;
+constexpr float kStoredRow = 18446744073709551616.f;  // 2^64
 bool strip_overlap(const Shape& sh);
+bool stored_rows(const Shape& sh);  // it may read rows (patches above 4 x 4)
 uint32_t column_bins(const Shape& sh);
 hipError_t launch_bins(const int32_t* pos, const uint32_t* sel, uint32_t nb, const Shape& sh, int32_t* off,
                        int2* recs, hipStream_t s);
@@ -149,7 +153,7 @@ hipError_t launch_cover(const int32_t* off, const int2* recs, const uint8_t* d2,
 hipError_t launch_lead(const float* factors, uint32_t nb, uint32_t nvar_stored, const Shape& sh, float* w0, float* v0,
                        uint32_t* wstat, hipStream_t s);
 struct OverlapSrc {
-  const float *factors = nullptr, *dr = nullptr, *w0 = nullptr, *v0 = nullptr;
+  const float *factors = nullptr, *dr = nullptr, *rows = nullptr, *w0 = nullptr, *v0 = nullptr;
   const int2* recs = nullptr;
   const int32_t* off = nullptr;
   const uint32_t* wstat = nullptr;

@@ -21,16 +21,18 @@ namespace {
 // KB.  Frames above 1,024 rows take up to 7,600 cells (within 64 KB) and 512
 // threads, or their halo (bs - 1 columns) would outweigh the strip.  Small
 // frames take fewer columns a strip, so that a call of a few windows still
-// has a workgroup for every CU.
+// has a workgroup for every CU; patches above 4 x 4, with a wider halo,
+// more.
 struct Strips {
   uint32_t tr, tc, ld, nr, nc, threads;  // ld: column stride in LDS; nr x nc strips a frame
 };
-Strips strips_of(uint32_t n) {
+Strips strips_of(uint32_t n, uint32_t bs) {
   Strips s;
   s.tr = std::min(n, 2048u);
   const uint32_t cells = s.tr <= 1024 ? 4096 : 7600;
   s.threads = s.tr <= 1024 ? 256 : 512;
-  s.tc = std::max(1u, std::min({cells / s.tr, 16u, std::max(4u, n / 8)}));
+  s.tc = std::max(1u, bs <= 4 ? std::min({cells / s.tr, 16u, std::max(4u, n / 8)})
+                              : std::min({cells / s.tr, 32u, std::max(8u, n / 4)}));
   // 8 lanes of a half-wave's row group and the 4 patch columns of a row
   // meet in distinct banks when the stride is 8 mod 32 cells
   s.ld = ((s.tr + 23) / 32) * 32 + 8;
@@ -181,7 +183,8 @@ __global__ __launch_bounds__(256) void k_cover(const int2* __restrict__ recs, co
 }
 
 // ---------------------------------------------------- leading vectors --
-// By patch, from the U variant's factors: w_0 (w0 [nb][p_sel][m]) and v_0 as
+// By patch, from the U variant's factors: w_0 (w0 [nb][p_sel][m], may be
+// null) and v_0 as
 // one plane per frame (v0 [nb][nw][p_sel]), and the window's largest finite
 // s_0 (wstat[2 b], as the bits of a non-negative float).  A workgroup takes
 // 64 patches: 16 lanes read a patch's vectors, v_0 turns in LDS, so that
@@ -199,7 +202,8 @@ __global__ __launch_bounds__(256) void k_lead(const float* __restrict__ factors,
     if (p >= p_sel) continue;
     const float* F = factors + ((size_t)b * nvar_stored * p_sel + p) * fstride;
     const float* FW = F + nw * SR;
-    for (uint32_t i = l; i < m; i += 16) w0[((size_t)b * p_sel + p) * m + i] = FW[i];
+    if (w0)
+      for (uint32_t i = l; i < m; i += 16) w0[((size_t)b * p_sel + p) * m + i] = FW[i];
     for (uint32_t k = l; k < nw; k += 16) tv[k][pl] = F[k];
     if (l == 0) {
       const uint32_t u = __float_as_uint(FW[nw * m]);
@@ -219,7 +223,7 @@ __global__ __launch_bounds__(256) void k_lead(const float* __restrict__ factors,
 
 // --------------------------------------------------------- overlap-add --
 struct OverlapArgs {
-  const float *factors, *dr, *w0, *v0;
+  const float *factors, *dr, *rows, *w0, *v0;
   const int2* recs;
   const int32_t* off;
   const double *invw, *u64;
@@ -260,11 +264,12 @@ __device__ __forceinline__ void load_run(const float* __restrict__ p, float (&x)
 // Uhat = (sum of the patches' rows over each voxel) / W.  The row of patch p
 // in frame k is B[q][k] = d_0 (w_0[q] v_0[k]), then fma(d_r w_r[q], v_r[k],
 // .) over further kept ranks, FP32, in rank order; d_r by rank and patch
-// from k_round_prep, d_0 negative when rank 1 is kept too.
+// from k_round_prep, d_0 negative when rank 1 is kept too.  Patches above 4
+// x 4 take (d_0 w_0[q]) v_0[k], and where d_0 is marked the row that k_rows
+// stored.
 //
 // A workgroup owns a strip of one frame and walks the records of the patches
-// that reach it, 4 lanes to a patch (one per patch column of BS elements),
-// adding each element to the strip's cells in LDS as a 64-bit integer: x is
+// that reach it, one lane per patch column of BS elements, adding each element to the strip's cells in LDS as a 64-bit integer: x is
 // rounded to a multiple of a quantum q (x + 1.5 2^52 q leaves the multiple
 // in the low bits of the double) and the integers are added by ds_add_u64.
 // Integer sums are the same in every order, so the result is reproducible
@@ -328,9 +333,12 @@ __global__ __launch_bounds__(512) void k_overlap(const OverlapArgs a) {
   const float* D = a.dr + (size_t)slot * a.nw * a.p_sel;  // [rank][patch]
   const float* V = a.v0 + tab * a.p_sel;
   const int cb = (int)(threadIdx.x % LG), grp = (int)(threadIdx.x / LG), G = (int)(blockDim.x / LG);
-  const float* W = a.w0 + (size_t)b * a.p_sel * M + cb * BS;
   const uint32_t sr = (a.nw + 3) & ~3u;
   const float* Fu = a.factors + (size_t)b * a.nvar_stored * a.p_sel * a.fstride;  // the U variant
+  // w_0 by patch: a 4 x 4 patch's 64 bytes share a cache line with its
+  // neighbour's in w0, larger ones fill their lines in the factors
+  const float* W = BS <= 4 ? a.w0 + (size_t)b * a.p_sel * M : Fu + a.nw * sr;
+  const size_t wst = BS <= 4 ? M : a.fstride;
   // further kept ranks of patch id, elements of patch column col, onto x
   auto further = [&](uint32_t id, int col, float (&x)[BS]) {
     const float* F = Fu + (size_t)id * a.fstride;
@@ -344,10 +352,13 @@ __global__ __launch_bounds__(512) void k_overlap(const OverlapArgs a) {
       for (int q = 0; q < BS; ++q) x[q] = fmaf(d * wr[q], vk, x[q]);
     }
   };
+  // rank 0 alone, as each form has always rounded it
   auto leading = [&](float d0, float w, float v) {
 #pragma clang fp contract(off)
     return BS <= 4 ? d0 * (w * v) : (d0 * w) * v;
   };
+  // stored rows of frame k (patches above 4 x 4)
+  const float* S = BS > 4 ? a.rows + ((size_t)slot * a.nw + k) * a.p_sel * M : nullptr;
   int2 rec[U];
   auto fetch = [&](int32_t j0) {
 #pragma unroll
@@ -372,7 +383,7 @@ __global__ __launch_bounds__(512) void k_overlap(const OverlapArgs a) {
       if (in[u]) {
         d0[u] = D[id[u]];
         v[u] = V[id[u]];
-        load_run<BS>(W + (size_t)id[u] * M, w[u]);
+        load_run<BS>(W + (size_t)id[u] * wst + cb * BS, w[u]);
       }
     }
     if (j0 + U * G < hi) fetch(j0 + U * G);
@@ -381,8 +392,13 @@ __global__ __launch_bounds__(512) void k_overlap(const OverlapArgs a) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const float dd = fabsf(d0[u]);
-      more[u] = d0[u] < 0.f;
+      const bool stored = BS > 4 && d0[u] < -2.f;
+      more[u] = d0[u] < 0.f && !stored;
       some = some || more[u];
+      if (stored) {
+        load_run<BS>(S + (size_t)id[u] * M + cb * BS, x[u]);
+        continue;
+      }
 #pragma unroll
       for (int q = 0; q < BS; ++q) x[u][q] = leading(dd, w[u][q], v[u]);
     }
@@ -471,9 +487,13 @@ __global__ __launch_bounds__(512) void k_overlap(const OverlapArgs a) {
         const float dd = D[id];
         if (dd == 0.f) continue;
         float x[BS], wr[BS];
-        load_run<BS>(a.w0 + ((size_t)b * a.p_sel + id) * M + col * BS, wr);
-        for (int z = 0; z < BS; ++z) x[z] = leading(fabsf(dd), wr[z], V[id]);
-        if (dd < 0.f) further(id, col, x);
+        if (BS > 4 && dd < -2.f) {
+          load_run<BS>(S + (size_t)id * M + col * BS, x);
+        } else {
+          load_run<BS>(W + (size_t)id * wst + col * BS, wr);
+          for (int z = 0; z < BS; ++z) x[z] = leading(fabsf(dd), wr[z], V[id]);
+          if (dd < 0.f) further(id, col, x);
+        }
         float xv = x[0];
 #pragma unroll
         for (int z = 1; z < BS; ++z) xv = q == z ? x[z] : xv;
@@ -547,17 +567,18 @@ hipError_t launch_lead(const float* factors, uint32_t nb, uint32_t nvar_stored, 
 }
 
 uint32_t overlap_blocks(const Shape& sh, int mode, uint32_t nk) {
-  const Strips st = strips_of(sh.nr);
+  const Strips st = strips_of(sh.nr, sh.bs);
   return st.nr * st.nc * (mode == 1 ? 1 : (nk == 0 || nk > sh.nw ? sh.nw : nk));
 }
 
 hipError_t launch_overlap(const OverlapSrc& src, const double* invw, const double* u64, const WinMeta* meta,
                           const uint32_t* wl, uint32_t na, const Shape& sh, int mode, double* out, double* partial,
                           hipStream_t s, uint32_t nk) {
-  const Strips st = strips_of(sh.nr);
+  const Strips st = strips_of(sh.nr, sh.bs);
   OverlapArgs a;
   a.factors = src.factors;
   a.dr = src.dr;
+  a.rows = src.rows;
   a.w0 = src.w0;
   a.v0 = src.v0;
   a.recs = src.recs;
@@ -590,7 +611,7 @@ hipError_t launch_overlap(const OverlapSrc& src, const double* invw, const doubl
       hipLaunchKernelGGL((k_overlap<B, false>), grid, dim3(st.threads), lds, s, a);                \
     return hipGetLastError();
   switch (sh.bs) {
-    PG_OV(2) PG_OV(3) PG_OV(4)
+    PG_OV(2) PG_OV(3) PG_OV(4) PG_OV(5) PG_OV(6) PG_OV(7) PG_OV(8) PG_OV(16)
     default: return hipErrorInvalidValue;
   }
 #undef PG_OV
