@@ -697,7 +697,7 @@ struct Pipeline {
   DBuf<char> divq;  // per (patch, variant) singular values and divergence factors (PGURE)
   // SVD input variants, factors and U reconstructions: FP32, or FP64 for
   // the precision study (sh.fp64); sized in bytes
-  DBuf<char> uvar, factors, B0, dr;  // B0: reconstructed rows (patches above 4 x 4); dr: the factors d_r
+  DBuf<char> uvar, factors, B0, dr;  // B0: reconstructed rows; dr: the factors d_r
   DBuf<int32_t> pos, cnt, off, list, inv;
   // the fused evaluation's static data per window (patches up to 4 x 4):
   // rows w_0 v_0[k] and singular pairs (s_0, s_1) per (frame, bucket place)
@@ -831,10 +831,10 @@ struct Pipeline {
     return m;
   }
 
-  // what an evaluation writes: the factors d_r of the kept ranks, and (FP64:
-  // instead) rows of patches above 4 x 4
+  // what an evaluation writes: the factors d_r of the kept ranks, and rows of
+  // the patches (FP64: one or the other)
   bool uses_dr() const { return strip_overlap(sh) || fused_eval(sh); }
-  bool uses_rows() const { return stored_rows(sh) || !uses_dr(); }
+  bool uses_rows() const { return strip_overlap(sh) || !uses_dr(); }
   size_t values_per_place() const { return (uses_dr() ? 1 : 0) + (uses_rows() ? sh.m : 0); }
 
   size_t bytes_per_window() const {
@@ -2308,7 +2308,7 @@ int run_noalloc(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf,
     }
     L.invw = c.take<double>(vol);
     L.dw = optimize ? c.take<float>(vol) : nullptr;
-    if (!fused_eval(sh)) L.B0 = c.take<float>((size_t)g.Nw * sh.p_sel * sh.m);
+    if (!fused_eval(sh) || !stated) L.B0 = c.take<float>((size_t)g.Nw * sh.p_sel * sh.m);
     if (fused_eval(sh) || !stated) L.dr = c.take<float>((size_t)g.Nw * sh.p_sel);
     if (fused_eval(sh) && stated) {
       c.take<char>(singular_pair_bytes(sh));

@@ -1044,15 +1044,12 @@ __global__ __launch_bounds__(256) void k_divq(const T* __restrict__ factors, con
 // 135-146 with src/utils.hpp:96-106), d_r = g(s_r)/s_r, w_r = X v_r = s_r u_r;
 // factors are sorted by descending s and g(s)/s grows with s, so the kept
 // ranks (d_r > 0) are a prefix.  FP32: the thread writes them to dr
-// [slot][r][p], followed by a 0 when fewer than n are kept; the overlap-add
-// forms the rows from them and the leading vectors and factors.  d_0 is
-// negative when rank 1 is kept too, and scaled by kStoredRow (a power of
-// two) when more than kInlineRanks are (patches above 4 x 4): k_rows then forms the patch's rows
-// of every frame once.  FP64: the gather forms d_0 and whether rank
-// 1 is kept itself, from the static singular pairs at every bucket place;
-// the thread writes the further kept ranks to dr [slot][p][r], r >= 1.
-// Either way the reconstruction itself is never written.  With PGURE (qdiv set) the thread also adds the
-// patch's divergence sum sum_r (d1_r q1_r - 2 d0_r q0_r + d2_r q2_r)
+// [slot][r][p], followed by a 0 when fewer than n are kept, d_0 negative when
+// rank 1 is kept too (k_rows then forms the patch's rows of every frame).
+// FP64: the gather forms d_0 and whether rank 1 is kept itself, from the
+// static singular pairs at every bucket place; the thread writes the further
+// kept ranks to dr [slot][p][r], r >= 1.  With PGURE (qdiv set) the thread
+// also adds the patch's divergence sum sum_r (d1_r q1_r - 2 d0_r q0_r + d2_r q2_r)
 // (src/pgure.hpp:136, see k_divq) to the FP64 partial of its block.  The
 // singular values and divergence factors come from the rank-major planes of
 // k_divq, or (qdiv null) the U variant's singular values from its factors.
@@ -1103,7 +1100,7 @@ __global__ __launch_bounds__(256) void k_round_prep(const T* __restrict__ factor
     }
     if (v == 0 && dr) {
       if (r > 1 && r < n) dr[dr_at(r)] = T(0);  // end of the kept ranks
-      if (PLANES) dr[dr_at(0)] = BS > 4 && r > kInlineRanks ? -first * T(kStoredRow) : r > 1 ? -first : first;
+      if (PLANES) dr[dr_at(0)] = r > 1 ? -first : first;
     }
     kr += r;
   }
@@ -1117,69 +1114,80 @@ __global__ __launch_bounds__(256) void k_round_prep(const T* __restrict__ factor
   if (kept) block_count(kept + (size_t)slot * gridDim.x + blockIdx.x, kr);
 }
 
-// Rows of the patches that keep more than kInlineRanks ranks (d_0 marked by
-// k_round_prep), all frames, by patch: rows [slot][frame][p][row], read by
-// the overlap-add.  Inline, a patch's row of every frame would read each
-// kept rank's w_r again; here a wave holds them for all frames.  A wave
-// looks at 16 patches and works off those marked, lane q on row q of B
-// (rows q, q + 64, ... above 8 x 8), the chain of the inline form.
+// Rows of the patches that keep more ranks than the first (d_0 negative), all
+// frames, by patch: rows [slot][frame][p][row], read by the overlap-add:
+// d_0 w_0[q] v_0[k], then fma(d_r w_r[q], v_r[k], .) in rank order.  A group
+// of L lanes (lane q: row q of B, and q + 64, ... above 8 x 8) reads the
+// patch's vectors once for every frame.  A wave looks at LOOK patches and
+// works off those marked, one per group at a time.
 // RT: window length n = nw at run time (n <= N).
 template <int BS, int N, bool RT = false>
 __global__ __launch_bounds__(256) void k_rows(const float* __restrict__ factors, const float* __restrict__ dr,
                                               const uint32_t* __restrict__ wl, uint32_t nvar_stored, uint32_t p_sel,
                                               uint32_t nw, uint32_t fstride, float* __restrict__ rows) {
-  constexpr int M = BS * BS, SRN = (N + 3) & ~3, RQ = (M + 63) / 64, NV = SRN / 4;
+  constexpr int M = BS * BS, L = M <= 16 ? 16 : 64, G = 64 / L, LOOK = 16 * G;
+  constexpr int SRN = (N + 3) & ~3, RQ = (M + L - 1) / L, NV = SRN / 4;
   const int n = RT ? (int)nw : N;
   const int SR = RT ? ((n + 3) & ~3) : SRN;
   const uint32_t slot = blockIdx.y, b = wl[slot];
-  const int lane = (int)(threadIdx.x % 64);
-  const uint32_t p0 = (blockIdx.x * 4 + threadIdx.x / 64) * 16;
+  const int wl_ = (int)(threadIdx.x % 64), lane = wl_ % L, grp = wl_ / L;
+  const uint32_t p0 = (blockIdx.x * 4 + threadIdx.x / 64) * LOOK;
   const float* D = dr + (size_t)slot * nw * p_sel;
-  const float first = (lane < 16 && p0 + lane < p_sel) ? D[p0 + lane] : 0.f;
-  uint64_t todo = __ballot(first < -2.f);
+  const float first = (wl_ < LOOK && p0 + wl_ < p_sel) ? D[p0 + wl_] : 0.f;
+  uint64_t todo = __ballot(first < 0.f);
   while (todo) {
-    const int l = __ffsll((unsigned long long)todo) - 1;
-    todo &= todo - 1;
+    // this group's patch: the grp-th one still marked (or none)
+    int l = -1;
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const int at = todo ? __ffsll((unsigned long long)todo) - 1 : -1;
+      todo &= todo - (todo ? 1 : 0);
+      if (g == grp) l = at;
+    }
+    if (l < 0) continue;  // (the last round's spare groups)
     const uint32_t p = p0 + (uint32_t)l;
     const float* F = factors + ((size_t)b * nvar_stored * p_sel + p) * fstride;  // the U variant
     const float* FW = F + n * SR;
-    float dl = lane < n ? D[(size_t)lane * p_sel + p] : 0.f;
-    if (lane == 0) dl = -dl * (1.f / kStoredRow);
-    // the kept ranks are a prefix, a 0 behind it
-    const int nkeep = __ffsll((unsigned long long)~__ballot(dl > 0.f)) - 1;
     float bq[RQ][N];
-#pragma unroll
-    for (int h = 0; h < RQ; ++h)
-#pragma unroll
-      for (int k = 0; k < N; ++k) bq[h][k] = 0.f;
     // rank loop, loads of rank r + 1 issued before the products of rank r
-    float wn[RQ];
+    float wn[RQ], dn;
     float4 vn[NV];
     auto fetch = [&](int r) {
+      dn = D[(size_t)r * p_sel + p];
 #pragma unroll
-      for (int h = 0; h < RQ; ++h) wn[h] = lane + 64 * h < M ? FW[r * M + lane + 64 * h] : 0.f;
+      for (int h = 0; h < RQ; ++h) wn[h] = lane + L * h < M ? FW[r * M + lane + L * h] : 0.f;
       const float4* vr = reinterpret_cast<const float4*>(F + r * SR);
 #pragma unroll
       for (int j = 0; j < NV; ++j) vn[j] = vr[j];
     };
     fetch(0);
-    for (int r = 0; r < nkeep; ++r) {
-      const float d = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, dl), r));
-      float y[RQ];
+    for (int r = 0; r < n; ++r) {
+      const float d = r == 0 ? -dn : dn;
+      if (!(d > 0.f)) break;  // the kept ranks are a prefix, a 0 behind it
+      float w[RQ], y[RQ];
 #pragma unroll
-      for (int h = 0; h < RQ; ++h) y[h] = d * wn[h];
+      for (int h = 0; h < RQ; ++h) {
+        w[h] = wn[h];
+        y[h] = d * wn[h];
+      }
       float4 vc[NV];
 #pragma unroll
       for (int j = 0; j < NV; ++j) vc[j] = vn[j];
-      if (r + 1 < nkeep) fetch(r + 1);
+      if (r + 1 < n) fetch(r + 1);
 #pragma unroll
       for (int h = 0; h < RQ; ++h) {
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
           const float t[4] = {vc[j].x, vc[j].y, vc[j].z, vc[j].w};
 #pragma unroll
-          for (int z = 0; z < 4; ++z)
-            if (4 * j + z < N) bq[h][4 * j + z] = fmaf(y[h], t[z], bq[h][4 * j + z]);
+          for (int z = 0; z < 4; ++z) {
+            if (4 * j + z >= N) continue;
+            float& o = bq[h][4 * j + z];
+            if (r > 0)
+              o = fmaf(y[h], t[z], o);
+            else
+              o = lead_product<(BS <= 4)>(d, w[h], t[z]);
+          }
         }
       }
     }
@@ -1189,7 +1197,7 @@ __global__ __launch_bounds__(256) void k_rows(const float* __restrict__ factors,
       const size_t at = (((size_t)slot * nw + k) * p_sel + p) * M;
 #pragma unroll
       for (int h = 0; h < RQ; ++h)
-        if (lane + 64 * h < M) rows[at + lane + 64 * h] = bq[h][k];
+        if (lane + L * h < M) rows[at + lane + L * h] = bq[h][k];
     }
   }
 }
@@ -1645,8 +1653,6 @@ bool fused_eval(const Shape& sh) { return sh.bs <= 4; }
 
 bool strip_overlap(const Shape& sh) { return !sh.fp64; }
 
-bool stored_rows(const Shape& sh) { return strip_overlap(sh) && sh.bs > 4; }
-
 uint32_t factor_stride(uint32_t nw, uint32_t m) {
   const uint32_t sr = (nw + 3) & ~3u;
   return ((nw * sr + nw * m + nw + 31) & ~31u) | 32u;
@@ -1661,25 +1667,22 @@ uint32_t eval_blocks(const Shape& sh, uint32_t nvar_run) {
 // the rows of the marked patches (see k_rows)
 static hipError_t launch_rows(const float* factors, const float* dr, const uint32_t* wl, uint32_t na,
                               uint32_t nvar_stored, const Shape& sh, float* rows, hipStream_t s) {
-  const dim3 grid((sh.p_sel + 63) / 64, na);
+  const uint32_t look = 4 * (sh.m <= 16 ? 64 : 16);  // patches a workgroup looks at
+  const dim3 grid((sh.p_sel + look - 1) / look, na);
 #define PG_RW(B, N, L, LS)                                                                                       \
-  if constexpr (B > 4) {                                                                                       \
-    if (sh.bs == B && sh.nw == N) {                                                                            \
-      hipLaunchKernelGGL((k_rows<B, N>), grid, dim3(256), 0, s, factors, dr, wl, nvar_stored, sh.p_sel, sh.nw,  \
-                         sh.fstride, rows);                                                                    \
-      return hipGetLastError();                                                                                \
-    }                                                                                                          \
+  if (sh.bs == B && sh.nw == N) {                                                                              \
+    hipLaunchKernelGGL((k_rows<B, N>), grid, dim3(256), 0, s, factors, dr, wl, nvar_stored, sh.p_sel, sh.nw,    \
+                       sh.fstride, rows);                                                                      \
+    return hipGetLastError();                                                                                  \
   }
   PG_SHAPES(PG_RW)
 #undef PG_RW
   const uint32_t nm = shape_generic(sh.bs, sh.nw);
 #define PG_RWG(B, NM, L, LE)                                                                                     \
-  if constexpr (B > 4) {                                                                                       \
-    if (sh.bs == B && nm == NM) {                                                                              \
-      hipLaunchKernelGGL((k_rows<B, NM, true>), grid, dim3(256), 0, s, factors, dr, wl, nvar_stored, sh.p_sel,  \
-                         sh.nw, sh.fstride, rows);                                                             \
-      return hipGetLastError();                                                                                \
-    }                                                                                                          \
+  if (sh.bs == B && nm == NM) {                                                                                \
+    hipLaunchKernelGGL((k_rows<B, NM, true>), grid, dim3(256), 0, s, factors, dr, wl, nvar_stored, sh.p_sel,    \
+                       sh.nw, sh.fstride, rows);                                                               \
+    return hipGetLastError();                                                                                  \
   }
   PG_GENERIC(PG_RWG)
 #undef PG_RWG
@@ -1695,7 +1698,7 @@ hipError_t launch_evaluation(const Shape& sh, const void* factors, const void* d
                        kept);
   const hipError_t e = launch_round_prep(factors, nvar_run == 3 ? divq : nullptr, meta, wl, na, nvar_stored, sh, exp_w,
                                          slot_lam, dr, nvar_run == 3 ? partial : nullptr, kept, s);
-  if (e != hipSuccess || !stored_rows(sh)) return e;
+  if (e != hipSuccess) return e;
   return launch_rows((const float*)factors, (const float*)dr, wl, na, nvar_stored, sh, (float*)rows, s);
 }
 

@@ -136,15 +136,11 @@ hipError_t launch_gather(const GatherSrc& src, const int32_t* off, const double*
 // launch_lead lays the U variant's v_0 (v0 [nb][nw][p_sel]) and, for patches
 // up to 4 x 4, w_0 (w0 [nb][p_sel][m]; null for larger ones) out by patch, and launch_overlap adds the rows up, with
 // d_r from launch_evaluation (dr [na][nw][p_sel], by rank, ended by a 0; d_0
-// negative where rank 1 is kept too) and, for patches above 4 x 4 that keep
-// more than kInlineRanks ranks (d_0 scaled by kStoredRow), their rows of
-// every frame (rows [na][nw][p_sel][m]).  wstat [nb][2]: the window's
-// largest s_0 (bits of a float) and largest W; zeroed by the caller before
-// launch_cover and launch_lead raise them.  Modes and nk as launch_gather.
-constexpr int kInlineRanks = 6;
-constexpr float kStoredRow = 18446744073709551616.f;  // 2^64
+// negative where rank 1 is kept too: then the patch's rows of every frame are
+// in rows [na][nw][p_sel][m]).  wstat [nb][2]: the window's largest s_0 (bits
+// of a float) and largest W; zeroed by the caller before launch_cover and
+// launch_lead raise them.  Modes and nk as launch_gather.
 bool strip_overlap(const Shape& sh);
-bool stored_rows(const Shape& sh);  // it may read rows (patches above 4 x 4)
 uint32_t column_bins(const Shape& sh);
 hipError_t launch_bins(const int32_t* pos, const uint32_t* sel, uint32_t nb, const Shape& sh, int32_t* off,
                        int2* recs, hipStream_t s);

@@ -54,4 +54,12 @@ __device__ __forceinline__ double group_sum(double v) {
   return v;
 }
 
+// d_0 w_0 v_0 as each form of the overlap-add has always rounded it: patches
+// up to 4 x 4 d_0 (w_0 v_0), larger ones (d_0 w_0) v_0; never contracted.
+template <bool SMALL>
+__device__ __forceinline__ float lead_product(float d0, float w0, float v0) {
+#pragma clang fp contract(off)
+  return SMALL ? d0 * (w0 * v0) : (d0 * w0) * v0;
+}
+
 }  // namespace pgsvt

@@ -8,6 +8,7 @@
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "lanes.hpp"
 
 namespace pgsvt {
 
@@ -17,22 +18,27 @@ namespace {
 // columns, accumulated in LDS.  Column-major frames make a strip of whole
 // columns one run of memory and the patches that reach it one run of the
 // column bins, so strips take every row; only frames above 2,048 rows are
-// cut.  4,096 cells are 32 KB: 4 workgroups of 256 threads share a CU's 160
-// KB.  Frames above 1,024 rows take up to 7,600 cells (within 64 KB) and 512
-// threads, or their halo (bs - 1 columns) would outweigh the strip.  Small
-// frames take fewer columns a strip, so that a call of a few windows still
-// has a workgroup for every CU; patches above 4 x 4, with a wider halo,
-// more.
+// cut.  From 192 rows, up to 6,144 cells (48 KB, 3 workgroups a CU) and 512
+// threads: wide strips repeat little halo (bs - 1 columns), 24 waves a CU
+// cover the loads (searches, ms a call for 8, 12, 16 and 24 columns: 256 rows
+// 35.5, 32.2, 29.6, 28.4, with 256 threads 30.1, 28.8, 30.9, 35.4; 512 rows
+// 12 columns 24.2, with 256 threads and 8 columns 30.8).  Smaller frames take
+// 256 threads and fewer columns a strip, so that a call of a few windows
+// still has a workgroup for every CU (128 rows: 16 columns 3.9, 12 4.1, 8
+// 4.4); patches above 4 x 4, with a wider halo, more.
 struct Strips {
   uint32_t tr, tc, ld, nr, nc, threads;  // ld: column stride in LDS; nr x nc strips a frame
 };
 Strips strips_of(uint32_t n, uint32_t bs) {
   Strips s;
   s.tr = std::min(n, 2048u);
-  const uint32_t cells = s.tr <= 1024 ? 4096 : 7600;
-  s.threads = s.tr <= 1024 ? 256 : 512;
-  s.tc = std::max(1u, bs <= 4 ? std::min({cells / s.tr, 16u, std::max(4u, n / 8)})
-                              : std::min({cells / s.tr, 32u, std::max(8u, n / 4)}));
+  if (n >= 192) {
+    s.threads = 512;
+    s.tc = (s.tr <= 1024 ? 6144 : 7600) / s.tr;
+  } else {
+    s.threads = 256;
+    s.tc = bs <= 4 ? std::min(16u, std::max(4u, n / 8)) : std::min({4096 / n, 32u, std::max(8u, n / 4)});
+  }
   // 8 lanes of a half-wave's row group and the 4 patch columns of a row
   // meet in distinct banks when the stride is 8 mod 32 cells
   s.ld = ((s.tr + 23) / 32) * 32 + 8;
@@ -262,14 +268,13 @@ __device__ __forceinline__ void load_run(const float* __restrict__ p, float (&x)
 }
 
 // Uhat = (sum of the patches' rows over each voxel) / W.  The row of patch p
-// in frame k is B[q][k] = d_0 (w_0[q] v_0[k]), then fma(d_r w_r[q], v_r[k],
-// .) over further kept ranks, FP32, in rank order; d_r by rank and patch
-// from k_round_prep, d_0 negative when rank 1 is kept too.  Patches above 4
-// x 4 take (d_0 w_0[q]) v_0[k], and where d_0 is marked the row that k_rows
-// stored.
+// in frame k is B[q][k] = d_0 w_0[q] v_0[k] (lead_product) where the patch
+// keeps rank 0 alone (d_0 > 0, by patch, from k_round_prep), and the row that
+// k_rows stored where it keeps more (d_0 < 0).
 //
 // A workgroup owns a strip of one frame and walks the records of the patches
-// that reach it, one lane per patch column of BS elements, adding each element to the strip's cells in LDS as a 64-bit integer: x is
+// that reach it, one lane per patch column of BS elements, adding each
+// element to the strip's cells in LDS as a 64-bit integer: x is
 // rounded to a multiple of a quantum q (x + 1.5 2^52 q leaves the multiple
 // in the low bits of the double) and the integers are added by ds_add_u64.
 // Integer sums are the same in every order, so the result is reproducible
@@ -280,11 +285,14 @@ __device__ __forceinline__ void load_run(const float* __restrict__ p, float (&x)
 // of it.  A column whose |x| reach 2^e (NaN, infinity) flags its cells,
 // which are then summed in FP64 from the records.
 //
-// Bound: instruction issue.  The form before (rows of a 32 x 8 tile staged
-// in LDS from bucket-sorted rows, each voxel reading its 16 positions and
-// looping over further patches of a position) issued 1,197 vector
-// instructions per 64 voxels, at 4 cycles each all of its 33 ps a voxel
-// (256 x 256 x 15 windows).
+// Bound: instruction issue and the LDS atomics, then memory (28 bytes a
+// voxel).  256 x 256 x 15 windows at searched lambdas: 15.2 ps a voxel.  The
+// form before (rows of a 32 x 8 tile staged in LDS from bucket-sorted rows,
+// each voxel reading its 16 positions and looping over further patches of a
+// position) issued 1,197 vector instructions per 64 voxels, at 4 cycles each
+// all of its 33 ps.  Further ranks formed here, as a row needs them, instead
+// of by k_rows: 128 x 128 x 30 over 64 lambdas 50.9 ms a call instead of 31.7
+// (every frame reads each kept rank's w_r again).
 //   mode 0: risk sums per block: sum Uhat^2, sum Uhat, sum Uhat U, sum U, sum U^2
 //   mode 1: final frame: Y(:,:,out) = uMax * Uhat(:,:,ref)
 //   mode 2: whole window volume of slot 0 into out
@@ -339,105 +347,62 @@ __global__ __launch_bounds__(512) void k_overlap(const OverlapArgs a) {
   // neighbour's in w0, larger ones fill their lines in the factors
   const float* W = BS <= 4 ? a.w0 + (size_t)b * a.p_sel * M : Fu + a.nw * sr;
   const size_t wst = BS <= 4 ? M : a.fstride;
-  // further kept ranks of patch id, elements of patch column col, onto x
-  auto further = [&](uint32_t id, int col, float (&x)[BS]) {
-    const float* F = Fu + (size_t)id * a.fstride;
-    for (uint32_t rk = 1; rk < a.nw; ++rk) {
-      const float d = D[(size_t)rk * a.p_sel + id];
-      if (!(d > 0.f)) break;
-      const float vk = F[rk * sr + k];
-      float wr[BS];
-      load_run<BS>(F + a.nw * sr + rk * M + col * BS, wr);
+  // stored rows of frame k
+  const float* S = a.rows + ((size_t)slot * a.nw + k) * a.p_sel * M;
+  // Three stages in flight: the records of the rows after the next ones, d_0
+  // and v_0 of the next ones (by their patch), the row or w_0 of this one
+  // (by its d_0), so that a round of rows waits for memory once.
+  auto fetch = [&](int32_t j0, int2 (&r)[U]) {
 #pragma unroll
-      for (int q = 0; q < BS; ++q) x[q] = fmaf(d * wr[q], vk, x[q]);
+    for (int u = 0; u < U; ++u) r[u] = R[min(j0 + u * G, hi - 1)];
+  };
+  // column and row of the record's first element in the strip; false: the
+  // lane's column lies outside it
+  auto place = [&](int32_t j, int2 r, int& col, int& row) {
+    col = ((r.x >> 16) & 0xffff) + cb - c0;
+    row = (r.x & 0xffff) - r0;
+    return j < hi && (LG == BS || cb < BS) && (uint32_t)col < cols && (!CUT || (row < (int)rows && row + BS > 0));
+  };
+  auto lead = [&](int32_t j0, const int2 (&r)[U], float (&d)[U], float (&v)[U]) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      int col, row;
+      d[u] = 0.f;
+      v[u] = 0.f;
+      if (place(j0 + u * G, r[u], col, row)) {
+        d[u] = D[(uint32_t)r[u].y];
+        v[u] = V[(uint32_t)r[u].y];
+      }
     }
   };
-  // rank 0 alone, as each form has always rounded it
-  auto leading = [&](float d0, float w, float v) {
-#pragma clang fp contract(off)
-    return BS <= 4 ? d0 * (w * v) : (d0 * w) * v;
-  };
-  // stored rows of frame k (patches above 4 x 4)
-  const float* S = BS > 4 ? a.rows + ((size_t)slot * a.nw + k) * a.p_sel * M : nullptr;
-  int2 rec[U];
-  auto fetch = [&](int32_t j0) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) rec[u] = R[min(j0 + u * G, hi - 1)];
-  };
+  int2 rec[U], rec1[U];
+  float d0[U], v[U];
   int32_t j0 = lo + grp;
-  if (j0 < hi) fetch(j0);
+  if (j0 < hi) {
+    fetch(j0, rec);
+    fetch(j0 + U * G, rec1);
+    lead(j0, rec, d0, v);
+  }
   for (; j0 < hi; j0 += U * G) {
-    float d0[U], v[U], w[U][BS];
+    float x[U][BS];
     uint32_t cell[U], id[U];
     int row[U];  // (used by cut strips only)
-    bool in[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int r = rec[u].x & 0xffff, c = ((rec[u].x >> 16) & 0xffff) + cb - c0;
+      int col;
+      (void)place(j0 + u * G, rec[u], col, row[u]);
+      cell[u] = (uint32_t)col * st.ld + (uint32_t)row[u];
       id[u] = (uint32_t)rec[u].y;
-      in[u] = j0 + u * G < hi && (LG == BS || cb < BS) && (uint32_t)c < cols;
-      row[u] = r - r0;
-      if (CUT) in[u] = in[u] && row[u] < (int)rows && row[u] + BS > 0;
-      cell[u] = (uint32_t)c * st.ld + (uint32_t)row[u];
-      d0[u] = 0.f;
-      if (in[u]) {
-        d0[u] = D[id[u]];
-        v[u] = V[id[u]];
-        load_run<BS>(W + (size_t)id[u] * wst + cb * BS, w[u]);
-      }
+      if (d0[u] != 0.f) load_run<BS>((d0[u] < 0.f ? S + (size_t)id[u] * M : W + (size_t)id[u] * wst) + cb * BS, x[u]);
     }
-    if (j0 + U * G < hi) fetch(j0 + U * G);
-    float x[U][BS];
-    bool more[U], some = false;
+    int2 rec2[U];
+    float d1[U], v1[U];
+    fetch(j0 + 2 * U * G, rec2);
+    lead(j0 + U * G, rec1, d1, v1);
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const float dd = fabsf(d0[u]);
-      const bool stored = BS > 4 && d0[u] < -2.f;
-      more[u] = d0[u] < 0.f && !stored;
-      some = some || more[u];
-      if (stored) {
-        load_run<BS>(S + (size_t)id[u] * M + cb * BS, x[u]);
-        continue;
-      }
+    for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int q = 0; q < BS; ++q) x[u][q] = leading(dd, w[u][q], v[u]);
-    }
-    if (some) {
-      // further kept ranks of the U rows together; d_r + 1 is read beside
-      // the vectors of rank r, so a rank waits for memory once
-      const float* F[U];
-      float d[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        F[u] = Fu + (size_t)id[u] * a.fstride;
-        d[u] = more[u] ? D[(size_t)a.p_sel + id[u]] : 0.f;
-      }
-      for (uint32_t rk = 1;;) {
-        float dn[U], vk[U], wr[U][BS];
-        some = false;
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          more[u] = d[u] > 0.f;
-          some = some || more[u];
-          dn[u] = 0.f;
-          if (more[u]) {
-            if (rk + 1 < a.nw) dn[u] = D[(size_t)(rk + 1) * a.p_sel + id[u]];
-            vk[u] = F[u][rk * sr + k];
-            load_run<BS>(F[u] + a.nw * sr + rk * M + cb * BS, wr[u]);
-          }
-        }
-        if (!some) break;
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          if (more[u]) {
-#pragma unroll
-            for (int q = 0; q < BS; ++q) x[u][q] = fmaf(d[u] * wr[u][q], vk[u], x[u][q]);
-          }
-          d[u] = dn[u];
-        }
-        ++rk;
-      }
-    }
+      for (int q = 0; q < BS; ++q) x[u][q] = d0[u] < 0.f ? x[u][q] : lead_product<(BS <= 4)>(d0[u], x[u][q], v[u]);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (d0[u] == 0.f) continue;  // nothing kept, or outside the strip
@@ -461,6 +426,13 @@ __global__ __launch_bounds__(512) void k_overlap(const OverlapArgs a) {
           __hip_atomic_fetch_add(&acc[cell[u] + q], __builtin_bit_cast(unsigned long long, h), __ATOMIC_RELAXED,
                                  __HIP_MEMORY_SCOPE_WORKGROUP);
       }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      rec[u] = rec1[u];
+      rec1[u] = rec2[u];
+      d0[u] = d1[u];
+      v[u] = v1[u];
     }
   }
   __syncthreads();
@@ -486,14 +458,10 @@ __global__ __launch_bounds__(512) void k_overlap(const OverlapArgs a) {
         const uint32_t id = (uint32_t)R[j].y;
         const float dd = D[id];
         if (dd == 0.f) continue;
-        float x[BS], wr[BS];
-        if (BS > 4 && dd < -2.f) {
-          load_run<BS>(S + (size_t)id * M + col * BS, x);
-        } else {
-          load_run<BS>(W + (size_t)id * wst + col * BS, wr);
-          for (int z = 0; z < BS; ++z) x[z] = leading(fabsf(dd), wr[z], V[id]);
-          if (dd < 0.f) further(id, col, x);
-        }
+        float x[BS];
+        load_run<BS>((dd < 0.f ? S + (size_t)id * M : W + (size_t)id * wst) + col * BS, x);
+        if (dd > 0.f)
+          for (int z = 0; z < BS; ++z) x[z] = lead_product<(BS <= 4)>(dd, x[z], V[id]);
         float xv = x[0];
 #pragma unroll
         for (int z = 1; z < BS; ++z) xv = q == z ? x[z] : xv;
