@@ -894,15 +894,6 @@ __device__ __forceinline__ int32_t row_bcast(int32_t v) {
   return __builtin_amdgcn_mov_dpp(v, 0x150 + K, 0xF, 0xF, true);
 }
 
-// f(std::integral_constant<int, K>) for K = K0 .. K1 - 1, in order
-template <int K0, int K1, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-  if constexpr (K0 < K1) {
-    f(std::integral_constant<int, K0>());
-    static_for<K0 + 1, K1>(f);
-  }
-}
-
 // Lane K of the group of L lanes (16: DPP row broadcast, 64: the wave's
 // lane K), in every lane of the group.
 template <int L, int K, class V>
