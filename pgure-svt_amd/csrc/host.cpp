@@ -685,8 +685,7 @@ struct Pipeline {
   DBuf<uint8_t> d2;
   DBuf<uint32_t> sel_d;
   // batch buffers
-  uint32_t NB = 0;  // windows of a batch
-  uint32_t NS = 0;  // evaluations of a round (alloc_batch)
+  uint32_t NB = 0;
   DBuf<WinMeta> meta_d;
   DBuf<uint32_t> wl_d;
   HBuf<WinMeta> meta_h;
@@ -864,24 +863,7 @@ struct Pipeline {
     return b;
   }
 
-  // The evaluations of one round of launches: a batch's windows, or, where the
-  // caller has more of them than windows (a grid of lambdas, the probe's
-  // three), as many as make kSlotPatches patches.  Smaller rounds are bound
-  // by their four launches (32 x 32 x 14 over 64 lambdas: 3.8 ms a call in rounds
-  // of the 14 windows, 1.8 in rounds of 311; at 128 x 128 x 30 the windows
-  // alone make 469 k).
-  static constexpr uint32_t kSlotPatches = 1u << 18;
-  uint32_t slots_wanted(uint32_t want, uint32_t evals) const {
-    if (!strip_overlap(sh)) return want;
-    return std::max(want, std::min(std::min(evals, 4096u), kSlotPatches / sh.p_sel));
-  }
-  size_t bytes_per_slot() const {
-    return 4ull * sh.nw * (size_t)sh.p_sel * values_per_place() +
-           8ull * (eval_blocks(sh, 3) + (size_t)frame_blocks(0) * 5) + 128;
-  }
-
-  // want: windows of a batch; evals: evaluations it has at once
-  void alloc_batch(uint32_t want, uint32_t evals = 0) {
+  void alloc_batch(uint32_t want) {
     int dev = 0;
     hipchk(hipGetDevice(&dev), "hipGetDevice");
     // Calls of this process size and allocate their batches one at a time
@@ -895,11 +877,6 @@ struct Pipeline {
     const size_t per = bytes_per_window();
     NB = (uint32_t)std::max<size_t>(1, std::min<size_t>(want, budget / per));
     if (const char* e = std::getenv("PGSVT_BATCH")) NB = std::max(1u, std::min<uint32_t>(NB, (uint32_t)atoi(e)));
-    NS = NB;
-    if (NB >= want && budget > NB * per) {
-      const size_t more = (budget - NB * per) / bytes_per_slot();
-      NS += (uint32_t)std::min<size_t>(slots_wanted(NB, evals) - NB, more);
-    }
     // Other processes can still take memory between the estimate and the
     // allocation: a batch that does not fit is halved (buffers of the failed
     // attempt go back to the cache, which a failing hipMalloc empties).
@@ -908,10 +885,9 @@ struct Pipeline {
         alloc_batch_buffers();
         return;
       } catch (const HipError& e) {
-        if (e.e != hipErrorOutOfMemory || (NB == 1 && NS == NB)) throw;
+        if (e.e != hipErrorOutOfMemory || NB == 1) throw;
         (void)hipGetLastError();
-        if (NS == NB) NB = std::max(1u, NB / 2);
-        NS = NB;
+        NB = std::max(1u, NB / 2);
       }
     }
   }
@@ -921,7 +897,7 @@ struct Pipeline {
     wl_d.alloc(NB);
     meta_h.alloc(NB);
     wl_h.alloc(NB);
-    sums_h.alloc((size_t)NS * 6);
+    sums_h.alloc((size_t)NB * 6);
     kept_h.alloc(NB);
     u64.alloc((size_t)NB * sh.vol);
     if (median) w64.alloc((size_t)NB * sh.vol);
@@ -943,8 +919,8 @@ struct Pipeline {
     }
     invw.alloc((size_t)NB * sh.vol);
     if (optimize) dw.alloc((size_t)NB * sh.vol * (sh.fp64 ? sizeof(double) : sizeof(float)));
-    if (uses_dr()) dr.alloc((size_t)NS * sh.nw * sh.p_sel * es);
-    if (uses_rows()) B0.alloc((size_t)NS * sh.nw * sh.p_sel * sh.m * es);
+    if (uses_dr()) dr.alloc((size_t)NB * sh.nw * sh.p_sel * es);
+    if (uses_rows()) B0.alloc((size_t)NB * sh.nw * sh.p_sel * sh.m * es);
     if (fused_eval(sh) && !strip_overlap(sh)) {
       w0b.alloc((size_t)NB * sh.nw * sh.p_sel * sh.m * es);
       s01b.alloc((size_t)NB * singular_pair_bytes(sh));
@@ -952,9 +928,9 @@ struct Pipeline {
     factors.alloc((size_t)NB * nvar * sh.p_sel * sh.fstride * es);
     if (optimize) divq.alloc((size_t)NB * nvar * sh.p_sel * 2 * ((sh.nw + 3) & ~3u) * es);
     risk_blocks = frame_blocks(0);
-    partial.alloc((size_t)NS * eval_blocks(sh, 3));
-    partial_b.alloc((size_t)NS * risk_blocks * 5);
-    sums.alloc((size_t)NS * 6);
+    partial.alloc((size_t)NB * eval_blocks(sh, 3));
+    partial_b.alloc((size_t)NB * risk_blocks * 5);
+    sums.alloc((size_t)NB * 6);
     partial_k.alloc((size_t)NB * eval_blocks(sh, 3));
     kept_d.alloc(NB);
     max_jobs = 2 * g.Nw;
@@ -962,9 +938,9 @@ struct Pipeline {
     if (probe_on) {
       factors_s.alloc((size_t)NB * 3 * sh_s.p_sel * sh.fstride * es);
       divq_s.alloc((size_t)NB * 3 * sh_s.p_sel * 2 * ((sh.nw + 3) & ~3u) * es);
-      partial_s.alloc((size_t)NS * eval_blocks(sh_s, 3));
-      lam_s.alloc(NS);
-      wl_s.alloc(NS);
+      partial_s.alloc((size_t)NB * eval_blocks(sh_s, 3));
+      lam_s.alloc(NB);
+      wl_s.alloc(NB);
     }
     stats.alloc(1);
     hipchk(launch_fill32(stats.p, stats.n, 0, s), "clear stats");
@@ -1129,9 +1105,9 @@ struct Pipeline {
     const double fk = (double)sh.nw / nk, fp = (double)sh.p_sel / sh_s.p_sel;
     hipchk(hipMemcpyAsync(meta_d.p, ms.data(), nb * sizeof(WinMeta), hipMemcpyHostToDevice, s), "H2D meta");
     risk.assign(nslot, 0.0);
-    std::vector<uint32_t> wl(NS);
-    for (uint32_t c0 = 0; c0 < nslot; c0 += NS) {
-      const uint32_t na = std::min(NS, nslot - c0);
+    std::vector<uint32_t> wl(NB);
+    for (uint32_t c0 = 0; c0 < nslot; c0 += NB) {
+      const uint32_t na = std::min(NB, nslot - c0);
       for (uint32_t i = 0; i < na; ++i) wl[i] = wins[(c0 + i) / 3];
       hipchk(hipMemcpyAsync(wl_s.p, wl.data(), na * 4, hipMemcpyHostToDevice, s), "H2D probe list");
       hipchk(hipMemcpyAsync(lam_s.p, lam.data() + c0, na * 8, hipMemcpyHostToDevice, s), "H2D probe lambdas");
@@ -1623,14 +1599,6 @@ std::vector<uint32_t> feature_sample(uint32_t p_sel, uint32_t nsamp) {
 
 constexpr uint32_t kFeatureSamples = 256;
 
-// Where all three parameters are given, no method but the first (which
-// refuses a window of too few leaves) takes anything from the leaves: none are
-// formed (99 x 99 x 23 of u8, windows of 9, 16 threads: 5.4 ms a call with
-// them, 3.6 without).
-bool leaves_needed(double alpha, double mu, double sigma, uint32_t method) {
-  return !(alpha >= 0.0 && mu >= 0.0 && sigma >= 0.0) || method == 1;
-}
-
 // Where the leaf statistics of the noise estimator are formed (the results
 // are the same bit for bit).  The host threads cost the GPU nothing while it
 // decomposes: about 60 ns a value and thread (distinct (frame,
@@ -1653,7 +1621,7 @@ bool leaves_on_gpu_pay(uint64_t values, uint32_t threads, double matrices, const
 // fixed lambda); 1: lambda proposed by the learned network; 2: only the
 // learned-lambda features of each window (no output frames); 3: PGURE risk
 // over a grid of lambdas per window, least risk chosen, the whole GPU work of
-// a batch up to its risk sums captured in one graph.
+// a batch captured in one graph.
 
 // Lanes-per-matrix mapping of the SVD per (patch, window) shape.  The two
 // mappings sum the column dot products in different orders, so their
@@ -1790,7 +1758,7 @@ int run_core(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf, co
   }
   {
     HostTimer t("host_alloc_batch");
-    P.alloc_batch(count, count * (rs.mode == 3 ? G : probe ? 3 : 1));
+    P.alloc_batch(count);
   }
 
   // Noise estimates on host threads.  Reference path: leaf statistics per
@@ -1816,7 +1784,6 @@ int run_core(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf, co
     }
   } leaf_joiner{leaf_thread};
   const double gmax = *std::max_element(P.fmaxX.begin(), P.fmaxX.end());
-  const bool want_leaves = leaves_needed(alpha0, mu0, sigma0, p.noise_method);
   if (P.optimize || learned) {
     // the distinct (frame, normalisation) pairs of the windows
     std::map<std::pair<uint32_t, uint64_t>, uint32_t> key_of;
@@ -1826,7 +1793,7 @@ int run_core(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf, co
       const double scale = learned ? gmax : m.uMax;
       uint64_t sbits;
       std::memcpy(&sbits, &scale, 8);
-      for (uint32_t k = 0; want_leaves && k < g.Nw; ++k) {
+      for (uint32_t k = 0; k < g.Nw; ++k) {
         const auto it = key_of.emplace(std::make_pair(m.s0 + k, sbits), (uint32_t)leaf_jobs.size());
         if (it.second) {
           leaf_jobs.emplace_back(new LeafJob{m.s0 + k, scale, {}, {}});
@@ -1836,7 +1803,7 @@ int run_core(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf, co
       }
     }
     const bool leaves_on_gpu =
-        want_leaves && nr >= 16 && (learned || leaves_on_gpu_pay((uint64_t)leaf_jobs.size() * P.sh.fs, thread_count(p.n_jobs),
+        nr >= 16 && (learned || leaves_on_gpu_pay((uint64_t)leaf_jobs.size() * P.sh.fs, thread_count(p.n_jobs),
                                                   (double)count * P.nvar * P.sh.p_sel, P.sh, rs.mode == 3));
     std::vector<std::function<void(PrepPool&)>> jobs;
     uint32_t made = 0;  // leaf jobs in the list (host)
@@ -1858,7 +1825,7 @@ int run_core(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf, co
         });
       }
       const double ratio = gmax / m.uMax;
-      jobs.push_back([t, need, ratio, learned, want_leaves, &leaf_jobs, &P, &p, &rs, g, nr, nc, lambda0, alpha0, mu0,
+      jobs.push_back([t, need, ratio, learned, &leaf_jobs, &P, &p, &rs, g, nr, nc, lambda0, alpha0, mu0,
                       sigma0](PrepPool& pool) {
         WindowPrep w;
         w.alpha = alpha0;
@@ -1876,7 +1843,7 @@ int run_core(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf, co
             }
             leaves.push_back(lv);
           }
-          if (want_leaves) estimate_from_leaves(leaves, nr, p.noise_method, w.alpha, w.mu, w.sigma);
+          estimate_from_leaves(leaves, nr, p.noise_method, w.alpha, w.mu, w.sigma);
           const double OoNxNyNt = 1.0 / (nc * nr * g.Nt);
           const double start = (lambda0 >= 0.0) ? lambda0 : P.host_window_accu(t) * OoNxNyNt;
           w.start = std::max(0.0, start);
@@ -1937,9 +1904,21 @@ int run_core(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf, co
     if (rs.mode == 3) {
       std::vector<WindowPrep> prep(nb);
       P.upload_batch(ms);
+      std::vector<double> nz((size_t)nb * 3);
+      {
+        HostTimer tw("host_noise_wait");
+        for (uint32_t b = 0; b < nb; ++b) {
+          prep[b] = pool->wait(t0 + b - rs.tb);
+          prep[b].check();
+          nz[3 * b] = prep[b].alpha;
+          nz[3 * b + 1] = prep[b].mu;
+          nz[3 * b + 2] = prep[b].sigma;
+        }
+      }
       std::vector<uint32_t> wlg((size_t)nb * G), wlf(nb);
       for (uint32_t q = 0; q < nb * G; ++q) wlg[q] = q / G;
       for (uint32_t b = 0; b < nb; ++b) wlf[b] = b;
+      hipchk(hipMemcpyAsync(noise_g.p, nz.data(), nz.size() * 8, hipMemcpyHostToDevice, P.s), "H2D noise");
       hipchk(hipMemcpyAsync(wl_g.p, wlg.data(), wlg.size() * 4, hipMemcpyHostToDevice, P.s), "H2D grid list");
       hipchk(hipMemcpyAsync(P.wl_d.p, wlf.data(), wlf.size() * 4, hipMemcpyHostToDevice, P.s), "H2D list");
       hipchk(hipStreamSynchronize(P.s), "grid upload sync");
@@ -1984,10 +1963,11 @@ int run_core(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf, co
         if (graph) (void)hipGraphDestroy(graph);
         gexec = nullptr;
         graph = nullptr;
-        // one graph: decomposition, lambda grid, risk sums of every candidate
-        // in chunks of NS slots
+        // one graph: decomposition, lambda grid, risk of every candidate in
+        // chunks of NB slots, argmin, final frames
         const uint32_t s_at = g.Nw * ((g.Nw + 3) & ~3u) + g.Nw * P.sh.m;
-        const uint32_t slots = nb * G, C = P.NS;
+        const uint32_t slots = nb * G, C = P.NB;
+        const double OoN = 1.0 / ((double)nr * nc * g.Nw);
         P.prof->suspended = true;
         hipchk(hipStreamBeginCapture(P.s, hipStreamCaptureModeThreadLocal), "begin capture");
         P.decompose_kernels(nb, P.nvar, svd_mapping);
@@ -2002,6 +1982,10 @@ int run_core(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf, co
                                     sums_g.p + (size_t)c0 * 6, P.s),
                  "grid reduce");
         }
+        hipchk(launch_grid_select(sums_g.p, noise_g.p, nb, G, OoN, P.eps2, lam_g.p, P.meta_d.p, risk_g.p, P.s),
+               "grid select");
+        P.evaluate(P.wl_d.p, nb, 1, nullptr, nullptr, nullptr);
+        P.overlap(P.wl_d.p, nb, 1, P.Yout, nullptr);
         const hipError_t ce = hipStreamEndCapture(P.s, &graph);
         P.prof->suspended = false;
         hipchk(ce, "end capture");
@@ -2009,29 +1993,6 @@ int run_core(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf, co
         graph_nb = nb;
       }
       P.prof->run("grid_graph", (double)nb * G, [&] { hipchk(hipGraphLaunch(gexec, P.s), "graph launch"); });
-      // (an estimate that fails leaves with the graph at its end)
-      struct Drain {
-        hipStream_t s;
-        ~Drain() { (void)hipStreamSynchronize(s); }
-      } drain{P.s};
-      // the noise estimates only now: the risk sums do not depend on them
-      std::vector<double> nz((size_t)nb * 3);
-      {
-        HostTimer tw("host_noise_wait");
-        for (uint32_t b = 0; b < nb; ++b) {
-          prep[b] = pool->wait(t0 + b - rs.tb);
-          prep[b].check();
-          nz[3 * b] = prep[b].alpha;
-          nz[3 * b + 1] = prep[b].mu;
-          nz[3 * b + 2] = prep[b].sigma;
-        }
-      }
-      hipchk(hipMemcpyAsync(noise_g.p, nz.data(), nz.size() * 8, hipMemcpyHostToDevice, P.s), "H2D noise");
-      const double OoN = 1.0 / ((double)nr * nc * g.Nw);
-      hipchk(launch_grid_select(sums_g.p, noise_g.p, nb, G, OoN, P.eps2, lam_g.p, P.meta_d.p, risk_g.p, P.s),
-             "grid select");
-      P.evaluate(P.wl_d.p, nb, 1, nullptr, nullptr, nullptr);
-      P.overlap(P.wl_d.p, nb, 1, P.Yout, nullptr);
       hipchk(hipMemcpyAsync(ms.data(), P.meta_d.p, nb * sizeof(WinMeta), hipMemcpyDeviceToHost, P.s), "D2H meta");
       hipchk(hipStreamSynchronize(P.s), "graph sync");
       P.prof->flush();
@@ -2446,8 +2407,7 @@ int run_noalloc(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf,
       hipchk(hipMemcpyAsync(hw.data(), L.Xw, vol * sizeof(double), hipMemcpyDeviceToHost, s), "D2H window");
       hipchk(hipStreamSynchronize(s), "window sync");
       for (double& v : hw) v /= m.uMax;
-      if (leaves_needed(alpha, mu, sigma, p.noise_method))
-        estimate_noise(hw.data(), nr, g.Nw, p.noise_method, alpha, mu, sigma);
+      estimate_noise(hw.data(), nr, g.Nw, p.noise_method, alpha, mu, sigma);
       double a1 = 0, a2 = 0;  // accu(u) in Armadillo's even / odd order
       size_t i = 0;
       for (; i + 1 < vol; i += 2) {
