@@ -685,7 +685,8 @@ struct Pipeline {
   DBuf<uint8_t> d2;
   DBuf<uint32_t> sel_d;
   // batch buffers
-  uint32_t NB = 0;
+  uint32_t NB = 0;  // windows of a batch
+  uint32_t NS = 0;  // evaluations of a round (alloc_batch)
   DBuf<WinMeta> meta_d;
   DBuf<uint32_t> wl_d;
   HBuf<WinMeta> meta_h;
@@ -863,7 +864,24 @@ struct Pipeline {
     return b;
   }
 
-  void alloc_batch(uint32_t want) {
+  // The evaluations of one round of launches: a batch's windows, or, where the
+  // caller has more of them than windows (a grid of lambdas, the probe's
+  // three), as many as make kSlotPatches patches.  Smaller rounds are bound
+  // by their four launches (32 x 32 x 14 over 64 lambdas: 3.8 ms a call in rounds
+  // of the 14 windows, 1.8 in rounds of 311; at 128 x 128 x 30 the windows
+  // alone make 469 k).
+  static constexpr uint32_t kSlotPatches = 1u << 18;
+  uint32_t slots_wanted(uint32_t want, uint32_t evals) const {
+    if (!strip_overlap(sh)) return want;
+    return std::max(want, std::min(std::min(evals, 4096u), kSlotPatches / sh.p_sel));
+  }
+  size_t bytes_per_slot() const {
+    return 4ull * sh.nw * (size_t)sh.p_sel * values_per_place() +
+           8ull * (eval_blocks(sh, 3) + (size_t)frame_blocks(0) * 5) + 128;
+  }
+
+  // want: windows of a batch; evals: evaluations it has at once
+  void alloc_batch(uint32_t want, uint32_t evals = 0) {
     int dev = 0;
     hipchk(hipGetDevice(&dev), "hipGetDevice");
     // Calls of this process size and allocate their batches one at a time
@@ -877,6 +895,11 @@ struct Pipeline {
     const size_t per = bytes_per_window();
     NB = (uint32_t)std::max<size_t>(1, std::min<size_t>(want, budget / per));
     if (const char* e = std::getenv("PGSVT_BATCH")) NB = std::max(1u, std::min<uint32_t>(NB, (uint32_t)atoi(e)));
+    NS = NB;
+    if (NB >= want && budget > NB * per) {
+      const size_t more = (budget - NB * per) / bytes_per_slot();
+      NS += (uint32_t)std::min<size_t>(slots_wanted(NB, evals) - NB, more);
+    }
     // Other processes can still take memory between the estimate and the
     // allocation: a batch that does not fit is halved (buffers of the failed
     // attempt go back to the cache, which a failing hipMalloc empties).
@@ -885,9 +908,10 @@ struct Pipeline {
         alloc_batch_buffers();
         return;
       } catch (const HipError& e) {
-        if (e.e != hipErrorOutOfMemory || NB == 1) throw;
+        if (e.e != hipErrorOutOfMemory || (NB == 1 && NS == NB)) throw;
         (void)hipGetLastError();
-        NB = std::max(1u, NB / 2);
+        if (NS == NB) NB = std::max(1u, NB / 2);
+        NS = NB;
       }
     }
   }
@@ -897,7 +921,7 @@ struct Pipeline {
     wl_d.alloc(NB);
     meta_h.alloc(NB);
     wl_h.alloc(NB);
-    sums_h.alloc((size_t)NB * 6);
+    sums_h.alloc((size_t)NS * 6);
     kept_h.alloc(NB);
     u64.alloc((size_t)NB * sh.vol);
     if (median) w64.alloc((size_t)NB * sh.vol);
@@ -919,8 +943,8 @@ struct Pipeline {
     }
     invw.alloc((size_t)NB * sh.vol);
     if (optimize) dw.alloc((size_t)NB * sh.vol * (sh.fp64 ? sizeof(double) : sizeof(float)));
-    if (uses_dr()) dr.alloc((size_t)NB * sh.nw * sh.p_sel * es);
-    if (uses_rows()) B0.alloc((size_t)NB * sh.nw * sh.p_sel * sh.m * es);
+    if (uses_dr()) dr.alloc((size_t)NS * sh.nw * sh.p_sel * es);
+    if (uses_rows()) B0.alloc((size_t)NS * sh.nw * sh.p_sel * sh.m * es);
     if (fused_eval(sh) && !strip_overlap(sh)) {
       w0b.alloc((size_t)NB * sh.nw * sh.p_sel * sh.m * es);
       s01b.alloc((size_t)NB * singular_pair_bytes(sh));
@@ -928,9 +952,9 @@ struct Pipeline {
     factors.alloc((size_t)NB * nvar * sh.p_sel * sh.fstride * es);
     if (optimize) divq.alloc((size_t)NB * nvar * sh.p_sel * 2 * ((sh.nw + 3) & ~3u) * es);
     risk_blocks = frame_blocks(0);
-    partial.alloc((size_t)NB * eval_blocks(sh, 3));
-    partial_b.alloc((size_t)NB * risk_blocks * 5);
-    sums.alloc((size_t)NB * 6);
+    partial.alloc((size_t)NS * eval_blocks(sh, 3));
+    partial_b.alloc((size_t)NS * risk_blocks * 5);
+    sums.alloc((size_t)NS * 6);
     partial_k.alloc((size_t)NB * eval_blocks(sh, 3));
     kept_d.alloc(NB);
     max_jobs = 2 * g.Nw;
@@ -938,9 +962,9 @@ struct Pipeline {
     if (probe_on) {
       factors_s.alloc((size_t)NB * 3 * sh_s.p_sel * sh.fstride * es);
       divq_s.alloc((size_t)NB * 3 * sh_s.p_sel * 2 * ((sh.nw + 3) & ~3u) * es);
-      partial_s.alloc((size_t)NB * eval_blocks(sh_s, 3));
-      lam_s.alloc(NB);
-      wl_s.alloc(NB);
+      partial_s.alloc((size_t)NS * eval_blocks(sh_s, 3));
+      lam_s.alloc(NS);
+      wl_s.alloc(NS);
     }
     stats.alloc(1);
     hipchk(launch_fill32(stats.p, stats.n, 0, s), "clear stats");
@@ -1105,9 +1129,9 @@ struct Pipeline {
     const double fk = (double)sh.nw / nk, fp = (double)sh.p_sel / sh_s.p_sel;
     hipchk(hipMemcpyAsync(meta_d.p, ms.data(), nb * sizeof(WinMeta), hipMemcpyHostToDevice, s), "H2D meta");
     risk.assign(nslot, 0.0);
-    std::vector<uint32_t> wl(NB);
-    for (uint32_t c0 = 0; c0 < nslot; c0 += NB) {
-      const uint32_t na = std::min(NB, nslot - c0);
+    std::vector<uint32_t> wl(NS);
+    for (uint32_t c0 = 0; c0 < nslot; c0 += NS) {
+      const uint32_t na = std::min(NS, nslot - c0);
       for (uint32_t i = 0; i < na; ++i) wl[i] = wins[(c0 + i) / 3];
       hipchk(hipMemcpyAsync(wl_s.p, wl.data(), na * 4, hipMemcpyHostToDevice, s), "H2D probe list");
       hipchk(hipMemcpyAsync(lam_s.p, lam.data() + c0, na * 8, hipMemcpyHostToDevice, s), "H2D probe lambdas");
@@ -1766,7 +1790,7 @@ int run_core(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf, co
   }
   {
     HostTimer t("host_alloc_batch");
-    P.alloc_batch(count);
+    P.alloc_batch(count, count * (rs.mode == 3 ? G : probe ? 3 : 1));
   }
 
   // Noise estimates on host threads.  Reference path: leaf statistics per
@@ -1973,9 +1997,9 @@ int run_core(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf, co
         gexec = nullptr;
         graph = nullptr;
         // one graph: decomposition, lambda grid, risk of every candidate in
-        // chunks of NB slots, argmin, final frames
+        // chunks of NS slots, argmin, final frames
         const uint32_t s_at = g.Nw * ((g.Nw + 3) & ~3u) + g.Nw * P.sh.m;
-        const uint32_t slots = nb * G, C = P.NB;
+        const uint32_t slots = nb * G, C = P.NS;
         const double OoN = 1.0 / ((double)nr * nc * g.Nw);
         P.prof->suspended = true;
         hipchk(hipStreamBeginCapture(P.s, hipStreamCaptureModeThreadLocal), "begin capture");
