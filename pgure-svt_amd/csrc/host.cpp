@@ -1653,7 +1653,7 @@ bool leaves_on_gpu_pay(uint64_t values, uint32_t threads, double matrices, const
 // fixed lambda); 1: lambda proposed by the learned network; 2: only the
 // learned-lambda features of each window (no output frames); 3: PGURE risk
 // over a grid of lambdas per window, least risk chosen, the whole GPU work of
-// a batch captured in one graph.
+// a batch up to its risk sums captured in one graph.
 
 // Lanes-per-matrix mapping of the SVD per (patch, window) shape.  The two
 // mappings sum the column dot products in different orders, so their
@@ -1937,21 +1937,9 @@ int run_core(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf, co
     if (rs.mode == 3) {
       std::vector<WindowPrep> prep(nb);
       P.upload_batch(ms);
-      std::vector<double> nz((size_t)nb * 3);
-      {
-        HostTimer tw("host_noise_wait");
-        for (uint32_t b = 0; b < nb; ++b) {
-          prep[b] = pool->wait(t0 + b - rs.tb);
-          prep[b].check();
-          nz[3 * b] = prep[b].alpha;
-          nz[3 * b + 1] = prep[b].mu;
-          nz[3 * b + 2] = prep[b].sigma;
-        }
-      }
       std::vector<uint32_t> wlg((size_t)nb * G), wlf(nb);
       for (uint32_t q = 0; q < nb * G; ++q) wlg[q] = q / G;
       for (uint32_t b = 0; b < nb; ++b) wlf[b] = b;
-      hipchk(hipMemcpyAsync(noise_g.p, nz.data(), nz.size() * 8, hipMemcpyHostToDevice, P.s), "H2D noise");
       hipchk(hipMemcpyAsync(wl_g.p, wlg.data(), wlg.size() * 4, hipMemcpyHostToDevice, P.s), "H2D grid list");
       hipchk(hipMemcpyAsync(P.wl_d.p, wlf.data(), wlf.size() * 4, hipMemcpyHostToDevice, P.s), "H2D list");
       hipchk(hipStreamSynchronize(P.s), "grid upload sync");
@@ -1996,11 +1984,10 @@ int run_core(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf, co
         if (graph) (void)hipGraphDestroy(graph);
         gexec = nullptr;
         graph = nullptr;
-        // one graph: decomposition, lambda grid, risk of every candidate in
-        // chunks of NS slots, argmin, final frames
+        // one graph: decomposition, lambda grid, risk sums of every candidate
+        // in chunks of NS slots
         const uint32_t s_at = g.Nw * ((g.Nw + 3) & ~3u) + g.Nw * P.sh.m;
         const uint32_t slots = nb * G, C = P.NS;
-        const double OoN = 1.0 / ((double)nr * nc * g.Nw);
         P.prof->suspended = true;
         hipchk(hipStreamBeginCapture(P.s, hipStreamCaptureModeThreadLocal), "begin capture");
         P.decompose_kernels(nb, P.nvar, svd_mapping);
@@ -2015,10 +2002,6 @@ int run_core(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf, co
                                     sums_g.p + (size_t)c0 * 6, P.s),
                  "grid reduce");
         }
-        hipchk(launch_grid_select(sums_g.p, noise_g.p, nb, G, OoN, P.eps2, lam_g.p, P.meta_d.p, risk_g.p, P.s),
-               "grid select");
-        P.evaluate(P.wl_d.p, nb, 1, nullptr, nullptr, nullptr);
-        P.overlap(P.wl_d.p, nb, 1, P.Yout, nullptr);
         const hipError_t ce = hipStreamEndCapture(P.s, &graph);
         P.prof->suspended = false;
         hipchk(ce, "end capture");
@@ -2026,6 +2009,29 @@ int run_core(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf, co
         graph_nb = nb;
       }
       P.prof->run("grid_graph", (double)nb * G, [&] { hipchk(hipGraphLaunch(gexec, P.s), "graph launch"); });
+      // (an estimate that fails leaves with the graph at its end)
+      struct Drain {
+        hipStream_t s;
+        ~Drain() { (void)hipStreamSynchronize(s); }
+      } drain{P.s};
+      // the noise estimates only now: the risk sums do not depend on them
+      std::vector<double> nz((size_t)nb * 3);
+      {
+        HostTimer tw("host_noise_wait");
+        for (uint32_t b = 0; b < nb; ++b) {
+          prep[b] = pool->wait(t0 + b - rs.tb);
+          prep[b].check();
+          nz[3 * b] = prep[b].alpha;
+          nz[3 * b + 1] = prep[b].mu;
+          nz[3 * b + 2] = prep[b].sigma;
+        }
+      }
+      hipchk(hipMemcpyAsync(noise_g.p, nz.data(), nz.size() * 8, hipMemcpyHostToDevice, P.s), "H2D noise");
+      const double OoN = 1.0 / ((double)nr * nc * g.Nw);
+      hipchk(launch_grid_select(sums_g.p, noise_g.p, nb, G, OoN, P.eps2, lam_g.p, P.meta_d.p, risk_g.p, P.s),
+             "grid select");
+      P.evaluate(P.wl_d.p, nb, 1, nullptr, nullptr, nullptr);
+      P.overlap(P.wl_d.p, nb, 1, P.Yout, nullptr);
       hipchk(hipMemcpyAsync(ms.data(), P.meta_d.p, nb * sizeof(WinMeta), hipMemcpyDeviceToHost, P.s), "D2H meta");
       hipchk(hipStreamSynchronize(P.s), "graph sync");
       P.prof->flush();
