@@ -1637,16 +1637,16 @@ bool leaves_needed(double alpha, double mu, double sigma, uint32_t method) {
 // normalisation) pairs x pixels) against the decomposition's 0.85 ns a
 // matrix and its 14 m n^2 + 8 n^3 flops at 25 TFLOP/s (256 x 256 x 100: the
 // call takes 116 ms with the host's, 119 with the GPU's, whose leaves share
-// the SIMDs with the SVD).  Where they would end after it, or nothing runs
-// beside them (the lambda grid's graph waits for every estimate), the GPU
+// the SIMDs with the SVD).  Where they would end after it, the GPU
 // forms them (512 x 512 x 40, windows of 7: 101 ms with the host's, 91 with
-// the GPU's; 128 x 128 x 30 over a grid: 53.8 against 50.5).  Below 2^18
-// values the host is done first (64 x 64 x 20: 3.7 against 4.4 ms).
-bool leaves_on_gpu_pay(uint64_t values, uint32_t threads, double matrices, const Shape& sh, bool waits) {
+// the GPU's; 128 x 128 x 30 over a grid, whose rounds run on: 24.3 with the
+// host's, 24.7 with the GPU's).  Below 2^18 values the host is done first
+// (64 x 64 x 20: 3.7 against 4.4 ms).
+bool leaves_on_gpu_pay(uint64_t values, uint32_t threads, double matrices, const Shape& sh) {
   if (values < ((uint64_t)1 << 18)) return false;
   const double host = 60e-9 * (double)values / threads;
   const double flops = 14.0 * sh.m * sh.nw * sh.nw + 8.0 * sh.nw * sh.nw * sh.nw;
-  return waits || host > matrices * (0.85e-9 + flops / 25e12);
+  return host > matrices * (0.85e-9 + flops / 25e12);
 }
 
 // What one call computes.  mode 0: the reference driver (PGURE search or the
@@ -1837,7 +1837,7 @@ int run_core(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf, co
     }
     const bool leaves_on_gpu =
         want_leaves && nr >= 16 && (learned || leaves_on_gpu_pay((uint64_t)leaf_jobs.size() * P.sh.fs, thread_count(p.n_jobs),
-                                                  (double)count * P.nvar * P.sh.p_sel, P.sh, rs.mode == 3));
+                                                  (double)count * P.nvar * P.sh.p_sel, P.sh));
     std::vector<std::function<void(PrepPool&)>> jobs;
     uint32_t made = 0;  // leaf jobs in the list (host)
     for (uint32_t t = rs.tb; t < rs.te; ++t) {

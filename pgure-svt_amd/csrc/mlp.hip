@@ -18,12 +18,10 @@ namespace {
 typedef short v4s __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-// float -> bfloat16 bits, round to nearest even (NaN kept a NaN)
-__device__ __forceinline__ short to_bf16(float x) {
-  uint32_t u = __float_as_uint(x);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (short)((u >> 16) | 0x40);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (short)(u >> 16);
+// float -> bfloat16, round to nearest even (v_cvt_pk_bf16_f32)
+__device__ __forceinline__ v4s to_bf16(const float (&x)[4]) {
+  typedef __bf16 v4b __attribute__((ext_vector_type(4)));
+  return __builtin_bit_cast(v4s, __builtin_convertvector((v4f{x[0], x[1], x[2], x[3]}), v4b));
 }
 
 __device__ __forceinline__ float gelu(float x) { return 0.5f * x * (1.f + erff(x * 0.70710678118654752f)); }
@@ -32,30 +30,98 @@ __device__ __forceinline__ float gelu_grad(float x) {
   return 0.5f * (1.f + erff(x * 0.70710678118654752f)) + x * 0.39894228040143268f * expf(-0.5f * x * x);
 }
 
+// K per buffered piece of the product: 8 matrix instructions, 64 values a lane
+constexpr int kPiece = 128, kInstr = kPiece / 16;
+
+// 16 x 16 tile of a strided operand: the four values k = kq .. kq + 3 of a
+// lane's row for each instruction of the piece at k0.  K1: contiguous in k,
+// one load of four (rows start at any float: the type states 4-byte alignment).
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+template <bool K1>
+__device__ __forceinline__ void load_piece(const float* __restrict__ p, int64_t sk, int k0, int kq, int K,
+                                           float (&x)[kInstr][4]) {
+  if (k0 + kPiece <= K) {
+    const float* q = p + (int64_t)(k0 + kq) * (K1 ? 1 : sk);
+#pragma unroll
+    for (int u = 0; u < kInstr; ++u) {
+      if constexpr (K1) {
+        const f4u t = *(const f4u*)(q + 16 * u);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) x[u][v] = t[v];
+      } else {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) x[u][v] = q[(int64_t)(16 * u + v) * sk];
+      }
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < kInstr; ++u)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int k = k0 + 16 * u + kq + v;
+        const float t = p[(int64_t)min(k, K - 1) * (K1 ? 1 : sk)];
+        x[u][v] = k < K ? t : 0.f;
+      }
+  }
+}
+
 // C(m, n) = act(sum_k A(m, k) B(k, n) + bias[n]) with A(m, k) = A[m*sam +
 // k*sak], B(k, n) = B[k*sbk + n*sbn]; operands rounded to bf16, products
-// summed in FP32 by v_mfma_f32_16x16x16_bf16.  One wave per 16 x 16 tile
-// of C.  Lane l holds A rows l%16, k = 4(l/16)..+3 and B columns l%16,
-// same k; it receives C rows 4(l/16)..+3 of column l%16.
-__global__ __launch_bounds__(256) void k_gemm(const float* __restrict__ A, int64_t sam, int64_t sak,
-                                              const float* __restrict__ B, int64_t sbk, int64_t sbn,
-                                              float* __restrict__ C, int64_t ldc, int M, int N, int K,
-                                              const float* __restrict__ bias, int act, float* __restrict__ pre) {
-  const int wave = (int)((blockIdx.x * blockDim.x + threadIdx.x) / 64), lane = (int)(threadIdx.x % 64);
+// summed in FP32 by v_mfma_f32_16x16x16_bf16, k ascending in one chain.  One
+// wave (and workgroup) per 16 x 16 tile of C.  Lane l holds A rows l%16, k =
+// 4(l/16)..+3 and B columns l%16, same k; it receives C rows 4(l/16)..+3 of
+// column l%16.
+//
+// Few tiles and a long chain (256 x 3843 x 128: 128 waves of 241
+// instructions): bound by the latency of a wave's loads, not by bytes or
+// matrix operations.  The next 128 k are on their way while the current ones
+// multiply, and each wave has a compute unit to itself: 28 us (and 76 us for
+// the 11 products of a training step of 256 rows; one load after the other,
+// operands rounded in integer arithmetic, four waves to a workgroup: 713 us).
+// Rows and columns past the edge read the last one: they reach only results
+// that are not stored.
+template <bool A1, bool B1>
+__global__ __launch_bounds__(64) void k_gemm(const float* __restrict__ A, int64_t sam, int64_t sak,
+                                             const float* __restrict__ B, int64_t sbk, int64_t sbn,
+                                             float* __restrict__ C, int64_t ldc, int M, int N, int K,
+                                             const float* __restrict__ bias, int act, float* __restrict__ pre) {
+  const int lane = (int)threadIdx.x;
   const int tiles_n = (N + 15) / 16;
-  const int tm = wave / tiles_n, tn = wave % tiles_n;
-  if (tm * 16 >= M) return;  // uniform per wave: the matrix op runs with every lane
-  const int i = tm * 16 + lane % 16, j = tn * 16 + lane % 16, kq = 4 * (lane / 16);
+  const int tm = (int)blockIdx.x / tiles_n, tn = (int)blockIdx.x % tiles_n;
+  const int kq = 4 * (lane / 16);
+  const float* pa = A + (int64_t)min(tm * 16 + lane % 16, M - 1) * sam;
+  const float* pb = B + (int64_t)min(tn * 16 + lane % 16, N - 1) * sbn;
   v4f acc = {0.f, 0.f, 0.f, 0.f};
-  for (int k0 = 0; k0 < K; k0 += 16) {
-    v4s a, b;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int k = k0 + kq + v;
-      a[v] = to_bf16((i < M && k < K) ? A[i * sam + k * sak] : 0.f);
-      b[v] = to_bf16((j < N && k < K) ? B[k * sbk + j * sbn] : 0.f);
+  float xa[kInstr][4], xb[kInstr][4];
+  load_piece<A1>(pa, sak, 0, kq, K, xa);
+  load_piece<B1>(pb, sbk, 0, kq, K, xb);
+  for (int k0 = 0; k0 < K; k0 += kPiece) {
+    float ya[kInstr][4], yb[kInstr][4];
+    const bool more = k0 + kPiece < K;  // (uniform)
+    if (more) {
+      load_piece<A1>(pa, sak, k0 + kPiece, kq, K, ya);
+      load_piece<B1>(pb, sbk, k0 + kPiece, kq, K, yb);
     }
-    acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
+    auto step = [&](int u) __attribute__((always_inline)) {
+      acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(to_bf16(xa[u]), to_bf16(xb[u]), acc, 0, 0, 0);
+    };
+    if (k0 + kPiece <= K) {
+#pragma unroll
+      for (int u = 0; u < kInstr; ++u) step(u);
+    } else {
+#pragma unroll
+      for (int u = 0; u < kInstr; ++u)
+        if (k0 + 16 * u < K) step(u);  // (uniform)
+    }
+    if (more) {
+#pragma unroll
+      for (int u = 0; u < kInstr; ++u)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          xa[u][v] = ya[u][v];
+          xb[u][v] = yb[u][v];
+        }
+    }
   }
 #pragma unroll
   for (int v = 0; v < 4; ++v) {
@@ -74,13 +140,32 @@ __global__ void k_gelu_bwd(const float* __restrict__ pre, const float* __restric
   if (i < n) dx[i] = dy[i] * gelu_grad(pre[i]);
 }
 
-// out[n] = sum over rows b of D[b*ld + n] (one thread per column, rows in order)
-__global__ void k_colsum(const float* __restrict__ D, int rows, int cols, int64_t ld, float* __restrict__ out) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= cols) return;
+// out[n] = sum over rows b of D[b*ld + n], rows in order: 16 columns a
+// workgroup, 256 rows at a time through LDS, so that the order costs LDS reads
+// and not a memory latency a row (256 x 128: 46 -> 3.4 us)
+__global__ __launch_bounds__(256) void k_colsum(const float* __restrict__ D, int rows, int cols, int64_t ld,
+                                                float* __restrict__ out) {
+  __shared__ float part[256][17];
+  const int t = (int)threadIdx.x, c = (int)blockIdx.x * 16 + t % 16;
   float s = 0.f;
-  for (int b = 0; b < rows; ++b) s += D[b * ld + c];
-  out[c] = s;
+  for (int b0 = 0; b0 < rows; b0 += 256) {
+    float x[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      const int b = b0 + 16 * u + t / 16;
+      x[u] = D[(int64_t)min(b, rows - 1) * ld + min(c, cols - 1)];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 16; ++u) part[16 * u + t / 16][t % 16] = x[u];
+    __syncthreads();
+    const int nb = min(256, rows - b0);
+    if (t < 16) {
+#pragma unroll 16
+      for (int b = 0; b < nb; ++b) s += part[b][t];
+    }
+  }
+  if (t < 16 && c < cols) out[c] = s;
 }
 
 // mean squared error of y[b*ldy] against t[b]: dy = 2 (y - t) / n, loss
@@ -152,10 +237,11 @@ hipError_t launch_gather_rows(const float* X, const uint32_t* idx, uint32_t rows
 
 hipError_t launch_gemm(const float* A, int64_t sam, int64_t sak, const float* B, int64_t sbk, int64_t sbn, float* C,
                        int64_t ldc, int M, int N, int K, const float* bias, int act, float* pre, hipStream_t s) {
-  const int64_t waves = (int64_t)((M + 15) / 16) * ((N + 15) / 16);
-  const int64_t blocks = (waves + 3) / 4;
-  hipLaunchKernelGGL(k_gemm, dim3((uint32_t)blocks), dim3(256), 0, s, A, sam, sak, B, sbk, sbn, C, ldc, M, N, K,
-                     bias, act, pre);
+  if (M <= 0 || N <= 0 || K <= 0) return hipErrorInvalidValue;
+  const dim3 grid((uint32_t)((int64_t)((M + 15) / 16) * ((N + 15) / 16)));
+  auto* k = sak == 1 ? (sbk == 1 ? k_gemm<true, true> : k_gemm<true, false>)
+                     : (sbk == 1 ? k_gemm<false, true> : k_gemm<false, false>);
+  hipLaunchKernelGGL(k, grid, dim3(64), 0, s, A, sam, sak, B, sbk, sbn, C, ldc, M, N, K, bias, act, pre);
   return hipGetLastError();
 }
 
@@ -165,7 +251,7 @@ hipError_t launch_gelu_bwd(const float* pre, const float* dy, float* dx, int64_t
 }
 
 hipError_t launch_colsum(const float* D, int rows, int cols, int64_t ld, float* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_colsum, dim3((cols + 255) / 256), dim3(256), 0, s, D, rows, cols, ld, out);
+  hipLaunchKernelGGL(k_colsum, dim3((cols + 15) / 16), dim3(256), 0, s, D, rows, cols, ld, out);
   return hipGetLastError();
 }
 
