@@ -233,14 +233,26 @@ hipError_t launch_fill_ref(const WinMeta* meta, uint32_t nb, const Shape& sh, in
 // reference does; ties go to the first index.  The visited map (checkMat)
 // lives in LDS, one bit per candidate offset, laid out word-major so that
 // consecutive threads hit consecutive banks.
-// Search windows up to kArpsMaxMw (2 * 15 + 1 offsets a side) run 128
-// threads per block; wider ones, up to kArpsMaxMwWide, 64 threads with a
-// larger visited map each.
+//
+// Search windows up to kArpsMaxMw search in a tile of the destination frame in
+// LDS: a workgroup takes tr x tc neighbouring blocks, and every candidate that
+// the search can reach lies within the window (or 2 at column 0) around its
+// own.  A candidate is read by its neighbours too, so each pixel comes from
+// memory a few times instead of some hundred, and a candidate costs one
+// address (256 x 256 x 100, windows of 7: 7.2 -> 5.5 ms; the vector cache
+// was busy for 5.1 ms of it and the vector units for 4.0).  Wider windows, up to kArpsMaxMwWide, read the frame: a
+// tile and their visited maps would leave a wave or two per compute unit.
 constexpr int kArpsMaxMw = 15, kArpsMaxMwWide = 31;
-template <int MW>
-struct ArpsCfg {
-  static constexpr int kWords = ((2 * MW + 1) * (2 * MW + 1) + 31) / 32;
-  static constexpr int kThreads = MW <= 15 ? 128 : 64;
+constexpr int kArpsWideThreads = 64;
+constexpr int arps_words(int mw) { return ((2 * mw + 1) * (2 * mw + 1) + 31) / 32; }
+// waves per SIMD the registers (the block's 2 BS^2 and those of a candidate)
+// are held to
+constexpr int arps_waves(int bs) { return bs <= 4 ? 4 : bs <= 6 ? 3 : 2; }
+template <int BS, int MW>
+struct ArpsTile {
+  static constexpr int kThreads = BS > 8 ? 128 : 256;
+  static constexpr int kRows = 64;                          // block rows at most
+  static constexpr int kStride = kRows + BS - 1 + 2 * MW;  // pixels a column
 };
 
 // The reference block: held in registers up to 8 x 8, read from the source
@@ -265,27 +277,88 @@ struct ArpsRef<BS, false> {
   __device__ double operator[](int q) const { return S[(q % BS) + (size_t)nr * (q / BS)]; }
 };
 
-template <int BS>
-__device__ __forceinline__ double arps_cost(const ArpsRef<BS>& ref, const double* __restrict__ F, uint32_t nr,
-                                            int r0, int c0, double inv) {
+// the candidate at base, columns `stride` apart
+template <int BS, class S>
+__device__ __forceinline__ double arps_cost(const ArpsRef<BS>& ref, const double* base, S stride, double inv) {
 #pragma clang fp contract(off)
   double a1 = 0.0, a2 = 0.0;
+  if constexpr (BS > 8) {  // a column at a time (BS is even: rows alternate)
+    static_assert(BS % 2 == 0, "the sums would change places at every column");
+#pragma unroll 1
+    for (int c = 0; c < BS; ++c) {
+      const double *u = ref.S + (size_t)ref.nr * c, *v = base + stride * c;
+#pragma unroll
+      for (int r = 0; r < BS; r += 2) {
+        const double d1 = u[r] - v[r];
+        a1 += d1 * d1;
+        const double d2 = u[r + 1] - v[r + 1];
+        a2 += d2 * d2;
+      }
+    }
+    return (a1 + a2) * inv;
+  }
   constexpr int n = BS * BS;
-  const double* base = F + r0 + (size_t)nr * c0;
   int q = 0;
 #pragma unroll
   for (; q + 1 < n; q += 2) {
-    const double d1 = ref[q] - base[(q % BS) + (size_t)nr * (q / BS)];
+    const double d1 = ref[q] - base[(q % BS) + stride * (q / BS)];
     a1 += d1 * d1;
-    const double d2 = ref[q + 1] - base[((q + 1) % BS) + (size_t)nr * ((q + 1) / BS)];
+    const double d2 = ref[q + 1] - base[((q + 1) % BS) + stride * ((q + 1) / BS)];
     a2 += d2 * d2;
   }
   if (q < n) {
-    const double d1 = ref[q] - base[(q % BS) + (size_t)nr * (q / BS)];
+    const double d1 = ref[q] - base[(q % BS) + stride * (q / BS)];
     a1 += d1 * d1;
   }
   return (a1 + a2) * inv;
 }
+
+// the same of two blocks in memory, for the rare case
+template <int BS>
+__device__ __forceinline__ double arps_cost_far(const double* B, const double* C, uint32_t nr, double inv) {
+#pragma clang fp contract(off)
+  double a1 = 0.0, a2 = 0.0;
+#pragma unroll 1
+  for (int q = 0; q < BS * BS; ++q) {
+    const size_t at = (q % BS) + (size_t)nr * (q / BS);
+    const double d = B[at] - C[at], dd = d * d;
+    a1 = q % 2 == 0 ? a1 + dd : a1;
+    a2 = q % 2 == 1 ? a2 + dd : a2;
+  }
+  return (a1 + a2) * inv;
+}
+
+// candidates of a destination frame D in memory
+template <int BS>
+struct ArpsFrame {
+  const double* D;
+  uint32_t nr;
+  __device__ double cost(const ArpsRef<BS>& ref, int r, int c, double inv) const {
+    return arps_cost<BS>(ref, D + r + (size_t)nr * c, (size_t)nr, inv);
+  }
+  __device__ double cost_any(const ArpsRef<BS>& ref, const double*, int r, int c, double inv) const {
+    return cost(ref, r, c, inv);
+  }
+};
+
+// and of its tile in LDS, from row r0 and column c0
+template <int BS, int STRIDE>
+struct ArpsLds {
+  const double* t;
+  int r0, c0, rows, cols;
+  const double* D;
+  uint32_t nr;
+  __device__ double cost(const ArpsRef<BS>& ref, int r, int c, double inv) const {
+    return arps_cost<BS>(ref, t + (r - r0) + STRIDE * (c - c0), STRIDE, inv);
+  }
+  // A candidate that may lie outside: a first search over values that are no
+  // numbers can end anywhere, and the second starts from there.  B: the
+  // reference block in its frame.
+  __device__ double cost_any(const ArpsRef<BS>& ref, const double* B, int r, int c, double inv) const {
+    if (r >= r0 && c >= c0 && r + BS <= r0 + rows && c + BS <= c0 + cols) return cost(ref, r, c, inv);
+    return arps_cost_far<BS>(B, D + r + (size_t)nr * c, nr, inv);
+  }
+};
 
 struct Visit {
   uint32_t* w;
@@ -303,19 +376,24 @@ struct Visit {
   }
 };
 
-template <int BS>
-__device__ void arps_search(const double* __restrict__ win, uint32_t nr, uint32_t nc, uint32_t fs, int n1, int it,
-                            int src, int dst, int pmy, int pmx, int mw, Visit& vis, int& oy, int& ox) {
-  const int i = it % n1, j = it / n1;
+// Up to this block side the points of a search step are unrolled; above it
+// their candidates in flight would cost waves (4 x 4: 5.5 ms unrolled, 6.1
+// not; 8 x 8: 10.3 unrolled, 7.1 not).  Likewise the two searches of a job,
+// the first of which starts without motion.
+constexpr int kArpsUnrolled = 5;
+
+// the search of block (i, j) of the frame at S; D: its candidates
+template <int BS, class Dst>
+__device__ __forceinline__ void arps_search(const double* __restrict__ S, const Dst& D, uint32_t nr, uint32_t nc,
+                                            int i, int j, int pmy, int pmx, int mw, Visit& vis, int& oy, int& ox) {
   const int Nx = (int)nr, Ny = (int)nc;
   const double inv = 1.0 / (BS * BS);
   ArpsRef<BS> ref;
-  ref.load(win + (size_t)src * fs + i + (size_t)nr * j, nr);
-  const double* D = win + (size_t)dst * fs;
+  ref.load(S + i + (size_t)nr * j, nr);
   const int Wd = 2 * mw + 1;
   vis.clear((Wd * Wd + 31) / 32);
   int x = j, y = i;
-  double cost = arps_cost<BS>(ref, D, nr, i, j, inv);
+  double cost = D.cost(ref, i, j, inv);
   vis.set(mw, mw);
   int step, maxIdx;
   if (j == 0) {
@@ -326,29 +404,30 @@ __device__ void arps_search(const double* __restrict__ win, uint32_t nr, uint32_
     step = (xT <= yT) ? yT : xT;
     maxIdx = ((yT == 0 && xT == step) || (xT == 0 && yT == step)) ? 5 : 6;
   }
-  // LDSP (src/arps.hpp:206-294): points (hor, ver) in index order
-  const int lh[6] = {0, -step, 0, step, 0, pmx};
-  const int lv[6] = {-step, 0, 0, 0, step, pmy};
+  // LDSP (src/arps.hpp:206-294): points (hor, ver) in index order; k = 2 is
+  // the block's own place
   double best = 1e9;
-  int bh = lh[0], bv = lv[0];
-#pragma unroll
+  int bh = 0, bv = -step;
+#pragma unroll BS <= kArpsUnrolled ? 6 : 1
   for (int k = 0; k < 6; ++k) {
+    const int lh = k == 1 ? -step : k == 3 ? step : k == 5 ? pmx : 0;
+    const int lv = k == 0 ? -step : k == 4 ? step : k == 5 ? pmy : 0;
     double ck = 1e9;
     if (k == 2) {
       ck = cost;
     } else if (k < maxIdx) {
-      const int rv = y + lv[k], rh = x + lh[k];
+      const int rv = y + lv, rh = x + lh;
       const bool skip = (step == 0) || rh < 0 || rv < 0 || (rh + BS - 1) >= Ny || (rv + BS - 1) >= Nx;
       if (!skip) {
-        ck = arps_cost<BS>(ref, D, nr, rv, rh, inv);
-        const int vr = lv[k] + mw, vc = lh[k] + mw;
+        ck = D.cost_any(ref, S + i + (size_t)nr * j, rv, rh, inv);
+        const int vr = lv + mw, vc = lh + mw;
         if (vr >= 0 && vr < Wd && vc >= 0 && vc < Wd) vis.set(vr, vc);
       }
     }
     if (k == 0 || ck < best) {
       best = ck;
-      bh = lh[k];
-      bv = lv[k];
+      bh = lh;
+      bv = lv;
     }
   }
   x += bh;
@@ -356,34 +435,34 @@ __device__ void arps_search(const double* __restrict__ win, uint32_t nr, uint32_
   cost = best;
   // SDSP (src/arps.hpp:299-368); it can take at most Wd*Wd moves, since every
   // move goes to a freshly evaluated offset inside the search window.
-  const int sh_[5] = {0, -1, 0, 1, 0};
-  const int sv_[5] = {-1, 0, 0, 0, 1};
+  const int top = max(0, i - mw), bottom = min(Nx - BS, i + mw), left = max(0, j - mw), right = min(Ny - BS, j + mw);
   for (int n = 0; n < Wd * Wd + 2; ++n) {
     double b2 = 1e9;
-    int k2 = 0;
-#pragma unroll
+    int bs_h = 0, bs_v = -1;
+#pragma unroll BS <= kArpsUnrolled ? 5 : 1
     for (int k = 0; k < 5; ++k) {
+      const int sh = k == 1 ? -1 : k == 3 ? 1 : 0, sv = k == 0 ? -1 : k == 4 ? 1 : 0;
       double ck = 1e9;
       if (k == 2) {
         ck = cost;
       } else {
-        const int rv = y + sv_[k], rh = x + sh_[k];
-        bool skip = rh < 0 || rv < 0 || (rh + BS - 1) >= Ny || (rv + BS - 1) >= Nx || rh < (j - mw) ||
-                    rh > (j + mw) || rv < (i - mw) || rv > (i + mw);
-        if (!skip) skip = vis.get(y - i + sv_[k] + mw, x - j + sh_[k] + mw);
+        const int rv = y + sv, rh = x + sh;
+        bool skip = rv < top || rv > bottom || rh < left || rh > right;
+        if (!skip) skip = vis.get(rv - i + mw, rh - j + mw);
         if (!skip) {
-          ck = arps_cost<BS>(ref, D, nr, rv, rh, inv);
-          vis.set(y - i + sv_[k] + mw, x - j + sh_[k] + mw);
+          ck = D.cost(ref, rv, rh, inv);
+          vis.set(rv - i + mw, rh - j + mw);
         }
       }
       if (k == 0 || ck < b2) {
         b2 = ck;
-        k2 = k;
+        bs_h = sh;
+        bs_v = sv;
       }
     }
-    if (k2 == 2) break;
-    x += sh_[k2];
-    y += sv_[k2];
+    if (bs_h == 0 && bs_v == 0) break;
+    x += bs_h;
+    y += bs_v;
     cost = b2;
   }
   oy = y;
@@ -391,43 +470,105 @@ __device__ void arps_search(const double* __restrict__ win, uint32_t nr, uint32_
 }
 
 // jobs: int16 [nb][max_jobs][4] = (src_a, dst_a, src_b, dst_b); pass b (if
-// src_b >= 0) reads the motion pass a left in the same slot.
-template <int BS, int MW>
-__global__ __launch_bounds__(ArpsCfg<MW>::kThreads) void k_arps(const double* __restrict__ w64,
+// src_b >= 0) starts from the motion that pass a found for the same block.
+template <int BS>
+__global__ __launch_bounds__(kArpsWideThreads) void k_arps_wide(const double* __restrict__ w64,
                                                                 const int16_t* __restrict__ jobs, uint32_t max_jobs,
                                                                 uint32_t nr, uint32_t nc, uint32_t fs, uint32_t nw,
                                                                 uint32_t vol, uint32_t p_all, int n1, int mw,
                                                                 int32_t* __restrict__ pos) {
-  constexpr int kThreads = ArpsCfg<MW>::kThreads;
-  __shared__ uint32_t sv[ArpsCfg<MW>::kWords * kThreads];
+  __shared__ uint32_t sv[arps_words(kArpsMaxMwWide) * kArpsWideThreads];
   const uint32_t b = blockIdx.z, job = blockIdx.y;
   const int it = blockIdx.x * blockDim.x + threadIdx.x;
   const int16_t* J = jobs + ((size_t)b * max_jobs + job) * 4;
   const int sa = J[0], da = J[1], sb = J[2], db = J[3];
   if (sa < 0 || it >= (int)p_all) return;
-  Visit vis{sv + threadIdx.x, kThreads, 2 * mw + 1};
+  Visit vis{sv + threadIdx.x, kArpsWideThreads, 2 * mw + 1};
   const double* win = w64 + (size_t)b * vol;
+  const int i = it % n1, j = it / n1;
   int y, x;
-  arps_search<BS>(win, nr, nc, fs, n1, it, sa, da, 0, 0, mw, vis, y, x);
+  arps_search<BS>(win + (size_t)sa * fs, ArpsFrame<BS>{win + (size_t)da * fs, nr}, nr, nc, i, j, 0, 0, mw, vis, y, x);
   pos[((size_t)b * nw + da) * p_all + it] = (int32_t)(y | (x << 16));
   if (sb >= 0) {
-    const int i = it % n1, j = it / n1;
     int y2, x2;
-    arps_search<BS>(win, nr, nc, fs, n1, it, sb, db, y - i, x - j, mw, vis, y2, x2);
+    arps_search<BS>(win + (size_t)sb * fs, ArpsFrame<BS>{win + (size_t)db * fs, nr}, nr, nc, i, j, y - i, x - j, mw,
+                    vis, y2, x2);
     pos[((size_t)b * nw + db) * p_all + it] = (int32_t)(y2 | (x2 << 16));
   }
 }
 
-template <int MW>
-hipError_t launch_arps_mw(const double* w64, const int16_t* jobs, uint32_t max_jobs, uint32_t nb, const Shape& sh,
-                          int mw, int32_t* pos, hipStream_t s) {
-  constexpr int kThreads = ArpsCfg<MW>::kThreads;
-  const dim3 grid((sh.p_all + kThreads - 1) / kThreads, max_jobs, nb);
-  const dim3 blk(kThreads);
-#define PG_ARPS(B)                                                                                              \
-  case B:                                                                                                       \
-    hipLaunchKernelGGL((k_arps<B, MW>), grid, blk, 0, s, w64, jobs, max_jobs, sh.nr, sh.nc, sh.fs, sh.nw, sh.vol, \
-                       sh.p_all, (int)sh.n1, mw, pos);                                                          \
+// tr x tc blocks a workgroup, from block row (blockIdx.x % tiles_r) * tr;
+// dynamic LDS: the tile (kStride x (tc + BS - 1 + 2 halo) pixels), then the
+// visited maps
+template <int BS, int MW>
+__global__ __launch_bounds__((ArpsTile<BS, MW>::kThreads)) __attribute__((amdgpu_waves_per_eu(arps_waves(BS)))) void k_arps(
+    const double* __restrict__ w64, const int16_t* __restrict__ jobs, uint32_t max_jobs, uint32_t nr, uint32_t nc,
+    uint32_t fs, uint32_t nw, uint32_t vol, uint32_t p_all, int n1, int mw, int tr, int tc, int tiles_r,
+    int32_t* __restrict__ pos) {
+  using Tile = ArpsTile<BS, MW>;
+  constexpr int kThreads = Tile::kThreads, kStride = Tile::kStride;
+  extern __shared__ double arps_lds[];
+  const uint32_t b = blockIdx.z, job = blockIdx.y;
+  const int16_t* J = jobs + ((size_t)b * max_jobs + job) * 4;
+  const int sa = J[0], da = J[1], sb = J[2], db = J[3];
+  const int t = (int)threadIdx.x, halo = max(mw, 2);
+  const int i0 = ((int)blockIdx.x % tiles_r) * tr, j0 = ((int)blockIdx.x / tiles_r) * tc;
+  const int i = i0 + t % tr, j = j0 + t / tr;
+  const bool valid = t < tr * tc && i < n1 && j < n1;
+  const int it = i + n1 * j;
+  const double* win = w64 + (size_t)b * vol;
+  const int rows = tr + BS - 1 + 2 * halo, cols = tc + BS - 1 + 2 * halo;
+  Visit vis{(uint32_t*)(arps_lds + kStride * cols) + t, kThreads, 2 * mw + 1};
+  ArpsLds<BS, kStride> D{arps_lds, i0 - halo, j0 - halo, rows, cols, nullptr, nr};
+  int y = i, x = j;
+#pragma unroll BS <= kArpsUnrolled ? 2 : 1
+  for (int pass = 0; pass < 2; ++pass) {
+    const int src = pass ? sb : sa, dst = pass ? db : da;
+    if (src < 0) return;  // (the whole workgroup)
+    const double* F = D.D = win + (size_t)dst * fs;
+    __syncthreads();
+    // pixels outside the frame repeat its edge; no candidate reaches them
+    for (int c = t / 64; c < cols; c += kThreads / 64) {
+      const double* col = F + (size_t)nr * min(max(D.c0 + c, 0), (int)nc - 1);
+      for (int r = t % 64; r < rows; r += 64) arps_lds[r + kStride * c] = col[min(max(D.r0 + r, 0), (int)nr - 1)];
+    }
+    __syncthreads();
+    if (valid) {
+      const int pmy = y - i, pmx = x - j;
+      arps_search<BS>(win + (size_t)src * fs, D, nr, nc, i, j, pmy, pmx, mw, vis, y, x);
+      pos[((size_t)b * nw + dst) * p_all + it] = (int32_t)(y | (x << 16));
+    }
+  }
+}
+
+template <int BS, int MW>
+hipError_t launch_arps_tiles(const double* w64, const int16_t* jobs, uint32_t max_jobs, uint32_t nb, const Shape& sh,
+                             int mw, int32_t* pos, hipStream_t s) {
+  using Tile = ArpsTile<BS, MW>;
+  // full waves for every frame size: the block rows in equal tiles of at most
+  // 64, then as many columns as threads (and 64 KB of LDS) are left for
+  const int n1 = (int)sh.n1, tiles_r = (n1 + Tile::kRows - 1) / Tile::kRows, tr = (n1 + tiles_r - 1) / tiles_r;
+  int tc = std::min(std::min(Tile::kThreads / tr, n1), 16);
+  auto bytes = [&](int c) {
+    return sizeof(double) * Tile::kStride * (c + BS - 1 + 2 * std::max(mw, 2)) + 4ull * arps_words(mw) * Tile::kThreads;
+  };
+  while (tc > 1 && bytes(tc) > 65536) --tc;
+  const dim3 grid(tiles_r * ((n1 + tc - 1) / tc), max_jobs, nb);
+  hipLaunchKernelGGL((k_arps<BS, MW>), grid, dim3(Tile::kThreads), bytes(tc), s, w64, jobs, max_jobs, sh.nr, sh.nc,
+                     sh.fs, sh.nw, sh.vol, sh.p_all, n1, mw, tr, tc, tiles_r, pos);
+  return hipGetLastError();
+}
+
+hipError_t launch_arps(const double* w64, const int16_t* jobs, uint32_t max_jobs, uint32_t nb, const Shape& sh,
+                       int mw, int32_t* pos, hipStream_t s) {
+  if (mw < 0 || mw > kArpsMaxMwWide) return hipErrorInvalidValue;
+#define PG_ARPS(B)                                                                                                 \
+  case B:                                                                                                          \
+    if (mw <= 7) return launch_arps_tiles<B, 7>(w64, jobs, max_jobs, nb, sh, mw, pos, s);                          \
+    if (mw <= kArpsMaxMw) return launch_arps_tiles<B, kArpsMaxMw>(w64, jobs, max_jobs, nb, sh, mw, pos, s);        \
+    hipLaunchKernelGGL((k_arps_wide<B>), dim3((sh.p_all + kArpsWideThreads - 1) / kArpsWideThreads, max_jobs, nb), \
+                       dim3(kArpsWideThreads), 0, s, w64, jobs, max_jobs, sh.nr, sh.nc, sh.fs, sh.nw, sh.vol,      \
+                       sh.p_all, (int)sh.n1, mw, pos);                                                             \
     break;
   switch (sh.bs) {
     PG_ARPS(2) PG_ARPS(3) PG_ARPS(4) PG_ARPS(5) PG_ARPS(6) PG_ARPS(7) PG_ARPS(8) PG_ARPS(16)
@@ -435,13 +576,6 @@ hipError_t launch_arps_mw(const double* w64, const int16_t* jobs, uint32_t max_j
   }
 #undef PG_ARPS
   return hipGetLastError();
-}
-
-hipError_t launch_arps(const double* w64, const int16_t* jobs, uint32_t max_jobs, uint32_t nb, const Shape& sh,
-                       int mw, int32_t* pos, hipStream_t s) {
-  if (mw <= kArpsMaxMw) return launch_arps_mw<kArpsMaxMw>(w64, jobs, max_jobs, nb, sh, mw, pos, s);
-  if (mw <= kArpsMaxMwWide) return launch_arps_mw<kArpsMaxMwWide>(w64, jobs, max_jobs, nb, sh, mw, pos, s);
-  return hipErrorInvalidValue;
 }
 
 // Shrink factor d = g(s)/s of a singular value s of a patch whose largest
