@@ -40,28 +40,50 @@ __device__ __forceinline__ double sqrt_(double x) { return sqrt(x); }
 __device__ __forceinline__ float rsq_(float x) { return __builtin_amdgcn_rsqf(x); }
 __device__ __forceinline__ double rsq_(double x) { return 1.0 / sqrt(x); }
 
-// The pairs of a sweep in groups of two: anti-diagonals i + j = 1 .. 2 N - 3,
-// neighbours (i, j) and (i + 1, j - 1) of one anti-diagonal together, a last
-// odd one alone (k >= l).
+// The pairs of a sweep in groups of at most four that share no column, with
+// the bits of the row-cyclic order (0, 1), (0, 2) .. (1, 2) ..: there column c
+// meets the others in ascending order, so a pair is due when each of its
+// columns is the other's next.  Of those due the lowest anti-diagonals go
+// first.
 struct PairGroup {
-  int i, j, k, l;
+  int n = 0, i[4] = {0, 0, 0, 0}, j[4] = {0, 0, 0, 0};
 };
 template <int N>
 struct Sweep {
-  static constexpr int first(int d) { return d > N - 1 ? d - (N - 1) : 0; }
-  static constexpr int pairs(int d) { return (d - 1) / 2 - first(d) + 1; }
-  static constexpr int count() {
-    int c = 0;
-    for (int d = 1; d < 2 * N - 2; ++d) c += (pairs(d) + 1) / 2;
-    return c;
+  struct Table {
+    PairGroup g[N * (N - 1) / 2];
+    int groups = 0;
+  };
+  static constexpr Table make() {
+    Table t{};
+    int next[N] = {};  // the column that column c meets next (N: none)
+    next[0] = 1;
+    for (int left = N * (N - 1) / 2; left > 0;) {
+      PairGroup q{};
+      for (; q.n < 4; ++q.n) {
+        int bi = -1;
+        for (int i = 0; i < N; ++i) {
+          const int k = next[i];
+          if (k <= i || k >= N || next[k] != i) continue;
+          bool in = false;
+          for (int z = 0; z < q.n; ++z) in = in || q.i[z] == i;
+          if (!in && (bi < 0 || i + k < bi + next[bi])) bi = i;
+        }
+        if (bi < 0) break;
+        q.i[q.n] = bi;
+        q.j[q.n] = next[bi];
+      }
+      for (int z = 0; z < q.n; ++z) {
+        const int i = q.i[z], k = q.j[z];
+        next[i] = k + 1;
+        next[k] = i + 1 == k ? k + 1 : i + 1;
+      }
+      t.g[t.groups++] = q;
+      left -= q.n;
+    }
+    return t;
   }
-  static constexpr int kGroups = count();
-  static constexpr PairGroup group(int g) {
-    int d = 1;
-    for (; g >= (pairs(d) + 1) / 2; ++d) g -= (pairs(d) + 1) / 2;
-    const int i = first(d) + 2 * g;
-    return {i, d - i, i + 1, d - i - 1};
-  }
+  static constexpr Table kTable = make();
 };
 template <class F, int... G>
 __device__ __forceinline__ void for_all(std::integer_sequence<int, G...>, F&& f) {
@@ -113,14 +135,20 @@ __device__ __forceinline__ void rotate2(double& xi, double& xj, double& yi, doub
 // Waves per SIMD the register allocator is held to: 130 registers would leave
 // the 64 x 15 matrices of patch 8 three; 31 columns, left alone, 172 for two
 // (64 x 31, 1.36 M matrices: 158 ms with two waves, 152 with three).
-template <int BS, int N, int L, class T>
+template <int BS, int N, int L, class T, bool RT>
 constexpr int svd_min_waves() {
-  if (sizeof(T) != 4) return 1;
+  if (sizeof(T) != 4 || RT) return 1;
   return N > 16 ? 3 : (BS == 8 && N == 15 && L == 16) ? 4 : 1;
 }
 
+// whether a sweep takes four pairs at a time
+template <int N, int L, class T>
+constexpr bool quads() {
+  return sizeof(T) == 4 && L >= 4 && N > 8;
+}
+
 template <int BS, int N, int L, class T, bool RT = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(svd_min_waves<BS, N, L, T>()))) void k_svd(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(svd_min_waves<BS, N, L, T, RT>()))) void k_svd(
     const T* __restrict__ u32, const int32_t* __restrict__ pos, const uint32_t* __restrict__ sel, uint32_t nvar,
     uint32_t nvar_stored, uint32_t p_sel, uint32_t p_all, uint32_t nr, uint32_t fs, uint32_t nw, uint32_t vol,
     uint32_t lim, uint32_t fstride, int max_sweeps, T tol2, T* __restrict__ factors, uint32_t* __restrict__ stats) {
@@ -195,54 +223,81 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(svd_min_wav
       tsum = fma(t, t, tsum);
       turn(i, j, cs, cs * t);
     };
-    auto two = [&](int i, int j, int k, int l) __attribute__((always_inline)) {
-      const T c = column_dot(i, j), e = column_dot(k, l);
-      const bool rc = c * c > tol2 * a[i] * a[j], re = e * e > tol2 * a[k] * a[l];
-      if (!__any(rc || re)) return;
-      const T t = tangent(i, j, c, rc), u = tangent(k, l, e, re);
-      const T cs = rsq_(fma(t, t, T(1))), du = rsq_(fma(u, u, T(1)));
-      a[i] = fma(-t, c, a[i]);
-      a[j] = fma(t, c, a[j]);
-      a[k] = fma(-u, e, a[k]);
-      a[l] = fma(u, e, a[l]);
+    // Up to four pairs that share no column.  Lane l of a group works out the
+    // rotation of pair l % 4 and hands it to its neighbours, where each lane
+    // had worked out every pair's: the reciprocals and roots take four times a
+    // plain instruction's slot, and were most of what a pair cost beside its
+    // dot product and update.
+    auto quad = [&](auto qc) __attribute__((always_inline)) {
+      constexpr PairGroup q = Sweep<N>::kTable.g[decltype(qc)::value];
+      const bool odd = lane & 1, high = lane & 2;
+      auto mine = [&](float v0, float v1, float v2, float v3) __attribute__((always_inline)) {
+        return high ? (odd ? v3 : v2) : (odd ? v1 : v0);
+      };
+      float c;
+      if constexpr (L == 4) {
+        // each lane ends with its own pair's sum, added as group_sum does
+        float d[4];
+        static_for<0, 4>([&](auto zc) __attribute__((always_inline)) {
+          constexpr int z = decltype(zc)::value;
+          d[z] = 0.f;
+          if constexpr (z < q.n) {
+            d[z] = x[0][q.i[z]] * x[0][q.j[z]];
+#pragma unroll
+            for (int h = 1; h < R; ++h) d[z] = fma(x[h][q.i[z]], x[h][q.j[z]], d[z]);
+            asm("" : "+v"(d[z]));  // (rounded before the sum)
+          }
+        });
+        const float s01 = (odd ? d[1] : d[0]) + dpp_f<0xB1>(odd ? d[0] : d[1]);
+        const float s23 = (odd ? d[3] : d[2]) + dpp_f<0xB1>(odd ? d[2] : d[3]);
+        c = (high ? s23 : s01) + dpp_f<0x4E>(high ? s01 : s23);
+      } else {
+        float d[4] = {0.f, 0.f, 0.f, 0.f};
+        static_for<0, 4>([&](auto zc) __attribute__((always_inline)) {
+          constexpr int z = decltype(zc)::value;
+          if constexpr (z < q.n) d[z] = column_dot(q.i[z], q.j[z]);
+        });
+        c = mine(d[0], d[1], d[2], d[3]);
+      }
+      float ai = mine(a[q.i[0]], a[q.i[1]], a[q.i[2]], a[q.i[3]]);
+      float aj = mine(a[q.j[0]], a[q.j[1]], a[q.j[2]], a[q.j[3]]);
+      const bool rot = c * c > tol2 * ai * aj;
+      const uint64_t rotates = __ballot(rot);
+      if (!rotates) return;
+      const float zeta = (aj - ai) * rcp_(c + c);
+      const float den = fabs(zeta) + sqrt_(fma(zeta, zeta, 1.f));
+      const float t = rot ? copysign(rcp_(den), zeta) : 0.f;
+      const float cs = rsq_(fma(t, t, 1.f)), sn = cs * t;
+      ai = fma(-t, c, ai);
+      aj = fma(t, c, aj);
       tsum = fma(t, t, tsum);
-      tsum = fma(u, u, tsum);
-      turn(i, j, cs, cs * t);
-      turn(k, l, du, du * u);
-    };
-    // The sweep's order is row-cyclic, (0, 1), (0, 2) .. (1, 2) ..  A pair
-    // depends on those before it that share a column, so the pairs of one
-    // anti-diagonal i + j = d, taken after every smaller d, give the same
-    // bits, and are independent of each other.  Matrices of 31 columns leave
-    // three waves a SIMD: there two pairs go at a time, one's chain (dot
-    // product, reciprocals and roots, update) in the other's waits (64 x 31:
-    // 179 -> 169 ms for 1.36 M matrices).  With more waves it costs: a pair
-    // that does not rotate is skipped only with its neighbour (16 x 15: 53.6
-    // -> 55.8 ms for 19.2 M).
-    // A run-time window length goes by the list as well: a loop that breaks at
-    // n is not unrolled, and X would live in scratch memory.
-    constexpr bool PAIRS = N > 16 && sizeof(T) == 4;
-    if constexpr (PAIRS || RT) {
-      for_all(std::make_integer_sequence<int, Sweep<N>::kGroups>{}, [&](auto gc) __attribute__((always_inline)) {
-        constexpr PairGroup q = Sweep<N>::group(decltype(gc)::value);
-        const bool in = !RT || q.j < n;  // (uniform)
-        if constexpr (q.k >= q.l) {
-          if (in) one(q.i, q.j);
-        } else if constexpr (PAIRS) {
-          if (in)
-            two(q.i, q.j, q.k, q.l);
-          else if (q.l < n)
-            one(q.k, q.l);
-        } else {
-          if (in) one(q.i, q.j);
-          if (!RT || q.l < n) one(q.k, q.l);
+      static_for<0, 4>([&](auto zc) __attribute__((always_inline)) {
+        constexpr int z = decltype(zc)::value, kFrom = z * 0x55;  // quad_perm [z, z, z, z]
+        if constexpr (z < q.n) {
+          if (rotates & (0x1111111111111111ull << z)) {
+            a[q.i[z]] = dpp_f<kFrom>(ai);
+            a[q.j[z]] = dpp_f<kFrom>(aj);
+            turn(q.i[z], q.j[z], dpp_f<kFrom>(cs), dpp_f<kFrom>(sn));
+          }
         }
       });
+    };
+    // Groups pay where they are full for most of a sweep (16 x 15, 19.2 M
+    // matrices: 51.4 -> 45.3 ms; 64 x 15, 1.14 M: 12.8 -> 11.5; 64 x 31, 1.36 M:
+    // 152 -> 130); 7 columns have two pairs to a group (16 x 7, 31 M: 25.9 ms a
+    // pair at a time, 26.1 in groups).
+    if constexpr (quads<N, L, T>() && !RT) {
+      for_all(std::make_integer_sequence<int, Sweep<N>::kTable.groups>{}, quad);
     } else {
 #pragma unroll
-      for (int i = 0; i < N - 1; ++i)
+      for (int i = 0; i < N - 1; ++i) {
+        if (RT && i >= n - 1) break;  // uniform
 #pragma unroll
-        for (int j = i + 1; j < N; ++j) one(i, j);
+        for (int j = i + 1; j < N; ++j) {
+          if (RT && j >= n) break;
+          one(i, j);
+        }
+      }
     }
     if (!__any(tsum > T(0))) break;
   }
@@ -296,10 +351,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(svd_min_wav
   // 19.2 M matrices: 53.6 -> 51.4 ms), at 31 columns fewer addresses (64 x 31:
   // 169 -> 165 ms); at 16 lanes the selects cost more than they save (36 x 15
   // in a batch: 17.6 -> 21.1 ms).
-  constexpr int KG = (L == 4 || N > 16) ? 4 : 1;
+  constexpr int KG = !RT && (L == 4 || N > 16) ? 4 : 1;
 #pragma unroll
   for (int k0 = 0; k0 < SRN; k0 += KG) {
-    if (RT && k0 >= SR) continue;  // (uniform)
+    if (RT && k0 >= SR) break;  // uniform
     if constexpr (KG > 1) {
       // the ranks anew: the row addresses of all N ranks, kept from one
       // group of columns to the next, would cost a wave per SIMD or two
@@ -321,7 +376,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(svd_min_wav
     }
 #pragma unroll
     for (int l = 0; l < N; ++l) {
-      if (RT && l >= n) continue;  // uniform: the zero columns
+      if (RT && l >= n) break;  // uniform: the zero columns
       T mine = T(0);
 #pragma unroll
       for (int z = 0; z < KG; ++z) {
