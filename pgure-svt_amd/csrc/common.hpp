@@ -13,12 +13,6 @@
 
 namespace pgsvt {
 
-// Fixed-point scale of the overlap-add accumulators: contributions are
-// rounded to multiples of 2^-32 and summed in int64, so the sum does not
-// depend on the order the atomics land in (deterministic overlap-add).
-constexpr float kFixScale = 4294967296.0f;   // 2^32
-constexpr double kFixInv = 1.0 / 4294967296.0;
-
 // Variants of the window decomposed for PGURE: the data U and the two
 // perturbed copies U +/- eps2*delta2 (src/pgure.hpp:80-91).  The fourth copy
 // U + eps1*delta1 of the reference equals U exactly (delta1 is an integer

@@ -8,7 +8,6 @@
 //   pos      int32  [nb][nw][p_all]         patch position, row | col << 16
 //   W        int32  [nb][vol]               overlap count per voxel
 //   factors  float  [nb][nvar][p_sel][fstride]  V^T (n x sr), W^T (n x m), s (n)
-//   acc      int64  [nb][nvar][vol]         fixed-point overlap-add sums
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

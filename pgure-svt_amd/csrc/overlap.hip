@@ -285,8 +285,9 @@ __device__ __forceinline__ void load_run(const float* __restrict__ p, float (&x)
 // of it.  A column whose |x| reach 2^e (NaN, infinity) flags its cells,
 // which are then summed in FP64 from the records.
 //
-// Bound: instruction issue and the LDS atomics, then memory (28 bytes a
-// voxel).  256 x 256 x 15 windows at searched lambdas: 15.2 ps a voxel.  The
+// Bound: instruction issue (333 vector instructions per 64 voxels, 16.6 of
+// 28.4 ms) and the LDS atomics (10.7 ms), then memory (28 bytes a voxel).
+// 256 x 256 x 15 windows at searched lambdas: 13.5 ps a voxel.  The
 // form before (rows of a 32 x 8 tile staged in LDS from bucket-sorted rows,
 // each voxel reading its 16 positions and looping over further patches of a
 // position) issued 1,197 vector instructions per 64 voxels, at 4 cycles each
