@@ -315,9 +315,9 @@ def roofline(prof):
 STAGE_KERNELS = {
     "svd_jacobi": ("pgsvt::k_svd<",),
     "divergence_factors": ("pgsvt::k_divq<",),
-    "leading_vectors": ("pgsvt::k_lead",),
-    "eval_reconstruct": ("pgsvt::k_round_prep<", "pgsvt::k_rows<", "pgsvt::k_eval<"),
-    "gather_risk": ("pgsvt::k_overlap<", "pgsvt::k_gather_"),
+    "leading_vectors": ("::k_lead",),
+    "eval_reconstruct": ("pgsvt::k_round_prep<", "::k_rows<", "pgsvt::k_eval<"),
+    "gather_risk": ("::k_overlap<", "pgsvt::k_gather_"),
 }
 
 
