@@ -957,7 +957,10 @@ struct Pipeline {
     sums.alloc((size_t)NS * 6);
     partial_k.alloc((size_t)NB * eval_blocks(sh, 3));
     kept_d.alloc(NB);
-    max_jobs = 2 * g.Nw;
+    // passes of a window at most (arps_jobs): a slot without a job still costs
+    // its workgroups' dispatch (8 x 8 patches of 256 x 256 x 24: 7.1 ms with
+    // 2 Nw slots, 6.8 with these)
+    max_jobs = std::max({1u, g.Nw - 1, 2 * g.fw});
     jobs_d.alloc((size_t)NB * max_jobs * 4);
     if (probe_on) {
       factors_s.alloc((size_t)NB * 3 * sh_s.p_sel * sh.fstride * es);
