@@ -1788,9 +1788,11 @@ uint32_t eval_blocks(const Shape& sh, uint32_t nvar_run) {
   return (sh.p_sel + 3) / 4;  // one 64-lane group per patch
 }
 
-// the rows of the marked patches (see k_rows)
+// the rows of the marked patches (see k_rows): only the FP32 round marks them,
+// and only its callers hold a buffer of rows
 static hipError_t launch_rows(const float* factors, const float* dr, const uint32_t* wl, uint32_t na,
                               uint32_t nvar_stored, const Shape& sh, float* rows, hipStream_t s) {
+  if (!strip_overlap(sh) || !rows) return hipErrorInvalidValue;
   const uint32_t look = 4 * (sh.m <= 16 ? 64 : 16);  // patches a workgroup looks at
   const dim3 grid((sh.p_sel + look - 1) / look, na);
 #define PG_RW(B, N, L, LS)                                                                                       \
@@ -1822,7 +1824,7 @@ hipError_t launch_evaluation(const Shape& sh, const void* factors, const void* d
                        kept);
   const hipError_t e = launch_round_prep(factors, nvar_run == 3 ? divq : nullptr, meta, wl, na, nvar_stored, sh, exp_w,
                                          slot_lam, dr, nvar_run == 3 ? partial : nullptr, kept, s);
-  if (e != hipSuccess) return e;
+  if (e != hipSuccess || !strip_overlap(sh)) return e;  // (FP64: the gather forms the rows)
   return launch_rows((const float*)factors, (const float*)dr, wl, na, nvar_stored, sh, (float*)rows, s);
 }
 
