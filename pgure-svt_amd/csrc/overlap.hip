@@ -135,8 +135,8 @@ __global__ __launch_bounds__(1024) void k_bin_columns(const int32_t* __restrict_
 // W of src/svt.hpp:157-163, the number of patches over each voxel, as 1/W
 // (FP64, 0 where nothing covers it) and, for the divergence sum, delta2/W.
 // One workgroup per strip and frame: a histogram of the patch positions in
-// LDS, then box sums down and across.  wstat[2 b + 1]: the window's largest
-// W (the overlap-add's headroom).
+// LDS, then box sums down and across.  wstat[b (1 + nw) + 1 + k]: the largest W
+// of frame k (the overlap-add's headroom).
 __global__ __launch_bounds__(256) void k_cover(const int2* __restrict__ recs, const int32_t* __restrict__ off,
                                                const uint8_t* __restrict__ d2, uint32_t n, uint32_t nw, uint32_t n1,
                                                uint32_t bs, uint32_t p_sel, uint32_t bins, uint32_t shift, Strips st,
@@ -185,14 +185,14 @@ __global__ __launch_bounds__(256) void k_cover(const int2* __restrict__ recs, co
   for (int o = 32; o > 0; o >>= 1) most = max(most, __shfl_xor(most, o));
   if (threadIdx.x % 64 == 0) wmax[threadIdx.x / 64] = most;
   __syncthreads();
-  if (threadIdx.x == 0) atomicMax(&wstat[2 * b + 1], (uint32_t)max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3])));
+  if (threadIdx.x == 0) atomicMax(&wstat[b * (1 + nw) + 1 + k], (uint32_t)max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3])));
 }
 
 // ---------------------------------------------------- leading vectors --
 // By patch, from the U variant's factors: w_0 (w0 [nb][p_sel][m], may be
 // null) and v_0 as
 // one plane per frame (v0 [nb][nw][p_sel]), and the window's largest finite
-// s_0 (wstat[2 b], as the bits of a non-negative float).  A workgroup takes
+// s_0 (wstat[b (1 + nw)], as the bits of a non-negative float).  A workgroup takes
 // 64 patches: 16 lanes read a patch's vectors, v_0 turns in LDS, so that
 // both sides move whole lines.
 __global__ __launch_bounds__(256) void k_lead(const float* __restrict__ factors, uint32_t nvar_stored, uint32_t p_sel,
@@ -224,7 +224,7 @@ __global__ __launch_bounds__(256) void k_lead(const float* __restrict__ factors,
   for (int o = 32; o > 0; o >>= 1) s = max(s, (uint32_t)__shfl_xor((int)s, o));
   if (threadIdx.x % 64 == 0) top[threadIdx.x / 64] = s;
   __syncthreads();
-  if (threadIdx.x == 0) atomicMax(&wstat[2 * b], max(max(top[0], top[1]), max(top[2], top[3])));
+  if (threadIdx.x == 0) atomicMax(&wstat[b * (1 + nw)], max(max(top[0], top[1]), max(top[2], top[3])));
 }
 
 // --------------------------------------------------------- overlap-add --
@@ -280,7 +280,9 @@ __device__ __forceinline__ void load_run(const float* __restrict__ p, float (&x)
 // Integer sums are the same in every order, so the result is reproducible
 // without a sort.  q = 2^(e - 51) with 2^e above the sum of any column's
 // |x| (the window's largest s_0 bounds the 2-norm of a row), raised where
-// more than 2^11 patches pile on a voxel: an FP32 contribution of at least
+// more than 2^11 patches pile on a voxel of the frame (without motion
+// estimation every patch of the other frames lies on (0, 0); the output frame's
+// sums must not pay for them): an FP32 contribution of at least
 // 2^-24 of the window's largest s_0 is held exactly, a smaller one to 2^-48
 // of it.  A column whose |x| reach 2^e (NaN, infinity) flags its cells,
 // which are then summed in FP64 from the records.
@@ -326,8 +328,9 @@ __global__ __launch_bounds__(512) void k_overlap(const OverlapArgs a) {
   const int32_t lo = O[(uint32_t)max(c0 - BS + 1, 0) >> a.shift];
   const int32_t hi = O[(min((uint32_t)c0 + cols - 1, a.n1 - 1) >> a.shift) + 1];
   // quantum and bound (see above)
-  const float smax = __uint_as_float(a.wstat[2 * b]);
-  const uint32_t wmax = a.wstat[2 * b + 1];
+  const uint32_t* fig = a.wstat + b * (1 + a.nw);
+  const float smax = __uint_as_float(fig[0]);
+  const uint32_t wmax = fig[1 + k];
   const int e = (smax > 0.f ? ilogbf(smax) : 0) + LOGC;
   const int head = max(0, (int)(32 - __clz((int)wmax | 1)) - 11);
   const double quantum = ldexp(1.0, e - 51 + head), magic = 1.5 * ldexp(1.0, e + 1 + head);
