@@ -703,7 +703,7 @@ struct Pipeline {
   // the fused evaluation's static data per window (patches up to 4 x 4):
   // rows w_0 v_0[k] and singular pairs (s_0, s_1) per (frame, bucket place)
   // (FP64; the FP32 overlap-add of strips takes the patches by column, their
-  // leading vectors by patch and 1 + nw figures per window, see launch_bins)
+  // leading vectors by patch and 2 + nw figures per window, see launch_bins)
   DBuf<char> w0b, s01b;
   DBuf<int2> recs;
   DBuf<float> w0, v0;
@@ -933,7 +933,7 @@ struct Pipeline {
       recs.alloc((size_t)NB * sh.nw * sh.p_sel);
       if (fused_eval(sh)) w0.alloc((size_t)NB * sh.p_sel * sh.m);
       v0.alloc((size_t)NB * sh.nw * sh.p_sel);
-      wstat.alloc((1 + sh.nw) * (size_t)NB);
+      wstat.alloc((2 + sh.nw) * (size_t)NB);
     } else {
       const size_t npos = (size_t)sh.n1 * sh.n1;
       cnt.alloc((size_t)NB * sh.nw * npos);
@@ -1007,7 +1007,7 @@ struct Pipeline {
     }
     prof->run("buckets_weights", (double)nb * sh.nw * sh.p_sel, [&] {
       if (strip_overlap(sh)) {
-        hipchk(launch_fill32(wstat.p, (1 + sh.nw) * (size_t)nb, 0, s), "clear window figures");
+        hipchk(launch_fill32(wstat.p, (2 + sh.nw) * (size_t)nb, 0, s), "clear window figures");
         hipchk(launch_bins(pos.p, sel_d.p, nb, sh, off.p, recs.p, s), "bins");
         hipchk(launch_cover(off.p, recs.p, d2.p, nb, sh, d2neg, d2pos, invw.p, optimize ? (float*)dw.p : nullptr,
                             wstat.p, s),
@@ -2341,7 +2341,7 @@ int run_noalloc(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf,
       L.recs = c.take<int2>((size_t)g.Nw * sh.p_sel);
       if (fused_eval(sh)) L.w0 = c.take<float>((size_t)sh.p_sel * sh.m);
       L.v0 = c.take<float>((size_t)g.Nw * sh.p_sel);
-      L.wstat = c.take<uint32_t>(1 + g.Nw);
+      L.wstat = c.take<uint32_t>(2 + g.Nw);
     } else {
       c.take<int32_t>((size_t)g.Nw * npos);
       c.take<int32_t>((size_t)g.Nw * (npos + 1));
@@ -2433,7 +2433,7 @@ int run_noalloc(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf,
     hipchk(launch_fill_ref(L.meta, 1, sh, L.pos, s), "fill_ref");
     if (p.motion_estimation)
       hipchk(launch_arps(median ? L.w64 : L.u64, L.jobs, max_jobs, 1, sh, (int)p.motion_window, L.pos, s), "arps");
-    hipchk(launch_fill32(L.wstat, 1 + g.Nw, 0, s), "clear window figures");
+    hipchk(launch_fill32(L.wstat, 2 + g.Nw, 0, s), "clear window figures");
     hipchk(launch_bins(L.pos, L.sel, 1, sh, L.off, L.recs, s), "bins");
     hipchk(launch_cover(L.off, L.recs, L.d2, 1, sh, d2neg, d2pos, L.invw, L.dw, L.wstat, s), "cover");
     hipchk(launch_fill32(L.stats, 1, 0, s), "clear stats");

@@ -137,9 +137,10 @@ hipError_t launch_gather(const GatherSrc& src, const int32_t* off, const double*
 // up to 4 x 4, w_0 (w0 [nb][p_sel][m]; null for larger ones) out by patch, and launch_overlap adds the rows up, with
 // d_r from launch_evaluation (dr [na][nw][p_sel], by rank, ended by a 0; d_0
 // negative where rank 1 is kept too: then the patch's rows of every frame are
-// in rows [na][nw][p_sel][m]).  wstat [nb][1 + nw]: the window's largest s_0
-// (bits of a float), then each frame's largest W; zeroed by the caller before
-// launch_cover and launch_lead raise them.  Modes and nk as launch_gather.
+// in rows [na][nw][p_sel][m]).  wstat [nb][2 + nw]: the window's largest s_0
+// and the complement of its smallest above 0 (bits of a float), then each
+// frame's largest W; zeroed by the caller before launch_cover and launch_lead
+// raise them.  Modes and nk as launch_gather.
 bool strip_overlap(const Shape& sh);
 uint32_t column_bins(const Shape& sh);
 hipError_t launch_bins(const int32_t* pos, const uint32_t* sel, uint32_t nb, const Shape& sh, int32_t* off,

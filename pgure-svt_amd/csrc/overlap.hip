@@ -46,6 +46,9 @@ Strips strips_of(uint32_t n, uint32_t bs) {
   s.nc = (n + s.tc - 1) / s.tc;
   return s;
 }
+// cells of a strip a thread holds at most (sum_by_magnitude): 4,096 over 256
+// threads, 7,600 over 512
+constexpr int kCellsPerThread = 16;
 // strips of the cover counts: their two LDS arrays stay within 60 KB
 Strips cover_strips(uint32_t n, uint32_t bs) {
   Strips s{};
@@ -135,7 +138,7 @@ __global__ __launch_bounds__(1024) void k_bin_columns(const int32_t* __restrict_
 // W of src/svt.hpp:157-163, the number of patches over each voxel, as 1/W
 // (FP64, 0 where nothing covers it) and, for the divergence sum, delta2/W.
 // One workgroup per strip and frame: a histogram of the patch positions in
-// LDS, then box sums down and across.  wstat[b (1 + nw) + 1 + k]: the largest W
+// LDS, then box sums down and across.  wstat[b (2 + nw) + 2 + k]: the largest W
 // of frame k (the overlap-add's headroom).
 __global__ __launch_bounds__(256) void k_cover(const int2* __restrict__ recs, const int32_t* __restrict__ off,
                                                const uint8_t* __restrict__ d2, uint32_t n, uint32_t nw, uint32_t n1,
@@ -185,24 +188,24 @@ __global__ __launch_bounds__(256) void k_cover(const int2* __restrict__ recs, co
   for (int o = 32; o > 0; o >>= 1) most = max(most, __shfl_xor(most, o));
   if (threadIdx.x % 64 == 0) wmax[threadIdx.x / 64] = most;
   __syncthreads();
-  if (threadIdx.x == 0) atomicMax(&wstat[b * (1 + nw) + 1 + k], (uint32_t)max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3])));
+  if (threadIdx.x == 0) atomicMax(&wstat[b * (2 + nw) + 2 + k], (uint32_t)max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3])));
 }
 
 // ---------------------------------------------------- leading vectors --
 // By patch, from the U variant's factors: w_0 (w0 [nb][p_sel][m], may be
 // null) and v_0 as
 // one plane per frame (v0 [nb][nw][p_sel]), and the window's largest finite
-// s_0 (wstat[b (1 + nw)], as the bits of a non-negative float).  A workgroup takes
-// 64 patches: 16 lanes read a patch's vectors, v_0 turns in LDS, so that
+// s_0 and the complement of its smallest above 0 (wstat[b (2 + nw)] and the
+// next word, as the bits of a float).  A workgroup takes 64 patches: 16 lanes read a patch's vectors, v_0 turns in LDS, so that
 // both sides move whole lines.
 __global__ __launch_bounds__(256) void k_lead(const float* __restrict__ factors, uint32_t nvar_stored, uint32_t p_sel,
                                               uint32_t nw, uint32_t m, uint32_t fstride, float* __restrict__ w0,
                                               float* __restrict__ v0, uint32_t* __restrict__ wstat) {
   __shared__ float tv[32][65];
-  __shared__ uint32_t top[4];
+  __shared__ uint32_t top[4], low[4];
   const uint32_t b = blockIdx.y, p0 = blockIdx.x * 64, SR = (nw + 3) & ~3u;
   const uint32_t g = threadIdx.x / 16, l = threadIdx.x % 16;
-  uint32_t s = 0;
+  uint32_t s = 0, c = 0;
   for (uint32_t q = 0; q < 4; ++q) {
     const uint32_t pl = q * 16 + g, p = p0 + pl;
     if (p >= p_sel) continue;
@@ -214,6 +217,7 @@ __global__ __launch_bounds__(256) void k_lead(const float* __restrict__ factors,
     if (l == 0) {
       const uint32_t u = __float_as_uint(FW[nw * m]);
       s = max(s, u < 0x7f800000u ? u : 0u);
+      c = max(c, u - 1u < 0x7f7fffffu ? ~u : 0u);
     }
   }
   __syncthreads();
@@ -221,10 +225,19 @@ __global__ __launch_bounds__(256) void k_lead(const float* __restrict__ factors,
     const uint32_t k = e / 64, pl = e % 64;
     if (p0 + pl < p_sel) v0[((size_t)b * nw + k) * p_sel + p0 + pl] = tv[k][pl];
   }
-  for (int o = 32; o > 0; o >>= 1) s = max(s, (uint32_t)__shfl_xor((int)s, o));
-  if (threadIdx.x % 64 == 0) top[threadIdx.x / 64] = s;
+  for (int o = 32; o > 0; o >>= 1) {
+    s = max(s, (uint32_t)__shfl_xor((int)s, o));
+    c = max(c, (uint32_t)__shfl_xor((int)c, o));
+  }
+  if (threadIdx.x % 64 == 0) {
+    top[threadIdx.x / 64] = s;
+    low[threadIdx.x / 64] = c;
+  }
   __syncthreads();
-  if (threadIdx.x == 0) atomicMax(&wstat[b * (1 + nw)], max(max(top[0], top[1]), max(top[2], top[3])));
+  if (threadIdx.x == 0) {
+    atomicMax(&wstat[b * (2 + nw)], max(max(top[0], top[1]), max(top[2], top[3])));
+    atomicMax(&wstat[b * (2 + nw) + 1], max(max(low[0], low[1]), max(low[2], low[3])));
+  }
 }
 
 // --------------------------------------------------------- overlap-add --
@@ -267,6 +280,85 @@ __device__ __forceinline__ void load_run(const float* __restrict__ p, float (&x)
   }
 }
 
+// A strip's sums with a quantum for each class of 2^27 in magnitude, in FP64
+// bits into the cells; each(f) calls f(x, cell, row) for every column of the
+// thread's records.  The first walk finds the largest column and the cells that
+// NaN or infinities reach (a cell's bits 1, 2, 4), each further one adds up
+// the columns of one class (by the sum of their finite |x|) and finds the
+// largest below it; the classes' sums are added from the largest down.  Every
+// column is held to 2^-25 of its own |x|, in any order, and a strip costs a few
+// walks (256 x 256 x 3, half of it 1e-20 of the rest, plain threshold 0: 0.16 ms
+// a lambda, 0.05 where no strip comes here; a walk of the strip's records for
+// each cell that is not finite 6.4).  The cells' places are worked out anew at
+// each use: 16 addresses held through the walks would cost the whole kernel
+// two of its six waves per SIMD.
+template <int BS, bool CUT, class Each>
+__device__ __forceinline__ void sum_by_magnitude(unsigned long long* acc, const Strips& st, uint32_t rows,
+                                                 uint32_t cols, int head, Each each) {
+  __shared__ unsigned long long top;  // the largest column left (bits of a non-negative double)
+  double run[kCellsPerThread];
+  auto own = [&](auto f) {
+    uint32_t t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+#pragma unroll
+    for (int i = 0; i < kCellsPerThread; ++i) {
+      const uint32_t v = t + (uint32_t)i * blockDim.x;
+      if (v < rows * cols) f(i, acc[v / rows * st.ld + v % rows]);
+    }
+  };
+  auto clear = [&] {
+    for (uint32_t c = threadIdx.x; c < st.tc * st.ld; c += blockDim.x) acc[c] = 0ull;
+    if (threadIdx.x == 0) top = 0ull;
+    __syncthreads();
+  };
+  auto inside = [&](int row) { return !CUT || (uint32_t)row < rows; };
+  auto magnitude = [](const float(&x)[BS]) {
+    double m = 0.0;
+    for (int q = 0; q < BS; ++q) m += __builtin_isfinite(x[q]) ? fabs((double)x[q]) : 0.0;
+    return m;
+  };
+  double most = 0.0;
+  clear();
+  each([&](const float(&x)[BS], uint32_t cell, int row) {
+    most = fmax(most, magnitude(x));
+    for (int q = 0; q < BS; ++q)
+      if (!__builtin_isfinite(x[q]) && inside(row + q))
+        atomicOr(&acc[cell + q], x[q] != x[q] ? 1ull : x[q] > 0.f ? 2ull : 4ull);
+  });
+  atomicMax(&top, __builtin_bit_cast(unsigned long long, most));
+  __syncthreads();
+  own([&](int i, unsigned long long bits) {
+    run[i] = (bits & 1ull) || (bits & 6ull) == 6ull ? __builtin_nan("")
+             : bits & 2ull                          ? __builtin_inf()
+             : bits & 4ull                          ? -__builtin_inf()
+                                                    : 0.0;
+  });
+  for (;;) {
+    const double t = __builtin_bit_cast(double, top);
+    __syncthreads();
+    if (!(t > 0.0)) break;  // (each class starts below the one before: 48 at most)
+    clear();
+    const int e = ilogb(t) + 1;
+    const double quantum = ldexp(1.0, e - 51 + head), magic = 1.5 * ldexp(1.0, e + 1 + head);
+    const double high = ldexp(1.0, e), low = ldexp(1.0, e - 27 + head);
+    most = 0.0;
+    each([&](const float(&x)[BS], uint32_t cell, int row) {
+      const double m = magnitude(x);
+      if (m < low) most = fmax(most, m);
+      if (!(m >= low && m < high)) return;
+      for (int q = 0; q < BS; ++q) {
+        const unsigned long long y = __builtin_bit_cast(unsigned long long, (double)x[q] + magic) -
+                                     __builtin_bit_cast(unsigned long long, magic);
+        if (__builtin_isfinite(x[q]) && inside(row + q)) atomicAdd(&acc[cell + q], y);
+      }
+    });
+    atomicMax(&top, __builtin_bit_cast(unsigned long long, most));
+    __syncthreads();
+    own([&](int i, unsigned long long bits) { run[i] += (double)(long long)bits * quantum; });
+  }
+  own([&](int i, unsigned long long& cell) { cell = __builtin_bit_cast(unsigned long long, run[i]); });
+}
+
 // Uhat = (sum of the patches' rows over each voxel) / W.  The row of patch p
 // in frame k is B[q][k] = d_0 w_0[q] v_0[k] (lead_product) where the patch
 // keeps rank 0 alone (d_0 > 0, by patch, from k_round_prep), and the row that
@@ -284,8 +376,11 @@ __device__ __forceinline__ void load_run(const float* __restrict__ p, float (&x)
 // estimation every patch of the other frames lies on (0, 0); the output frame's
 // sums must not pay for them): an FP32 contribution of at least
 // 2^-24 of the window's largest s_0 is held exactly, a smaller one to 2^-48
-// of it.  A column whose |x| reach 2^e (NaN, infinity) flags its cells,
-// which are then summed in FP64 from the records.
+// of it, which is 2^-25 of its own patch's s_0 or finer in every window whose
+// s_0 stay within a factor of 2^24 (16-bit counts do).  Strips with a column
+// that this does not hold, one whose |x| reach 2^e or are no numbers, or,
+// in a window of wider s_0, one whose |x| sum to less than 2^24 q, are
+// summed again by magnitude (sum_by_magnitude).
 //
 // Bound: instruction issue (333 vector instructions per 64 voxels, 16.6 of
 // 28.4 ms) and the LDS atomics (10.7 ms), then memory (28 bytes a voxel).
@@ -306,11 +401,10 @@ __global__ __launch_bounds__(512) void k_overlap(const OverlapArgs a) {
   constexpr int U = BS <= 4 ? 4 : BS <= 8 ? 2 : 1;  // rows in flight per lane group
   // 2^LOGC bounds sum |x| of a column over its 2-norm (sqrt(BS)), once doubled
   constexpr int LOGC = BS <= 4 ? 3 : 4;
-  extern __shared__ unsigned long long acc[];  // [tc][ld] cells, then a bit per cell
+  extern __shared__ unsigned long long acc[];  // [tc][ld] cells
   __shared__ double sm[5][8];
-  __shared__ uint32_t flagged;
+  __shared__ uint32_t beyond;  // a column the quantum does not hold
   const Strips st = a.st;
-  uint32_t* bad = reinterpret_cast<uint32_t*>(acc + st.tc * st.ld);
   uint32_t bx, slot;
   xcd_block(bx, slot);
   const uint32_t b = a.wl[slot];
@@ -328,17 +422,19 @@ __global__ __launch_bounds__(512) void k_overlap(const OverlapArgs a) {
   const int32_t lo = O[(uint32_t)max(c0 - BS + 1, 0) >> a.shift];
   const int32_t hi = O[(min((uint32_t)c0 + cols - 1, a.n1 - 1) >> a.shift) + 1];
   // quantum and bound (see above)
-  const uint32_t* fig = a.wstat + b * (1 + a.nw);
-  const float smax = __uint_as_float(fig[0]);
-  const uint32_t wmax = fig[1 + k];
+  const uint32_t* fig = a.wstat + b * (2 + a.nw);
+  const float smax = __uint_as_float(fig[0]), smin = __uint_as_float(~fig[1]);  // (NaN: no s_0 above 0)
+  const uint32_t wmax = fig[2 + k];
   const int e = (smax > 0.f ? ilogbf(smax) : 0) + LOGC;
   const int head = max(0, (int)(32 - __clz((int)wmax | 1)) - 11);
   const double quantum = ldexp(1.0, e - 51 + head), magic = 1.5 * ldexp(1.0, e + 1 + head);
-  const float bound = ldexpf(1.f, min(e, 127));
+  const uint32_t bound = __float_as_uint(ldexpf(1.f, min(e, 127)));
+  const float dim = ldexpf(1.f, min(e - 27 + head, 127));
+  const uint32_t least = smin < dim ? min(__float_as_uint(dim), bound) : 0u, span = bound - least;
   const uint32_t mhi = (uint32_t)(__double_as_longlong(magic) >> 32);
   const uint32_t cells = st.tc * st.ld;
-  for (uint32_t c = threadIdx.x; c < cells + (cells / 32 + 2) / 2; c += blockDim.x) acc[c] = 0ull;
-  if (threadIdx.x == 0) flagged = 0;
+  for (uint32_t c = threadIdx.x; c < cells; c += blockDim.x) acc[c] = 0ull;
+  if (threadIdx.x == 0) beyond = 0;
   __syncthreads();
 
   const int2* R = a.recs + tab * a.p_sel;
@@ -413,12 +509,8 @@ __global__ __launch_bounds__(512) void k_overlap(const OverlapArgs a) {
       float mag = fabsf(x[u][0]);
 #pragma unroll
       for (int q = 1; q < BS; ++q) mag += fabsf(x[u][q]);
-      if (!(mag < bound)) {
-        flagged = 1;
-        for (int q = 0; q < BS; ++q) {
-          const uint32_t at = cell[u] + q;
-          if (!CUT || (uint32_t)(row[u] + q) < rows) atomicOr(&bad[at / 32], 1u << (at % 32));
-        }
+      if (__float_as_uint(mag) - least >= span) {  // (NaN and infinity among them)
+        if (mag != 0.f) beyond = 1;
         continue;
       }
 #pragma unroll
@@ -444,7 +536,23 @@ __global__ __launch_bounds__(512) void k_overlap(const OverlapArgs a) {
   const double umax = a.meta[b].uMax;
   const size_t oslice = (size_t)a.meta[b].out * n * n;
   const size_t base = tab * n * n + (size_t)r0 + (size_t)n * c0;
-  const bool some_bad = flagged != 0;
+  const bool wide = beyond != 0;
+  if (__builtin_expect(wide, 0))
+    sum_by_magnitude<BS, CUT>(acc, st, rows, cols, head, [&](auto f) {
+      for (int32_t j = lo + grp; j < hi; j += G) {
+        const int2 r = R[j];
+        int col, row;
+        if (!place(j, r, col, row)) continue;
+        const uint32_t id = (uint32_t)r.y;
+        const float d = D[id], v0 = V[id];
+        if (d == 0.f) continue;
+        float x[BS];
+        load_run<BS>((d < 0.f ? S + (size_t)id * M : W + (size_t)id * wst) + cb * BS, x);
+        if (d > 0.f)
+          for (int q = 0; q < BS; ++q) x[q] = lead_product<(BS <= 4)>(d, x[q], v0);
+        f(x, (uint32_t)col * st.ld + (uint32_t)row, row);
+      }
+    });
   // cell of the strip's v-th voxel: column v / rows
   const uint32_t inv = (uint32_t)(((1ull << 32) + rows - 1) / rows);
   double s_q = 0, s_h = 0, s_hu = 0, s_u = 0, s_u2 = 0;
@@ -452,26 +560,7 @@ __global__ __launch_bounds__(512) void k_overlap(const OverlapArgs a) {
     const uint32_t c = CUT ? v / rows : __umulhi(v, inv), r = v - c * rows;  // exact: rows * cols < 2^16
     const size_t at = base + (CUT ? r + (size_t)n * c : v);
     const uint32_t cell = c * st.ld + r;
-    double sum = (double)(long long)acc[cell] * quantum;
-    if (some_bad && ((bad[cell / 32] >> (cell % 32)) & 1u)) {
-      sum = 0.0;
-      for (int32_t j = lo; j < hi; ++j) {
-        const int pr = R[j].x & 0xffff, pc = (R[j].x >> 16) & 0xffff;
-        const int q = r0 + (int)r - pr, col = c0 + (int)c - pc;
-        if (q < 0 || q >= BS || col < 0 || col >= BS) continue;
-        const uint32_t id = (uint32_t)R[j].y;
-        const float dd = D[id];
-        if (dd == 0.f) continue;
-        float x[BS];
-        load_run<BS>((dd < 0.f ? S + (size_t)id * M : W + (size_t)id * wst) + col * BS, x);
-        if (dd > 0.f)
-          for (int z = 0; z < BS; ++z) x[z] = lead_product<(BS <= 4)>(dd, x[z], V[id]);
-        float xv = x[0];
-#pragma unroll
-        for (int z = 1; z < BS; ++z) xv = q == z ? x[z] : xv;
-        sum += (double)xv;
-      }
-    }
+    const double sum = wide ? __builtin_bit_cast(double, acc[cell]) : (double)(long long)acc[cell] * quantum;
     const double uh = sum * a.invw[at];
     if (a.mode == 0) {
       const double u = a.u64[at];
@@ -574,7 +663,8 @@ hipError_t launch_overlap(const OverlapSrc& src, const double* invw, const doubl
   a.mode = mode;
   a.st = st;
   const dim3 grid(overlap_blocks(sh, mode, nk), na);
-  const size_t cells = (size_t)st.tc * st.ld, lds = cells * 8 + ((cells / 32 + 2) / 2) * 8;
+  if (st.tr * st.tc > (uint32_t)kCellsPerThread * st.threads) return hipErrorInvalidValue;
+  const size_t lds = (size_t)st.tc * st.ld * 8;
 #define PG_OV(B)                                                                                   \
   case B:                                                                                          \
     if (st.nr > 1)                                                                                 \
