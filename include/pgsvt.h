@@ -95,7 +95,7 @@ int pgsvt_denoise_device(const void* X_dev, int dtype, uint32_t n_rows,
 /* pgsvt_denoise_device that allocates no device memory.  No reference
  * counterpart: it is for callers that cannot allocate (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  Windows
- * are processed one at a time in a statically sized device array of 66 MiB
+ * are processed one at a time in a statically sized device array of 78 MiB
  * that each device the library runs on holds until the process ends; a
  * shape whose window needs more returns PGSVT_E_ARG with the size in the
  * message (64 x 64 frames fit with PGURE, 128 x 128 with a fixed lambda at
@@ -109,6 +109,14 @@ int pgsvt_denoise_device_noalloc(const void* X_dev, int dtype, uint32_t n_rows,
                                  uint32_t n_cols, uint32_t n_frames,
                                  const pgsvt_params* p, double* Y_dev,
                                  double* estimates, void* stream);
+
+/* Device scratch of such a call, worked out without a device: *stated is the
+ * size that the limit of 64 MiB per window is stated for, *held what the
+ * call's buffers take of the array.  Returns what the call would for this
+ * shape: 0, or PGSVT_E_ARG with its message. */
+int pgsvt_noalloc_scratch(uint32_t n_rows, uint32_t n_cols,
+                          uint32_t n_frames, const pgsvt_params* p,
+                          uint64_t* stated, uint64_t* held);
 
 /* pgsvt_denoise restricted to output frames t_begin .. t_end-1 (the windows
  * of those frames read the input frames they need from the whole cube).  Y

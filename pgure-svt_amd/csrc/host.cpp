@@ -2233,8 +2233,10 @@ int guarded(F f) {
 // order of every sum are those of pgsvt_denoise_device, so the results are
 // the same bit for bit.
 // The array is larger than the size that bounds the shapes, for layouts that
-// need a little more than the one the bound is stated for.
-constexpr size_t kNoAllocScratch = 64ull << 20, kNoAllocArray = 66ull << 20;
+// need more than the one the bound is stated for: 76.8 MiB at most, for windows
+// of one frame (4 x 4 patches, step 1, fixed lambda, 514 x 514), whose w_0
+// planes weigh as much as their rows.
+constexpr size_t kNoAllocScratch = 64ull << 20, kNoAllocArray = 78ull << 20;
 static __device__ __align__(256) unsigned char scratch[kNoAllocArray];
 
 std::mutex g_scratch_mu;
@@ -2277,16 +2279,9 @@ double window_risk_of(const double* S, double alpha, double mu, double sigma, co
          sigmasq;
 }
 
-int run_noalloc(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf, const pgsvt_params* pp, double* Y,
-                double* est, hipStream_t s) {
-  if (int rc = validate(X, dtype, nr, nc, nf, pp)) return rc;
-  if (!Y || !est) return fail(PGSVT_E_ARG, "null output pointer");
-  if (g_precision.load() != 32) return fail(PGSVT_E_ARG, "the entry point without allocation runs in FP32 only");
-  if (int rc = check_device()) return rc;
-  const pgsvt_params p = *pp;
+// shape of a call and its patch selection
+Shape noalloc_shape(uint32_t nr, uint32_t nc, const pgsvt_params& p, std::vector<uint32_t>& sel) {
   const Geometry g = geometry(p);
-  const bool optimize = p.optimize_pgure != 0, median = p.motion_filter > 0;
-  const uint32_t nvar = optimize ? 3 : 1;
   Shape sh;
   sh.nr = nr;
   sh.nc = nc;
@@ -2297,81 +2292,113 @@ int run_noalloc(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf,
   sh.m = sh.bs * sh.bs;
   sh.n1 = nr - sh.bs + 1;
   sh.p_all = sh.n1 * sh.n1;
-  const std::vector<uint32_t> sel = patch_indices(nr, sh.bs, p.patch_overlap);
+  sel = patch_indices(nr, sh.bs, p.patch_overlap);
   sh.p_sel = (uint32_t)sel.size();
-  const uint32_t sr = (g.Nw + 3) & ~3u;
   sh.fstride = factor_stride(g.Nw, sh.m);
-  const size_t npos = (size_t)sh.n1 * sh.n1, vol = sh.vol;
-  const uint32_t max_jobs = 2 * g.Nw, eblk = eval_blocks(sh, 3);
-  const uint32_t gblk = overlap_blocks(sh, 0);
-  const double vP = 0.5 + 0.5 * 1. / std::sqrt(1. * 1. + 4), vQ = 1 - vP;
-  const double d2neg = -1 * std::sqrt(vQ / vP), d2pos = std::sqrt(vP / vQ), eps2 = 1e-2;
-  // the layout: per call, then the window being processed
-  struct Layout {
-    uint8_t* d2;
-    uint32_t *sel, *wl, *stats;
-    double *fmax, *sums, *Xw, *Zw, *u64, *w64, *invw, *partial, *partial_b;
-    WinMeta* meta;
-    int16_t* jobs;
-    float *uvar, *dw, *B0, *dr, *factors, *divq, *w0, *v0;
-    int32_t *pos, *off;
-    int2* recs;
-    uint32_t* wstat;
-  } L{};
+  return sh;
+}
+
+// the layout: per call, then the window being processed
+struct NoAllocLayout {
+  uint8_t* d2;
+  uint32_t *sel, *wl, *stats;
+  double *fmax, *sums, *Xw, *Zw, *u64, *w64, *invw, *partial, *partial_b;
+  WinMeta* meta;
+  int16_t* jobs;
+  float *uvar, *dw, *B0, *dr, *factors, *divq, *w0, *v0;
+  int32_t *pos, *off;
+  int2* recs;
+  uint32_t* wstat;
   // stated: the layout with position buckets, by whose size the shapes this
   // entry point takes are stated: a shape is neither refused nor taken anew
   // when the layout changes
-  auto carve = [&](Carve& c, bool stated) {
-    L.d2 = optimize ? c.take<uint8_t>(vol) : nullptr;
-    L.sel = c.take<uint32_t>(sh.p_sel);
-    L.wl = c.take<uint32_t>(1);
-    L.stats = c.take<uint32_t>(1);
-    L.fmax = c.take<double>(2 * g.Nw);
-    L.sums = c.take<double>(6);
-    L.meta = c.take<WinMeta>(1);
-    L.jobs = c.take<int16_t>((size_t)max_jobs * 4);
-    L.Xw = c.take<double>(vol);
-    L.Zw = median ? c.take<double>(vol) : nullptr;
-    L.u64 = c.take<double>(vol);
-    L.w64 = median ? c.take<double>(vol) : nullptr;
-    L.uvar = c.take<float>((size_t)nvar * vol);
-    L.pos = c.take<int32_t>((size_t)g.Nw * sh.p_all);
+  void carve(Carve& c, const Shape& sh, const pgsvt_params& p, bool stated) {
+    const bool optimize = p.optimize_pgure != 0, median = p.motion_filter > 0;
+    const uint32_t nvar = optimize ? 3 : 1, sr = (sh.nw + 3) & ~3u;
+    const size_t npos = (size_t)sh.n1 * sh.n1, vol = sh.vol;
+    d2 = optimize ? c.take<uint8_t>(vol) : nullptr;
+    sel = c.take<uint32_t>(sh.p_sel);
+    wl = c.take<uint32_t>(1);
+    stats = c.take<uint32_t>(1);
+    fmax = c.take<double>(2 * sh.nw);
+    sums = c.take<double>(6);
+    meta = c.take<WinMeta>(1);
+    jobs = c.take<int16_t>((size_t)kJobs * sh.nw * 4);
+    Xw = c.take<double>(vol);
+    Zw = median ? c.take<double>(vol) : nullptr;
+    u64 = c.take<double>(vol);
+    w64 = median ? c.take<double>(vol) : nullptr;
+    uvar = c.take<float>((size_t)nvar * vol);
+    pos = c.take<int32_t>((size_t)sh.nw * sh.p_all);
     if (!stated) {
-      L.off = c.take<int32_t>((size_t)g.Nw * (column_bins(sh) + 1));
-      L.recs = c.take<int2>((size_t)g.Nw * sh.p_sel);
-      if (fused_eval(sh)) L.w0 = c.take<float>((size_t)sh.p_sel * sh.m);
-      L.v0 = c.take<float>((size_t)g.Nw * sh.p_sel);
-      L.wstat = c.take<uint32_t>(2 + g.Nw);
+      off = c.take<int32_t>((size_t)sh.nw * (column_bins(sh) + 1));
+      recs = c.take<int2>((size_t)sh.nw * sh.p_sel);
+      w0 = fused_eval(sh) ? c.take<float>((size_t)sh.p_sel * sh.m) : nullptr;
+      v0 = c.take<float>((size_t)sh.nw * sh.p_sel);
+      wstat = c.take<uint32_t>(2 + sh.nw);
     } else {
-      c.take<int32_t>((size_t)g.Nw * npos);
-      c.take<int32_t>((size_t)g.Nw * (npos + 1));
-      c.take<int32_t>((size_t)g.Nw * sh.p_sel);
-      c.take<int32_t>((size_t)g.Nw * sh.p_sel);
+      c.take<int32_t>((size_t)sh.nw * npos);
+      c.take<int32_t>((size_t)sh.nw * (npos + 1));
+      c.take<int32_t>((size_t)sh.nw * sh.p_sel);
+      c.take<int32_t>((size_t)sh.nw * sh.p_sel);
     }
-    L.invw = c.take<double>(vol);
-    L.dw = optimize ? c.take<float>(vol) : nullptr;
-    if (!fused_eval(sh) || !stated) L.B0 = c.take<float>((size_t)g.Nw * sh.p_sel * sh.m);
-    if (fused_eval(sh) || !stated) L.dr = c.take<float>((size_t)g.Nw * sh.p_sel);
+    invw = c.take<double>(vol);
+    dw = optimize ? c.take<float>(vol) : nullptr;
+    if (!fused_eval(sh) || !stated) B0 = c.take<float>((size_t)sh.nw * sh.p_sel * sh.m);
+    if (fused_eval(sh) || !stated) dr = c.take<float>((size_t)sh.nw * sh.p_sel);
     if (fused_eval(sh) && stated) {
       c.take<char>(singular_pair_bytes(sh));
-      c.take<float>((size_t)g.Nw * sh.p_sel * sh.m);
+      c.take<float>((size_t)sh.nw * sh.p_sel * sh.m);
     }
-    L.factors = c.take<float>((size_t)nvar * sh.p_sel * sh.fstride);
-    L.divq = optimize ? c.take<float>((size_t)nvar * sh.p_sel * 2 * sr) : nullptr;
-    L.partial = c.take<double>(!stated ? eblk : fused_eval(sh) ? (sh.p_sel + 255) / 256 : (sh.p_sel + 3) / 4);
-    L.partial_b = c.take<double>((size_t)(!stated ? gblk : pgsvt::gather_blocks(sh, 0)) * 5);
-  };
+    factors = c.take<float>((size_t)nvar * sh.p_sel * sh.fstride);
+    divq = optimize ? c.take<float>((size_t)nvar * sh.p_sel * 2 * sr) : nullptr;
+    partial = c.take<double>(!stated          ? eval_blocks(sh, 3)
+                             : fused_eval(sh) ? (sh.p_sel + 255) / 256
+                                              : (sh.p_sel + 3) / 4);
+    partial_b = c.take<double>((size_t)(!stated ? overlap_blocks(sh, 0) : pgsvt::gather_blocks(sh, 0)) * 5);
+  }
+  static constexpr uint32_t kJobs = 2;  // motion search passes per frame of the window
+};
+
+// sizes of both layouts, and whether the call fits
+int noalloc_sizes(const Shape& sh, const pgsvt_params& p, size_t& stated, size_t& held) {
+  NoAllocLayout l{};
   Carve count, real;
-  carve(count, true);
-  carve(real, false);
-  if (count.used > kNoAllocScratch)
-    return fail(PGSVT_E_ARG, "this shape needs " + std::to_string(count.used) + " bytes of device scratch per window; "
+  l.carve(count, sh, p, true);
+  l.carve(real, sh, p, false);
+  stated = count.used;
+  held = real.used;
+  if (stated > kNoAllocScratch)
+    return fail(PGSVT_E_ARG, "this shape needs " + std::to_string(stated) + " bytes of device scratch per window; "
                              "the entry point without allocation has " + std::to_string(kNoAllocScratch));
-  if (real.used > kNoAllocArray) return fail(PGSVT_E_ARG, "the scratch array is too small for this shape's layout");
+  if (held > kNoAllocArray) return fail(PGSVT_E_ARG, "the scratch array is too small for this shape's layout");
+  return 0;
+}
+
+int run_noalloc(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf, const pgsvt_params* pp, double* Y,
+                double* est, hipStream_t s) {
+  if (int rc = validate(X, dtype, nr, nc, nf, pp)) return rc;
+  if (!Y || !est) return fail(PGSVT_E_ARG, "null output pointer");
+  if (g_precision.load() != 32) return fail(PGSVT_E_ARG, "the entry point without allocation runs in FP32 only");
+  if (int rc = check_device()) return rc;
+  const pgsvt_params p = *pp;
+  const Geometry g = geometry(p);
+  const bool optimize = p.optimize_pgure != 0, median = p.motion_filter > 0;
+  const uint32_t nvar = optimize ? 3 : 1;
+  std::vector<uint32_t> sel;
+  const Shape sh = noalloc_shape(nr, nc, p, sel);
+  const size_t vol = sh.vol;
+  const uint32_t max_jobs = NoAllocLayout::kJobs * g.Nw, eblk = eval_blocks(sh, 3);
+  const uint32_t gblk = overlap_blocks(sh, 0);
+  const double vP = 0.5 + 0.5 * 1. / std::sqrt(1. * 1. + 4), vQ = 1 - vP;
+  const double d2neg = -1 * std::sqrt(vQ / vP), d2pos = std::sqrt(vP / vQ), eps2 = 1e-2;
+  size_t stated = 0, held = 0;
+  if (int rc = noalloc_sizes(sh, p, stated, held)) return rc;
+  NoAllocLayout L{};
   std::lock_guard<std::mutex> lock(g_scratch_mu);
   Carve at;
   at.base = scratch_address();
-  carve(at, false);
+  L.carve(at, sh, p, false);
 
   const size_t dsz = dtype_size(dtype);
   const uint64_t seed = seed_of(p);
@@ -2840,6 +2867,21 @@ int pgsvt_noise_estimate(const double* u, uint32_t n_rows, uint32_t n_cols, uint
   return guarded([&] {
     estimate_noise(u, n_rows, n_t, method, *alpha, *mu, *sigma);
     return 0;
+  });
+}
+
+int pgsvt_noalloc_scratch(uint32_t n_rows, uint32_t n_cols, uint32_t n_frames, const pgsvt_params* p, uint64_t* stated,
+                          uint64_t* held) {
+  if (!stated || !held) return fail(PGSVT_E_ARG, "null pointer");
+  *stated = *held = 0;
+  if (int rc = validate(p, PGSVT_U8, n_rows, n_cols, n_frames, p)) return rc;
+  return guarded([&] {
+    std::vector<uint32_t> sel;
+    size_t a = 0, b = 0;
+    const int rc = noalloc_sizes(noalloc_shape(n_rows, n_cols, *p, sel), *p, a, b);
+    *stated = a;
+    *held = b;
+    return rc;
   });
 }
 
