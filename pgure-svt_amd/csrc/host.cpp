@@ -86,11 +86,12 @@ struct HipError {
 // the N-th device buffer request of a call fail as out of memory (whether
 // the cache or hipMalloc would serve it), "hip:N" the
 // N-th checked HIP call (launch, copy, synchronisation) fail as a launch
-// failure, after the real call succeeded.  Read at the start of every
+// failure, after the real call succeeded, "leaf:N" the N-th buffer request of
+// the thread that forms the noise estimator's leaf statistics.  Read at the start of every
 // denoise call (fault_arm) and counted per calling thread; the failure
 // unwinds like a real one.
 struct FaultPlan {
-  int kind = 0;  // 0 none, 1 allocation, 2 HIP call
+  int kind = 0;  // 0 none, 1 allocation, 2 HIP call, 3 allocation of the leaf statistics' thread
   long left = 0;
 };
 thread_local FaultPlan g_fault;
@@ -104,7 +105,7 @@ void fault_arm() {
   if (c == std::string::npos) return;
   const std::string kind = v.substr(0, c);
   g_fault.left = std::atol(v.c_str() + c + 1);
-  g_fault.kind = kind == "alloc" ? 1 : kind == "hip" ? 2 : 0;
+  g_fault.kind = kind == "alloc" ? 1 : kind == "hip" ? 2 : kind == "leaf" ? 3 : 0;
 }
 
 bool fault_hit(int kind) {
@@ -1841,6 +1842,15 @@ int run_core(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf, co
     const bool leaves_on_gpu =
         want_leaves && nr >= 16 && (learned || leaves_on_gpu_pay((uint64_t)leaf_jobs.size() * P.sh.fs, thread_count(p.n_jobs),
                                                   (double)count * P.nvar * P.sh.p_sel, P.sh));
+    auto host_leaves = [&P, nr](LeafJob& J) {
+      try {
+        std::vector<double> buf((size_t)nr * nr);
+        P.host_frame(J.frame, J.scale, buf.data());
+        J.pr.set_value(std::make_shared<const FrameLeaves>(frame_leaves(buf.data(), nr)));
+      } catch (...) {
+        J.pr.set_exception(std::current_exception());
+      }
+    };
     std::vector<std::function<void(PrepPool&)>> jobs;
     uint32_t made = 0;  // leaf jobs in the list (host)
     for (uint32_t t = rs.tb; t < rs.te; ++t) {
@@ -1850,15 +1860,7 @@ int run_core(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf, co
         if (leaves_on_gpu || id < made) continue;
         LeafJob* J = leaf_jobs[id].get();
         made = id + 1;
-        jobs.push_back([J, &P, nr](PrepPool&) {
-          try {
-            std::vector<double> buf((size_t)nr * nr);
-            P.host_frame(J->frame, J->scale, buf.data());
-            J->pr.set_value(std::make_shared<const FrameLeaves>(frame_leaves(buf.data(), nr)));
-          } catch (...) {
-            J->pr.set_exception(std::current_exception());
-          }
-        });
+        jobs.push_back([J, host_leaves](PrepPool&) { host_leaves(*J); });
       }
       const double ratio = gmax / m.uMax;
       jobs.push_back([t, need, ratio, learned, want_leaves, &leaf_jobs, &P, &p, &rs, g, nr, nc, lambda0, alpha0, mu0,
@@ -1908,7 +1910,11 @@ int run_core(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf, co
       const double* Xd = P.Xd.p;
       auto queued = std::make_shared<OnceFlag>();
       if (learned) P.leaves_queued = queued->future;
-      leaf_thread = std::thread([&leaf_jobs, frames, scales, dev, nr, learned, Xd, queued]() {
+      const FaultPlan fault = g_fault;
+      const uint32_t threads = thread_count(p.n_jobs);
+      leaf_thread = std::thread([&leaf_jobs, frames, scales, dev, nr, learned, Xd, queued, host_leaves, fault,
+                                 threads]() {
+        if (fault.kind == 3) g_fault = FaultPlan{1, fault.left};
         size_t done = 0;
         try {
           hipchk(hipSetDevice(dev), "hipSetDevice");
@@ -1921,6 +1927,22 @@ int run_core(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf, co
                 done = i + 1;
               },
               queued.get());
+        } catch (const HipError& e) {
+          if (learned || e.e != hipErrorOutOfMemory) {
+            for (; done < leaf_jobs.size(); ++done) leaf_jobs[done]->pr.set_exception(std::current_exception());
+          } else {
+            // no memory beside the batch (up to 0.6 GB of scratch): the host's
+            // are the same
+            (void)hipGetLastError();
+            std::atomic<size_t> next{done};
+            std::vector<std::thread> th;
+            for (uint32_t k = 0; k < threads; ++k)
+              th.emplace_back([&] {
+                for (size_t j; (j = next.fetch_add(1)) < leaf_jobs.size();) host_leaves(*leaf_jobs[j]);
+              });
+            for (auto& x : th) x.join();
+          }
+          queued->set();
         } catch (...) {
           for (; done < leaf_jobs.size(); ++done) leaf_jobs[done]->pr.set_exception(std::current_exception());
           queued->set();
