@@ -46,9 +46,8 @@ Strips strips_of(uint32_t n, uint32_t bs) {
   s.nc = (n + s.tc - 1) / s.tc;
   return s;
 }
-// cells of a strip a thread holds at most (sum_by_magnitude): 4,096 over 256
-// threads, 7,600 over 512
-constexpr int kCellsPerThread = 16;
+// cells a thread holds at a time where a strip is summed by magnitude
+constexpr int kCellsHeld = 8;
 // strips of the cover counts: their two LDS arrays stay within 60 KB
 Strips cover_strips(uint32_t n, uint32_t bs) {
   Strips s{};
@@ -289,74 +288,84 @@ __device__ __forceinline__ void load_run(const float* __restrict__ p, float (&x)
 // column is held to 2^-25 of its own |x|, in any order, and a strip costs a few
 // walks (256 x 256 x 3, half of it 1e-20 of the rest, plain threshold 0: 0.16 ms
 // a lambda, 0.05 where no strip comes here; a walk of the strip's records for
-// each cell that is not finite 6.4).  The cells' places are worked out anew at
-// each use: 16 addresses held through the walks would cost the whole kernel
-// two of its six waves per SIMD.
+// each cell that is not finite 6.4).  The sums between the classes stay in
+// registers, kCellsHeld a thread, so a strip of more cells takes its parts one
+// after the other; and the cells' places are worked out anew at each use:
+// registers held here cost the whole kernel waves (16 sums a thread and their
+// addresses: four waves per SIMD for 4 x 4, 16 sums alone six for 8 x 8
+// against seven).
 template <int BS, bool CUT, class Each>
 __device__ __forceinline__ void sum_by_magnitude(unsigned long long* acc, const Strips& st, uint32_t rows,
                                                  uint32_t cols, int head, Each each) {
   __shared__ unsigned long long top;  // the largest column left (bits of a non-negative double)
-  double run[kCellsPerThread];
-  auto own = [&](auto f) {
-    uint32_t t = threadIdx.x;
-    asm volatile("" : "+v"(t));
+  const uint32_t part = (uint32_t)kCellsHeld * blockDim.x;
+#pragma unroll 1
+  for (uint32_t v0 = 0; v0 < rows * cols; v0 += part) {
+    double run[kCellsHeld];
+    // the part's cells: count of acc from first
+    const uint32_t first = v0 / rows * st.ld + v0 % rows;
+    const uint32_t v1 = v0 + part, count = (v1 < rows * cols ? v1 / rows * st.ld + v1 % rows : cols * st.ld) - first;
+    auto own = [&](auto f) {
+      uint32_t t = v0 + threadIdx.x;
+      asm volatile("" : "+v"(t));
 #pragma unroll
-    for (int i = 0; i < kCellsPerThread; ++i) {
-      const uint32_t v = t + (uint32_t)i * blockDim.x;
-      if (v < rows * cols) f(i, acc[v / rows * st.ld + v % rows]);
-    }
-  };
-  auto clear = [&] {
-    for (uint32_t c = threadIdx.x; c < st.tc * st.ld; c += blockDim.x) acc[c] = 0ull;
-    if (threadIdx.x == 0) top = 0ull;
-    __syncthreads();
-  };
-  auto inside = [&](int row) { return !CUT || (uint32_t)row < rows; };
-  auto magnitude = [](const float(&x)[BS]) {
-    double m = 0.0;
-    for (int q = 0; q < BS; ++q) m += __builtin_isfinite(x[q]) ? fabs((double)x[q]) : 0.0;
-    return m;
-  };
-  double most = 0.0;
-  clear();
-  each([&](const float(&x)[BS], uint32_t cell, int row) {
-    most = fmax(most, magnitude(x));
-    for (int q = 0; q < BS; ++q)
-      if (!__builtin_isfinite(x[q]) && inside(row + q))
-        atomicOr(&acc[cell + q], x[q] != x[q] ? 1ull : x[q] > 0.f ? 2ull : 4ull);
-  });
-  atomicMax(&top, __builtin_bit_cast(unsigned long long, most));
-  __syncthreads();
-  own([&](int i, unsigned long long bits) {
-    run[i] = (bits & 1ull) || (bits & 6ull) == 6ull ? __builtin_nan("")
-             : bits & 2ull                          ? __builtin_inf()
-             : bits & 4ull                          ? -__builtin_inf()
-                                                    : 0.0;
-  });
-  for (;;) {
-    const double t = __builtin_bit_cast(double, top);
-    __syncthreads();
-    if (!(t > 0.0)) break;  // (each class starts below the one before: 48 at most)
-    clear();
-    const int e = ilogb(t) + 1;
-    const double quantum = ldexp(1.0, e - 51 + head), magic = 1.5 * ldexp(1.0, e + 1 + head);
-    const double high = ldexp(1.0, e), low = ldexp(1.0, e - 27 + head);
-    most = 0.0;
-    each([&](const float(&x)[BS], uint32_t cell, int row) {
-      const double m = magnitude(x);
-      if (m < low) most = fmax(most, m);
-      if (!(m >= low && m < high)) return;
-      for (int q = 0; q < BS; ++q) {
-        const unsigned long long y = __builtin_bit_cast(unsigned long long, (double)x[q] + magic) -
-                                     __builtin_bit_cast(unsigned long long, magic);
-        if (__builtin_isfinite(x[q]) && inside(row + q)) atomicAdd(&acc[cell + q], y);
+      for (int i = 0; i < kCellsHeld; ++i) {
+        const uint32_t v = t + (uint32_t)i * blockDim.x;
+        if (v < rows * cols) f(i, acc[v / rows * st.ld + v % rows]);
       }
+    };
+    auto clear = [&] {
+      for (uint32_t c = threadIdx.x; c < count; c += blockDim.x) acc[first + c] = 0ull;
+      if (threadIdx.x == 0) top = 0ull;
+      __syncthreads();
+    };
+    auto inside = [&](uint32_t cell, int row) { return (!CUT || (uint32_t)row < rows) && cell - first < count; };
+    auto magnitude = [](const float(&x)[BS]) {
+      double m = 0.0;
+      for (int q = 0; q < BS; ++q) m += __builtin_isfinite(x[q]) ? fabs((double)x[q]) : 0.0;
+      return m;
+    };
+    double most = 0.0;
+    clear();
+    each([&](const float(&x)[BS], uint32_t cell, int row) {
+      most = fmax(most, magnitude(x));
+      for (int q = 0; q < BS; ++q)
+        if (!__builtin_isfinite(x[q]) && inside(cell + q, row + q))
+          atomicOr(&acc[cell + q], x[q] != x[q] ? 1ull : x[q] > 0.f ? 2ull : 4ull);
     });
     atomicMax(&top, __builtin_bit_cast(unsigned long long, most));
     __syncthreads();
-    own([&](int i, unsigned long long bits) { run[i] += (double)(long long)bits * quantum; });
+    own([&](int i, unsigned long long bits) {
+      run[i] = (bits & 1ull) || (bits & 6ull) == 6ull ? __builtin_nan("")
+               : bits & 2ull                          ? __builtin_inf()
+               : bits & 4ull                          ? -__builtin_inf()
+                                                      : 0.0;
+    });
+    for (;;) {
+      const double t = __builtin_bit_cast(double, top);
+      __syncthreads();
+      if (!(t > 0.0)) break;  // (each class starts below the one before: 48 at most)
+      clear();
+      const int e = ilogb(t) + 1;
+      const double quantum = ldexp(1.0, e - 51 + head), magic = 1.5 * ldexp(1.0, e + 1 + head);
+      const double high = ldexp(1.0, e), low = ldexp(1.0, e - 27 + head);
+      most = 0.0;
+      each([&](const float(&x)[BS], uint32_t cell, int row) {
+        const double m = magnitude(x);
+        if (m < low) most = fmax(most, m);
+        if (!(m >= low && m < high)) return;
+        for (int q = 0; q < BS; ++q) {
+          const unsigned long long y = __builtin_bit_cast(unsigned long long, (double)x[q] + magic) -
+                                       __builtin_bit_cast(unsigned long long, magic);
+          if (__builtin_isfinite(x[q]) && inside(cell + q, row + q)) atomicAdd(&acc[cell + q], y);
+        }
+      });
+      atomicMax(&top, __builtin_bit_cast(unsigned long long, most));
+      __syncthreads();
+      own([&](int i, unsigned long long bits) { run[i] += (double)(long long)bits * quantum; });
+    }
+    own([&](int i, unsigned long long& cell) { cell = __builtin_bit_cast(unsigned long long, run[i]); });
   }
-  own([&](int i, unsigned long long& cell) { cell = __builtin_bit_cast(unsigned long long, run[i]); });
 }
 
 // Uhat = (sum of the patches' rows over each voxel) / W.  The row of patch p
@@ -663,7 +672,6 @@ hipError_t launch_overlap(const OverlapSrc& src, const double* invw, const doubl
   a.mode = mode;
   a.st = st;
   const dim3 grid(overlap_blocks(sh, mode, nk), na);
-  if (st.tr * st.tc > (uint32_t)kCellsPerThread * st.threads) return hipErrorInvalidValue;
   const size_t lds = (size_t)st.tc * st.ld * 8;
 #define PG_OV(B)                                                                                   \
   case B:                                                                                          \
