@@ -1401,7 +1401,8 @@ struct OnceFlag {
 // (k_split_stats; ordered: rounded as the host's), the reference's recursion
 // on the host with those decisions, then the statistics of each distinct
 // leaf (k_leaf_*), in the tree's order per item.  Items go in groups whose
-// normalised frames take up to kLeafScratch values.  Frames of at least 16 x
+// normalised frames take up to kLeafScratch values and whose launches stay
+// within a grid's 65,536 rows.  Frames of at least 16 x
 // 16 (smaller ones never split and stay on the host).  queued: set when the
 // first group's leaf kernels are on the stream.
 void gpu_frame_leaves(const double* Xd, uint32_t n, const std::vector<uint32_t>& frames,
@@ -1423,7 +1424,7 @@ void gpu_frame_leaves(const double* Xd, uint32_t n, const std::vector<uint32_t>&
   add(0, 0, n);
   const uint64_t fs = (uint64_t)n * n;
   const uint32_t total = (uint32_t)frames.size(), nc = (uint32_t)(cand.size() / 3);
-  const uint32_t group = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(kLeafScratch / fs, total));
+  const uint32_t group = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>({kLeafScratch / fs, total, 65535}));
   DBuf<uint32_t> frames_d, cand_d, leaves_d;
   DBuf<uint64_t> boff_d;
   DBuf<double> scales_d, Z, stat_d, out_d, laps_d;
