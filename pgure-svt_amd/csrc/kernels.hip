@@ -597,10 +597,11 @@ __device__ __forceinline__ T shrink_factor(T s, T s0, double lam, int exp_w) {
 // S01 [nb][nw][p_sel][2].  4 lanes per (patch, frame), frames fastest, so
 // a patch's 15 rows read its w_0 from one cache line and each row is one
 // line-sized store.
-template <int BS, class T>
-__global__ __launch_bounds__(256) void k_static_rows(const T* __restrict__ factors, const int32_t* __restrict__ place,
-                                                     uint32_t nvar_stored, uint32_t p_sel, uint32_t nw,
-                                                     uint32_t fstride, T* __restrict__ W0, T* __restrict__ S01) {
+template <int BS>
+__global__ __launch_bounds__(256) void k_static_rows(const double* __restrict__ factors,
+                                                     const int32_t* __restrict__ place, uint32_t nvar_stored,
+                                                     uint32_t p_sel, uint32_t nw, uint32_t fstride,
+                                                     double* __restrict__ W0, double* __restrict__ S01) {
   constexpr int M = BS * BS, QL = (M + 3) / 4;  // row elements per lane
   const uint32_t b = blockIdx.y;
   const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -608,28 +609,22 @@ __global__ __launch_bounds__(256) void k_static_rows(const T* __restrict__ facto
   const uint32_t p = row / nw, k = row % nw;
   if (p >= p_sel) return;
   const uint32_t SR = (nw + 3) & ~3u;
-  const T* F = factors + ((size_t)b * nvar_stored * p_sel + p) * fstride;  // the U variant
-  const T* FW = F + (size_t)nw * SR;
-  const T* FS = FW + (size_t)nw * M;
-  const T v0k = F[k];  // V^T row 0, element k
+  const double* F = factors + ((size_t)b * nvar_stored * p_sel + p) * fstride;  // the U variant
+  const double* FW = F + (size_t)nw * SR;
+  const double* FS = FW + (size_t)nw * M;
+  const double v0k = F[k];  // V^T row 0, element k
   const int32_t jk = place[((size_t)b * nw + k) * p_sel + p];
-  T* o = W0 + (((size_t)b * nw + k) * p_sel + jk) * M;
-  if constexpr (M == 16 && sizeof(T) == 4) {  // lane sub: elements 4 sub .. 4 sub + 3
-    const float4 w = *reinterpret_cast<const float4*>(FW + 4 * sub);
-    *reinterpret_cast<float4*>(o + 4 * sub) = make_float4(w.x * v0k, w.y * v0k, w.z * v0k, w.w * v0k);
-  } else {
+  double* o = W0 + (((size_t)b * nw + k) * p_sel + jk) * M;
 #pragma unroll
-    for (int i = 0; i < QL; ++i) {
-      const uint32_t q = sub + 4 * i;
-      if (q < (uint32_t)M) o[q] = FW[q] * v0k;
-    }
+  for (int i = 0; i < QL; ++i) {
+    const uint32_t q = sub + 4 * i;
+    if (q < (uint32_t)M) o[q] = FW[q] * v0k;
   }
   if (sub == 0) {
-    typedef typename std::conditional<sizeof(T) == 4, float2, double2>::type T2;
-    T2 sp;
+    double2 sp;
     sp.x = FS[0];
-    sp.y = nw > 1 ? FS[1] : T(0);
-    reinterpret_cast<T2*>(S01)[((size_t)b * nw + k) * p_sel + jk] = sp;
+    sp.y = nw > 1 ? FS[1] : 0.0;
+    reinterpret_cast<double2*>(S01)[((size_t)b * nw + k) * p_sel + jk] = sp;
   }
 }
 
@@ -789,13 +784,10 @@ hipError_t launch_buckets(const int32_t* pos, const uint32_t* sel, uint32_t nb, 
 
 // weights of src/svt.hpp:157-163: W = number of patches covering a voxel
 // (from the bucket sizes), stored as 1/W (FP64, 0 where nothing covers it)
-// and as delta2/W for the divergence sum, in the reconstruction's type
-// (FP32: half the bytes the evaluation reads; its rounding, 6e-8 of each
-// term, is far below that of the FP32 reconstructions it multiplies).
-template <class D>
+// and as delta2/W for the divergence sum.  FP64 (FP32: launch_cover).
 __global__ void k_weights(const int32_t* __restrict__ off, const uint8_t* __restrict__ d2, uint32_t nr, uint32_t fs,
                           uint32_t vol, uint32_t n1, uint32_t bs, double d2neg, double d2pos,
-                          double* __restrict__ invw, D* __restrict__ dw) {
+                          double* __restrict__ invw, double* __restrict__ dw) {
   const uint32_t b = blockIdx.y;
   const uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
   if (v >= vol) return;
@@ -815,18 +807,15 @@ __global__ void k_weights(const int32_t* __restrict__ off, const uint8_t* __rest
   }
   const double iw = w > 0 ? 1.0 / (double)w : 0.0;
   invw[(size_t)b * vol + v] = iw;
-  if (dw) dw[(size_t)b * vol + v] = (D)((d2[v] ? d2neg : d2pos) * iw);
+  if (dw) dw[(size_t)b * vol + v] = (d2[v] ? d2neg : d2pos) * iw;
 }
 
 hipError_t launch_weights(const int32_t* off, const uint8_t* d2, uint32_t nb, const Shape& sh, double d2neg,
                           double d2pos, double* invw, void* dw, hipStream_t s) {
   const dim3 grid((sh.vol + 255) / 256, nb);
-  if (sh.fp64)
-    hipLaunchKernelGGL(k_weights<double>, grid, dim3(256), 0, s, off, d2, sh.nr, sh.fs, sh.vol, sh.n1, sh.bs, d2neg,
-                       d2pos, invw, (double*)dw);
-  else
-    hipLaunchKernelGGL(k_weights<float>, grid, dim3(256), 0, s, off, d2, sh.nr, sh.fs, sh.vol, sh.n1, sh.bs, d2neg,
-                       d2pos, invw, (float*)dw);
+  if (!sh.fp64) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_weights, grid, dim3(256), 0, s, off, d2, sh.nr, sh.fs, sh.vol, sh.n1, sh.bs, d2neg, d2pos,
+                     invw, (double*)dw);
   return hipGetLastError();
 }
 
@@ -887,18 +876,15 @@ __device__ __forceinline__ void block_count(double* out, int v) {
 // delta2_v / W_v of src/pgure.hpp:136 comes from the divergence factors of
 // the variants U, U + eps2 delta2, U - eps2 delta2 (k_divq) as
 // sum_r (d1_r q1_r - 2 d0_r q0_r + d2_r q2_r), in FP64.
-// RT: window length n = nw at run time (n <= N).  Patches above 8 x 8 give
-// each lane several rows of B (lane q rows q, q + L, ...).
-template <int BS, int N, int L, class T, bool RT = false>
+template <int BS, int N, int L>
 __global__ __launch_bounds__(256) void k_eval(
-    const T* __restrict__ factors, const WinMeta* __restrict__ meta, const uint32_t* __restrict__ wl,
+    const double* __restrict__ factors, const WinMeta* __restrict__ meta, const uint32_t* __restrict__ wl,
     uint32_t nvar_stored, uint32_t nvar_run, uint32_t p_sel, uint32_t nw, uint32_t fstride, int exp_w,
-    const T* __restrict__ divq, const int32_t* __restrict__ inv, T* __restrict__ B0,
+    const double* __restrict__ divq, const int32_t* __restrict__ inv, double* __restrict__ B0,
     double* __restrict__ partial, const double* __restrict__ slot_lam, double* __restrict__ kept) {
-  constexpr int M = BS * BS, G = 256 / L, SRN = (N + 3) & ~3, RQ = (M + L - 1) / L;
+  constexpr int M = BS * BS, G = 256 / L, n = N, SR = (N + 3) & ~3;
+  static_assert(M <= L, "one lane per row of B");
   __shared__ double red[4];
-  const int n = RT ? (int)nw : N;
-  const int SR = RT ? ((n + 3) & ~3) : SRN;
   uint32_t bx, slot;
   xcd_block(bx, slot);
   const uint32_t b = wl[slot];
@@ -907,18 +893,18 @@ __global__ __launch_bounds__(256) void k_eval(
   const bool valid = p < p_sel;
   const uint32_t pa = valid ? p : 0;  // addresses of groups past the end: patch 0
   const double lam = slot_lam ? slot_lam[slot] : meta[b].lambda;
-  const T* F = factors + ((size_t)b * nvar_stored * p_sel + pa) * fstride;  // the U variant's factors
-  const T* FW = F + n * SR;
-  const T* FS = FW + n * M;
+  const double* F = factors + ((size_t)b * nvar_stored * p_sel + pa) * fstride;  // the U variant's factors
+  const double* FW = F + n * SR;
+  const double* FS = FW + n * M;
   const bool pgq = nvar_run == 3;
   // singular values (lane r: s_r) of U, and with PGURE those of the
   // perturbed variants and the divergence factors of all three
   const int lk = min(lane, n - 1);
-  const T sl = FS[lk], smax = FS[0];
-  T sp[2] = {T(0), T(0)}, spm[2] = {T(0), T(0)}, ql[3] = {T(0), T(0), T(0)};
+  const double sl = FS[lk], smax = FS[0];
+  double sp[2] = {0.0, 0.0}, spm[2] = {0.0, 0.0}, ql[3] = {0.0, 0.0, 0.0};
   if (pgq) {
     // the patch's record: per variant sr singular values, sr factors
-    const T* Q = divq + ((size_t)b * p_sel + pa) * nvar_stored * 2 * SR;
+    const double* Q = divq + ((size_t)b * p_sel + pa) * nvar_stored * 2 * SR;
 #pragma unroll
     for (int v = 0; v < 3; ++v) ql[v] = Q[v * 2 * SR + SR + lk];
 #pragma unroll
@@ -929,87 +915,58 @@ __global__ __launch_bounds__(256) void k_eval(
   }
   // shrink factor g(s_r)/s_r in lane r < N; kept ranks: 1 + highest lane
   // of the group with g > 0
-  auto shrink = [&](T s, T s0) {
-    T d = T(0);
+  auto shrink = [&](double s, double s0) {
+    double d = 0.0;
     if (valid && lane < n) d = shrink_factor(s, s0, lam, exp_w);
     return d;
   };
-  auto kept_ranks = [&](T d) {
-    const uint64_t bal = __ballot(d > T(0));
+  auto kept_ranks = [&](double d) {
+    const uint64_t bal = __ballot(d > 0.0);
     const uint32_t gbits =
         (uint32_t)((bal >> ((threadIdx.x % 64) / L * L)) & ((L >= 64) ? ~0ull : ((1ull << L) - 1)));
     return gbits ? 32 - __clz(gbits) : 0;
   };
-  const T dl = shrink(sl, smax);
+  const double dl = shrink(sl, smax);
   const int nkeep = kept_ranks(dl);
   double s4 = 0.0;
   int kr = nkeep;  // kept ranks of the evaluated variants (profiling)
   if (pgq) {
     // lanes past the kept ranks have d_r = 0
-    s4 = -2.0 * (double)dl * (double)ql[0];
+    s4 = -2.0 * dl * ql[0];
 #pragma unroll
     for (int v = 0; v < 2; ++v) {
-      const T d = shrink(sp[v], spm[v]);
+      const double d = shrink(sp[v], spm[v]);
       kr += kept_ranks(d);
-      s4 = fma((double)d, (double)ql[v + 1], s4);
+      s4 = fma(d, ql[v + 1], s4);
     }
   }
-  T bq[RQ][N];
+  double bq[N];
 #pragma unroll
-  for (int h = 0; h < RQ; ++h)
-#pragma unroll
-    for (int k = 0; k < N; ++k) bq[h][k] = T(0);
+  for (int k = 0; k < N; ++k) bq[k] = 0.0;
   // rank loop, loads of rank r + 1 issued before the products of rank r
-  // (FP32: the V^T row as SR/4 float4 loads; FP64: SR scalar loads; with a
-  // window length known at run time the loads cover SRN values, within the
-  // factor block, and the values past n are never stored)
-  constexpr int VW = (sizeof(T) == 4) ? 4 : 1, NV = SRN / VW;
-  typedef typename std::conditional<sizeof(T) == 4, float4, double>::type VT;
-  T wn[RQ];
-  VT vn[NV];
+  double wn, vn[SR];
   auto fetch = [&](int r) {
+    wn = (valid && lane < M) ? FW[r * M + lane] : 0.0;
 #pragma unroll
-    for (int h = 0; h < RQ; ++h) wn[h] = (valid && lane + L * h < M) ? FW[r * M + lane + L * h] : T(0);
-    const VT* vr = reinterpret_cast<const VT*>(F + r * SR);
-#pragma unroll
-    for (int j = 0; j < NV; ++j) vn[j] = vr[j];
+    for (int j = 0; j < SR; ++j) vn[j] = F[r * SR + j];
   };
   if (nkeep > 0) fetch(0);
   for (int r = 0; r < nkeep; ++r) {
-    const T dr = __shfl(dl, r, L);
-    T y[RQ];
+    const double y = __shfl(dl, r, L) * wn;
+    double vc[N];
 #pragma unroll
-    for (int h = 0; h < RQ; ++h) y[h] = dr * wn[h];
-    VT vc[NV];
-#pragma unroll
-    for (int j = 0; j < NV; ++j) vc[j] = vn[j];
+    for (int j = 0; j < N; ++j) vc[j] = vn[j];
     if (r + 1 < nkeep) fetch(r + 1);
 #pragma unroll
-    for (int h = 0; h < RQ; ++h) {
-#pragma unroll
-      for (int j = 0; j < NV; ++j) {
-        if constexpr (VW == 4) {
-          const float4 t = vc[j];
-          if (4 * j < N) bq[h][4 * j] = fma(y[h], t.x, bq[h][4 * j]);
-          if (4 * j + 1 < N) bq[h][4 * j + 1] = fma(y[h], t.y, bq[h][4 * j + 1]);
-          if (4 * j + 2 < N) bq[h][4 * j + 2] = fma(y[h], t.z, bq[h][4 * j + 2]);
-          if (4 * j + 3 < N) bq[h][4 * j + 3] = fma(y[h], t.w, bq[h][4 * j + 3]);
-        } else {
-          if (j < N) bq[h][j] = fma(y[h], (T)vc[j], bq[h][j]);
-        }
-      }
-    }
+    for (int j = 0; j < N; ++j) bq[j] = fma(y, vc[j], bq[j]);
   }
   if (valid) {
     const int32_t* I = inv + (size_t)b * nw * p_sel + p;
 #pragma unroll
     for (int k = 0; k < N; ++k) {
-      if (RT && k >= n) break;
       // row of patch p for frame k at its bucket-sorted place
       const size_t at = (((size_t)slot * nw + k) * p_sel + I[(size_t)k * p_sel]) * M;
-#pragma unroll
-      for (int h = 0; h < RQ; ++h)
-        if (lane + L * h < M) B0[at + lane + L * h] = bq[h][k];
+      if (lane < M) B0[at + lane] = bq[k];
     }
   }
   if (!pgq) return;  // uniform over the launch
@@ -1336,8 +1293,8 @@ __global__ __launch_bounds__(256) void k_rows(const float* __restrict__ factors,
 // One thread per voxel.  For each patch column cb the buckets of positions
 // (r-bs+1 .. r, c-cb) are one contiguous run of rows in bucket order, read
 // straight from memory (neighbouring voxels share them in cache).
-template <int BS, class T>
-__global__ __launch_bounds__(256) void k_gather_direct(const T* __restrict__ B0, const int32_t* __restrict__ off,
+template <int BS>
+__global__ __launch_bounds__(256) void k_gather_direct(const double* __restrict__ B0, const int32_t* __restrict__ off,
                                                        const double* __restrict__ invw,
                                                        const double* __restrict__ u64,
                                                        const WinMeta* __restrict__ meta,
@@ -1359,48 +1316,37 @@ __global__ __launch_bounds__(256) void k_gather_direct(const T* __restrict__ B0,
     const uint32_t k = v / fs, pix = v % fs;
     const int r = (int)(pix % nr), c = (int)(pix / nr);
     const int32_t* O = off + ((size_t)b * nw + k) * ((size_t)n1 * n1 + 1);
-    const T* Bk = B0 + ((size_t)slot * nw + k) * p_sel * M;
-    // Patch columns in chunks of CH (all at once for small patches): bucket
-    // bounds of positions (r - ra, c - cb), bnd[.][e] for rows r-BS+1+e
-    // (clamped to the frame), e = BS the end of row r; then the first
-    // contribution of every bucket in one batch of independent loads, and
-    // further ones (buckets holding several patches) in order.
-    constexpr int CH = (BS <= 5) ? BS : 1;
+    const double* Bk = B0 + ((size_t)slot * nw + k) * p_sel * M;
+    // Per patch column: bucket bounds of positions (r - ra, pc), bnd[e] for
+    // rows r-BS+1+e (clamped to the frame), e = BS the end of row r; then the
+    // first contribution of every bucket in one batch of independent loads,
+    // and further ones (buckets holding several patches) in order.
     double acc = 0.0;
 #pragma unroll
-    for (int cb0 = 0; cb0 < BS; cb0 += CH) {
-      int32_t bnd[CH][BS + 1];
+    for (int cb = 0; cb < BS; ++cb) {
+      const int pc = c - cb;
+      const bool in = pc >= 0 && pc < (int)n1;
+      const size_t colq = (size_t)n1 * (in ? pc : 0);
+      int32_t bnd[BS + 1];
 #pragma unroll
-      for (int h = 0; h < CH; ++h) {
-        const int pc = c - (cb0 + h);
-        const bool in = pc >= 0 && pc < (int)n1;
-        const size_t colq = (size_t)n1 * (in ? pc : 0);
+      for (int e = 0; e <= BS; ++e) {
+        const int prc = min(max(r - (BS - 1) + e, 0), (int)n1);
+        bnd[e] = in ? O[colq + prc] : 0;
+      }
+      double first[BS];
 #pragma unroll
-        for (int e = 0; e <= BS; ++e) {
-          const int prc = min(max(r - (BS - 1) + e, 0), (int)n1);
-          bnd[h][e] = in ? O[colq + prc] : 0;
+      for (int ra = 0; ra < BS; ++ra) {
+        const int e = BS - 1 - ra;  // position r - ra
+        first[ra] = (bnd[e] < bnd[e + 1]) ? Bk[(size_t)bnd[e] * M + ra + BS * cb] : 0.0;
+      }
+#pragma unroll
+      for (int ra = 0; ra < BS; ++ra) {
+        const int e = BS - 1 - ra;
+        if (bnd[e] < bnd[e + 1]) {
+          acc += first[ra];
+          for (int32_t j = bnd[e] + 1; j < bnd[e + 1]; ++j) acc += Bk[(size_t)j * M + ra + BS * cb];
         }
       }
-      T first[CH][BS];
-#pragma unroll
-      for (int h = 0; h < CH; ++h)
-#pragma unroll
-        for (int ra = 0; ra < BS; ++ra) {
-          const int e = BS - 1 - ra;  // position r - ra
-          const int32_t j = bnd[h][e];
-          first[h][ra] = (j < bnd[h][e + 1]) ? Bk[(size_t)j * M + ra + BS * (cb0 + h)] : T(0);
-        }
-#pragma unroll
-      for (int h = 0; h < CH; ++h)
-#pragma unroll
-        for (int ra = 0; ra < BS; ++ra) {
-          const int e = BS - 1 - ra;
-          const int32_t j0 = bnd[h][e], j1 = bnd[h][e + 1];
-          if (j0 < j1) {
-            acc += (double)first[h][ra];
-            for (int32_t j = j0 + 1; j < j1; ++j) acc += (double)Bk[(size_t)j * M + ra + BS * (cb0 + h)];
-          }
-        }
     }
     const double uh = acc * invw[(size_t)b * vol + v];
     if (mode == 0) {
@@ -1467,10 +1413,11 @@ __global__ __launch_bounds__(256) void k_gather_direct(const T* __restrict__ B0,
 constexpr int kTileRows = 32, kTileCols = 8;
 static_assert(kTileRows * kTileCols == 256, "one voxel per thread");
 
-template <int BS, class T>
+template <int BS>
 __global__ __launch_bounds__(256) void k_gather_tile(
-    const T* __restrict__ factors, const T* __restrict__ dr, const T* __restrict__ S01, const T* __restrict__ W0,
-    const int32_t* __restrict__ list, const int32_t* __restrict__ off, const double* __restrict__ invw,
+    const double* __restrict__ factors, const double* __restrict__ dr, const double* __restrict__ S01,
+    const double* __restrict__ W0, const int32_t* __restrict__ list, const int32_t* __restrict__ off,
+    const double* __restrict__ invw,
     const double* __restrict__ u64, const WinMeta* __restrict__ meta, const uint32_t* __restrict__ wl,
     const double* __restrict__ slot_lam, int exp_w, uint32_t nr, uint32_t fs, uint32_t nw, uint32_t vol, uint32_t n1,
     uint32_t p_sel, uint32_t fstride, uint32_t nvar_stored, int mode, uint32_t nk, double* __restrict__ out,
@@ -1479,8 +1426,6 @@ __global__ __launch_bounds__(256) void k_gather_tile(
   // columns packed one after another
   constexpr int M = BS * BS, TR = kTileRows, TC = kTileCols, NC = TC + BS - 1, NRW = TR + BS, TOT = 448;
   constexpr int RS = TOT + 1;                                // plane stride (odd: spreads the planes over banks)
-  constexpr int W = (sizeof(T) == 4 && M % 4 == 0) ? 4 : 1;  // row values per thread while staging
-  typedef typename std::conditional<W == 4, float4, T>::type ST;
   // sB: staged patch rows, one plane per patch row q (plane q, LDS row j);
   // the pad element of each plane is read (and ignored) by empty buckets.
   // sP: first LDS row of each patch column.
@@ -1488,7 +1433,7 @@ __global__ __launch_bounds__(256) void k_gather_tile(
   // r0 - (BS-1) + i clamped to [0, n1], column c0 - (BS-1) + lc), all 0 for
   // columns outside the frame (empty buckets).  A voxel's bounds are then
   // cells at fixed offsets from one per-thread base.
-  __shared__ T sB[M * RS];
+  __shared__ double sB[M * RS];
   __shared__ int32_t sT[NC * NRW];
   __shared__ int32_t sP[NC];
   __shared__ double sm[5][4];
@@ -1515,11 +1460,11 @@ __global__ __launch_bounds__(256) void k_gather_tile(
   // at Ws + id * fstride + r * M (W^T) and v_r[k] at Vk + id * fstride +
   // r * sr (V^T)
   const uint32_t sr = (nw + 3) & ~3u;
-  const T* W0k = W0 + ((size_t)b * nw + k) * p_sel * M;
-  const T* Sk = S01 + ((size_t)b * nw + k) * p_sel * 2;
-  const T* Ds = dr + (size_t)slot * p_sel * nw;
-  const T* Vk = factors + (size_t)b * nvar_stored * p_sel * fstride + k;
-  const T* Ws = factors + (size_t)b * nvar_stored * p_sel * fstride + nw * sr;
+  const double* W0k = W0 + ((size_t)b * nw + k) * p_sel * M;
+  const double* Sk = S01 + ((size_t)b * nw + k) * p_sel * 2;
+  const double* Ds = dr + (size_t)slot * p_sel * nw;
+  const double* Vk = factors + (size_t)b * nvar_stored * p_sel * fstride + k;
+  const double* Ws = factors + (size_t)b * nvar_stored * p_sel * fstride + nw * sr;
   // the voxel's 1/W and U are independent of the staging: load them first
   const uint32_t pix = (uint32_t)min(r, (int)nr - 1) + nr * (uint32_t)min(c, (int)nr - 1), v = k * fs + pix;
   const double iw = invw[(size_t)b * vol + v];
@@ -1552,20 +1497,18 @@ __global__ __launch_bounds__(256) void k_gather_tile(
     if ((int)threadIdx.x == lc) sP[lc] = pre[lc];
   if (fits) {
     // the tile's rows in LDS order (row R of column lc is bucket place
-    // sT[lc][0] + R - pre[lc]): thread -> (rows lr0 + RPI s, values q ..
-    // q + W - 1), NS slots.  Every row's loads are issued first, then every
-    // row is formed.
-    constexpr int QW = M / W, RPI = 256 / QW, NS = (TOT + RPI - 1) / RPI;
-    const int lr0 = (int)threadIdx.x / QW, q = ((int)threadIdx.x % QW) * W;
+    // sT[lc][0] + R - pre[lc]): thread -> (rows lr0 + RPI s, value q), NS
+    // slots.  Every row's loads are issued first, then every row is formed.
+    constexpr int RPI = 256 / M, NS = (TOT + RPI - 1) / RPI;
+    const int lr0 = (int)threadIdx.x / M, q = (int)threadIdx.x % M;
     const int tot = pre[NC];
     // Every load of a row is at its bucket place (the patch index, the
-    // thread's values of the static row, the singular pair), issued for
+    // thread's value of the static row, the singular pair), issued for
     // every row before the first use; further ranks are read as needed.
     // Row value q: d_0 (w_0[q] v_0[k]), then the FMA chain of the
     // reconstruction over the further kept ranks, fma(d_r w_r[q], v_r[k], .).
     int32_t ids[NS];
-    ST w0[NS];
-    T s0[NS], s1[NS];
+    double w0[NS], s0[NS], s1[NS];
 #pragma unroll
     for (int sl = 0; sl < NS; ++sl) {
       const int R = lr0 + RPI * sl;
@@ -1580,37 +1523,26 @@ __global__ __launch_bounds__(256) void k_gather_tile(
         base = after ? pre[cc] : base;
       }
       const int32_t j = use ? sT[lc * NRW] + (R - base) : 0;
-      w0[sl] = *reinterpret_cast<const ST*>(W0k + (size_t)j * M + q);
+      w0[sl] = W0k[(size_t)j * M + q];
       ids[sl] = use ? Lk[j] : -1;
       s0[sl] = Sk[2 * (size_t)j];
       s1[sl] = Sk[2 * (size_t)j + 1];
     }
 #pragma unroll
     for (int sl = 0; sl < NS; ++sl) {
-      {
-        const T d0 = shrink_factor(s0[sl], s0[sl], lam, exp_w), d1 = shrink_factor(s1[sl], s0[sl], lam, exp_w);
-        if (ids[sl] >= 0) {
-          const int32_t id = ids[sl];
-          ST row;
-          T* ac = reinterpret_cast<T*>(&row);
-          const T* ww = reinterpret_cast<const T*>(&w0[sl]);
-#pragma unroll
-          for (int w = 0; w < W; ++w) ac[w] = (d0 > T(0)) ? d0 * ww[w] : T(0);
-          if (d1 > T(0)) {
-            for (int rk = 1; rk < (int)nw; ++rk) {
-              const T d = Ds[(size_t)id * nw + rk];
-              if (!(d > T(0))) break;
-              const T vk = Vk[(size_t)id * fstride + (size_t)rk * sr];
-              const ST wv = *reinterpret_cast<const ST*>(Ws + (size_t)id * fstride + (size_t)rk * M + q);
-              const T* wk = reinterpret_cast<const T*>(&wv);
-#pragma unroll
-              for (int w = 0; w < W; ++w) ac[w] = fma(d * wk[w], vk, ac[w]);
-            }
+      const double d0 = shrink_factor(s0[sl], s0[sl], lam, exp_w), d1 = shrink_factor(s1[sl], s0[sl], lam, exp_w);
+      if (ids[sl] >= 0) {
+        const int32_t id = ids[sl];
+        double row = (d0 > 0.0) ? d0 * w0[sl] : 0.0;
+        if (d1 > 0.0) {
+          for (int rk = 1; rk < (int)nw; ++rk) {
+            const double d = Ds[(size_t)id * nw + rk];
+            if (!(d > 0.0)) break;
+            const double vk = Vk[(size_t)id * fstride + (size_t)rk * sr];
+            row = fma(d * Ws[(size_t)id * fstride + (size_t)rk * M + q], vk, row);
           }
-          const int R = lr0 + RPI * sl;
-#pragma unroll
-          for (int w = 0; w < W; ++w) sB[(q + w) * RS + R] = ac[w];
         }
+        sB[q * RS + lr0 + RPI * sl] = row;
       }
     }
   }
@@ -1639,8 +1571,8 @@ __global__ __launch_bounds__(256) void k_gather_tile(
           const int32_t j0 = bnd[cb][e], n = bnd[cb][e + 1] - j0;
           // an empty bucket reads the first row of the next bucket or the
           // plane's pad element: in bounds, and not added
-          const T f = sB[(ra + BS * cb) * RS + j0 + base[cb]];
-          acc += (double)((n > 0) ? f : T(0));
+          const double f = sB[(ra + BS * cb) * RS + j0 + base[cb]];
+          acc += (n > 0) ? f : 0.0;
           multi = multi || n > 1;
         }
       }
@@ -1651,7 +1583,7 @@ __global__ __launch_bounds__(256) void k_gather_tile(
           for (int ra = 0; ra < BS; ++ra) {
             const int e = BS - 1 - ra;
             for (int32_t j = bnd[cb][e] + 1; j < bnd[cb][e + 1]; ++j)
-              acc += (double)sB[(ra + BS * cb) * RS + j + base[cb]];
+              acc += sB[(ra + BS * cb) * RS + j + base[cb]];
           }
         }
       }
@@ -1664,18 +1596,18 @@ __global__ __launch_bounds__(256) void k_gather_tile(
           for (int32_t j = bnd[cb][e]; j < bnd[cb][e + 1]; ++j) {
             // element qv of the patch's row, formed as in the staging
             const int32_t id = Lk[j];
-            const T sa = Sk[2 * (size_t)j], sb = Sk[2 * (size_t)j + 1];
-            const T d0 = shrink_factor(sa, sa, lam, exp_w);
-            T x = (d0 > T(0)) ? d0 * W0k[(size_t)j * M + qv] : T(0);
-            if (shrink_factor(sb, sa, lam, exp_w) > T(0)) {
+            const double sa = Sk[2 * (size_t)j], sb = Sk[2 * (size_t)j + 1];
+            const double d0 = shrink_factor(sa, sa, lam, exp_w);
+            double x = (d0 > 0.0) ? d0 * W0k[(size_t)j * M + qv] : 0.0;
+            if (shrink_factor(sb, sa, lam, exp_w) > 0.0) {
               for (int rk = 1; rk < (int)nw; ++rk) {
-                const T d = Ds[(size_t)id * nw + rk];
-                if (!(d > T(0))) break;
+                const double d = Ds[(size_t)id * nw + rk];
+                if (!(d > 0.0)) break;
                 x = fma(d * Ws[(size_t)id * fstride + (size_t)rk * M + qv], Vk[(size_t)id * fstride + (size_t)rk * sr],
                         x);
               }
             }
-            acc += (double)x;
+            acc += x;
           }
         }
     }
@@ -1763,7 +1695,7 @@ hipError_t launch_static_rows(const void* factors, const int32_t* place, uint32_
   const dim3 grid((uint32_t)(((size_t)sh.p_sel * sh.nw * 4 + 255) / 256), nb);
 #define PG_SR(B)                                                                                                 \
   case B:                                                                                                      \
-    hipLaunchKernelGGL((k_static_rows<B, double>), grid, dim3(256), 0, s, (const double*)factors, place,         \
+    hipLaunchKernelGGL((k_static_rows<B>), grid, dim3(256), 0, s, (const double*)factors, place,         \
                        nvar_stored, sh.p_sel, sh.nw, sh.fstride, (double*)W0, (double*)S01);                    \
     return hipGetLastError();
   switch (sh.bs) {
@@ -1874,7 +1806,7 @@ hipError_t launch_eval(const void* factors, const WinMeta* meta, const uint32_t*
 #define PG_EV(B, N, L, LS)                                                                                       \
   if constexpr (L == 64) {                                                                                     \
     if (sh.bs == B && sh.nw == N) {                                                                            \
-      hipLaunchKernelGGL((k_eval<B, N, L, double>), dim3(nblk, na), dim3(256), 0, s, (const double*)factors,    \
+      hipLaunchKernelGGL((k_eval<B, N, L>), dim3(nblk, na), dim3(256), 0, s, (const double*)factors,    \
                          meta, wl, nvar_stored, nvar_run, sh.p_sel, sh.nw, sh.fstride, exp_w,                   \
                          (const double*)divq, inv, (double*)B0, partial, slot_lam, kept);                      \
       return hipGetLastError();                                                                                \
@@ -1940,14 +1872,14 @@ hipError_t launch_gather(const GatherSrc& src, const int32_t* off, const double*
   if (!sh.fp64) return hipErrorInvalidValue;  // launch_overlap
 #define PG_GT(B)                                                                                                 \
   case B:                                                                                                      \
-    hipLaunchKernelGGL((k_gather_tile<B, double>), dim3(nblk, na), dim3(256), 0, s, (const double*)src.factors,  \
+    hipLaunchKernelGGL((k_gather_tile<B>), dim3(nblk, na), dim3(256), 0, s, (const double*)src.factors,  \
                        (const double*)src.dr, (const double*)src.S01, (const double*)src.W0, src.list, off,     \
                        invw, u64, meta, wl, src.slot_lam, src.exp_w, sh.nr, sh.fs, sh.nw, sh.vol, sh.n1,        \
                        sh.p_sel, sh.fstride, src.nvar_stored, mode, nkk, out, partial);                         \
     break;
 #define PG_GA(B)                                                                                                 \
   case B:                                                                                                      \
-    hipLaunchKernelGGL((k_gather_direct<B, double>), dim3(nblk, na), dim3(256), 0, s, (const double*)src.B0, off, \
+    hipLaunchKernelGGL((k_gather_direct<B>), dim3(nblk, na), dim3(256), 0, s, (const double*)src.B0, off, \
                        invw, u64, meta, wl, sh.nr, sh.fs, sh.nw, sh.vol, sh.n1, sh.p_sel, mode, out, partial);   \
     break;
   switch (sh.bs) {

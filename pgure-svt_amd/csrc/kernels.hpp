@@ -59,10 +59,10 @@ uint32_t svd_lanes(uint32_t bs, uint32_t nw, int mapping);
 // inv [nb][nw][p_sel]: bucket-sorted place of every patch
 hipError_t launch_buckets(const int32_t* pos, const uint32_t* sel, uint32_t nb, const Shape& sh, int32_t* cnt,
                           int32_t* off, int32_t* list, int32_t* inv, hipStream_t s);
-// 1/W and delta2/W per voxel, [nb][vol] (dw may be null)
+// 1/W and delta2/W per voxel, [nb][vol] (dw may be null); FP64 only
 hipError_t launch_weights(const int32_t* off, const uint8_t* d2, uint32_t nb, const Shape& sh, double d2neg,
                           double d2pos, double* invw, void* dw, hipStream_t s);
-// one lambda evaluation of the listed slots; B0 [na][nw][p_sel][m] (rows in
+// one lambda evaluation of the listed slots (FP64, patches above 4 x 4); B0 [na][nw][p_sel][m] (rows in
 // bucket order); partial [na][eval_blocks] (divergence sums, only with
 // nvar_run == 3, which needs divq); kept (optional, nvar_run == 3):
 // [na][eval_blocks] kept ranks of each block
@@ -72,9 +72,10 @@ hipError_t launch_eval(const void* factors, const WinMeta* meta, const uint32_t*
                        const int32_t* inv, void* B0, double* partial, hipStream_t s,
                        const double* slot_lam = nullptr, double* kept = nullptr);
 // divergence factors w_r^T D v_r of every rank of every (patch, variant),
-// D the patch's delta2/W along its trajectory (dw), after the SVD: divq
-// [nb][p_sel][nvar][2][sr] (sr = nw rounded up to 4), per (patch, variant)
-// its singular values (zero-padded) then its factors
+// D the patch's delta2/W along its trajectory (dw), after the SVD: the
+// singular values (zero-padded to sr = nw rounded up to 4), then the factors,
+// as planes divq [nb][nvar][2][sr][p_sel], or for FP64 patches above 4 x 4
+// [nb][p_sel][nvar][2][sr]
 hipError_t launch_divq(const void* factors, const int32_t* pos, const uint32_t* sel, const void* dw, uint32_t nb,
                        uint32_t nvar, const Shape& sh, void* divq, hipStream_t s);
 // FP32, and patches up to 4 x 4 in FP64, evaluate lambda in two launches: launch_round_prep

@@ -187,16 +187,17 @@ __global__ __launch_bounds__(256) void k_cover(const int2* __restrict__ recs, co
   for (int o = 32; o > 0; o >>= 1) most = max(most, __shfl_xor(most, o));
   if (threadIdx.x % 64 == 0) wmax[threadIdx.x / 64] = most;
   __syncthreads();
-  if (threadIdx.x == 0) atomicMax(&wstat[b * (2 + nw) + 2 + k], (uint32_t)max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3])));
+  if (threadIdx.x == 0)
+    atomicMax(&wstat[b * (2 + nw) + 2 + k], (uint32_t)max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3])));
 }
 
 // ---------------------------------------------------- leading vectors --
 // By patch, from the U variant's factors: w_0 (w0 [nb][p_sel][m], may be
-// null) and v_0 as
-// one plane per frame (v0 [nb][nw][p_sel]), and the window's largest finite
-// s_0 and the complement of its smallest above 0 (wstat[b (2 + nw)] and the
-// next word, as the bits of a float).  A workgroup takes 64 patches: 16 lanes read a patch's vectors, v_0 turns in LDS, so that
-// both sides move whole lines.
+// null) and v_0 as one plane per frame (v0 [nb][nw][p_sel]), and the window's
+// largest finite s_0 and the complement of its smallest above 0 (wstat[b (2 +
+// nw)] and the next word, as the bits of a float).  A workgroup takes 64
+// patches: 16 lanes read a patch's vectors, v_0 turns in LDS, so that both
+// sides move whole lines.
 __global__ __launch_bounds__(256) void k_lead(const float* __restrict__ factors, uint32_t nvar_stored, uint32_t p_sel,
                                               uint32_t nw, uint32_t m, uint32_t fstride, float* __restrict__ w0,
                                               float* __restrict__ v0, uint32_t* __restrict__ wstat) {
