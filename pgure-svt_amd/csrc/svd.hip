@@ -84,6 +84,25 @@ struct Sweep {
     return t;
   }
   static constexpr Table kTable = make();
+  // every pair once, each column's partners in ascending order, no column
+  // twice in a group
+  static constexpr bool sound() {
+    int last[N] = {}, pairs = 0;
+    for (int c = 0; c < N; ++c) last[c] = -1;
+    for (int g = 0; g < kTable.groups; ++g) {
+      const PairGroup& q = kTable.g[g];
+      if (q.n < 1 || q.n > 4) return false;
+      for (int z = 0; z < q.n; ++z, ++pairs) {
+        const int i = q.i[z], k = q.j[z];
+        if (i < 0 || i >= k || k >= N || k <= last[i] || i <= last[k]) return false;
+        for (int y = 0; y < z; ++y)
+          if (q.i[y] == i || q.j[y] == i || q.i[y] == k || q.j[y] == k) return false;
+        last[i] = k;
+        last[k] = i;
+      }
+    }
+    return pairs == N * (N - 1) / 2;
+  }
 };
 template <class F, int... G>
 __device__ __forceinline__ void for_all(std::integer_sequence<int, G...>, F&& f) {
@@ -103,7 +122,7 @@ __device__ __forceinline__ void rotate1(float& xi, float& xj, float cs, float sn
       "v_mul_f32 %1, %3, %1\n\t"
       "v_fmac_f32 %1, %4, %0\n\t"
       "v_fma_f32 %0, %3, %0, -%2"
-      : "+v"(xi), "+v"(xj), "=&v"(t)
+      : "+&v"(xi), "+&v"(xj), "=&v"(t)
       : "v"(cs), "v"(sn));
 }
 __device__ __forceinline__ void rotate2(float& xi, float& xj, float& yi, float& yj, float cs, float sn) {
@@ -116,7 +135,7 @@ __device__ __forceinline__ void rotate2(float& xi, float& xj, float& yi, float& 
       "v_fmac_f32 %3, %7, %2\n\t"
       "v_fma_f32 %0, %6, %0, -%4\n\t"
       "v_fma_f32 %2, %6, %2, -%5"
-      : "+v"(xi), "+v"(xj), "+v"(yi), "+v"(yj), "=&v"(t), "=&v"(u)
+      : "+&v"(xi), "+&v"(xj), "+&v"(yi), "+&v"(yj), "=&v"(t), "=&v"(u)
       : "v"(cs), "v"(sn));
 }
 __device__ __forceinline__ void rotate1(double& xi, double& xj, double cs, double sn) {
@@ -287,6 +306,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(svd_min_wav
     // 152 -> 130); 7 columns have two pairs to a group (16 x 7, 31 M: 25.9 ms a
     // pair at a time, 26.1 in groups).
     if constexpr (quads<N, L, T>() && !RT) {
+      static_assert(Sweep<N>::sound(), "a pair missing, repeated or out of order");
       for_all(std::make_integer_sequence<int, Sweep<N>::kTable.groups>{}, quad);
     } else {
 #pragma unroll
