@@ -1630,23 +1630,25 @@ constexpr uint32_t kFeatureSamples = 256;
 
 // Where all three parameters are given, no method but the first (which
 // refuses a window of too few leaves) takes anything from the leaves: none are
-// formed (99 x 99 x 23 of u8, windows of 9, 16 threads: 5.4 ms a call with
-// them, 3.6 without).
+// formed (99 x 99 x 23 of u8, windows of 9, 16 threads: 3.8 ms a call; 4.0 to
+// 4.7 with them).
 bool leaves_needed(double alpha, double mu, double sigma, uint32_t method) {
   return !(alpha >= 0.0 && mu >= 0.0 && sigma >= 0.0) || method == 1;
 }
 
 // Where the leaf statistics of the noise estimator are formed (the results
-// are the same bit for bit).  The host threads cost the GPU nothing while it
-// decomposes: about 60 ns a value and thread (distinct (frame,
-// normalisation) pairs x pixels) against the decomposition's 0.85 ns a
-// matrix and its 14 m n^2 + 8 n^3 flops at 25 TFLOP/s (256 x 256 x 100: the
-// call takes 116 ms with the host's, 119 with the GPU's, whose leaves share
-// the SIMDs with the SVD).  Where they would end after it, the GPU
-// forms them (512 x 512 x 40, windows of 7: 101 ms with the host's, 91 with
-// the GPU's; 128 x 128 x 30 over a grid, whose rounds run on: 24.3 with the
-// host's, 24.7 with the GPU's).  Below 2^18 values the host is done first
-// (64 x 64 x 20: 3.7 against 4.4 ms).
+// are the same bit for bit).  The host threads, about 60 ns a value and thread
+// (distinct (frame, normalisation) pairs x pixels), cost the GPU nothing while
+// it works; on the GPU the leaves share the SIMDs with the SVD.  So the host
+// keeps them up to a line of 0.85 ns a matrix and its 14 m n^2 + 8 n^3 flops at
+// 25 TFLOP/s, which lies above the decomposition itself (256 x 256 x 100: 76 ms
+// against 45): windows join the search as their estimates come, and need not
+// all be there when it starts.  Calls with the host's and with the GPU's, 16
+// threads: 256 x 256 x 100 (the host at 0.9 of the line) 92-95 and 101 ms; 128 x
+// 128 x 50 of u16 20.1-20.9 and 20.5-22.4; 512 x 512 x 40 in windows of 7 (past
+// the line) 96-108 and 82; 128 x 128 x 30 over a grid, whose rounds run on, 23.9
+// and 23.9-24.1.  Below 2^18 values the host is done first (64 x 64 x 20: 3.6
+// against 4.1 ms).
 bool leaves_on_gpu_pay(uint64_t values, uint32_t threads, double matrices, const Shape& sh) {
   if (values < ((uint64_t)1 << 18)) return false;
   const double host = 60e-9 * (double)values / threads;

@@ -287,8 +287,8 @@ __device__ __forceinline__ void load_run(const float* __restrict__ p, float (&x)
 // the columns of one class (by the sum of their finite |x|) and finds the
 // largest below it; the classes' sums are added from the largest down.  Every
 // column is held to 2^-25 of its own |x|, in any order, and a strip costs a few
-// walks (256 x 256 x 3, half of it 1e-20 of the rest, plain threshold 0: 0.16 ms
-// a lambda, 0.05 where no strip comes here; a walk of the strip's records for
+// walks (256 x 256 x 3, half of it 1e-20 of the rest, plain threshold 0: 0.25 ms
+// a lambda, 0.08 where no strip comes here; a walk of the strip's records for
 // each cell that is not finite 6.4).  The sums between the classes stay in
 // registers, kCellsHeld a thread, so a strip of more cells takes its parts one
 // after the other; and the cells' places are worked out anew at each use:
@@ -392,9 +392,10 @@ __device__ __forceinline__ void sum_by_magnitude(unsigned long long* acc, const 
 // in a window of wider s_0, one whose |x| sum to less than 2^24 q, are
 // summed again by magnitude (sum_by_magnitude).
 //
-// Bound: instruction issue (333 vector instructions per 64 voxels, 16.6 of
-// 28.4 ms) and the LDS atomics (10.7 ms), then memory (28 bytes a voxel).
-// 256 x 256 x 15 windows at searched lambdas: 13.5 ps a voxel.  The
+// Bound: instruction issue (355 vector instructions per 64 voxels, 17.1 of the
+// 26.0 ms of 1.9 G voxels) and the LDS atomics (about 10 ms), then memory (28
+// bytes a voxel).  256 x 256 x 15 windows at searched lambdas: 13.7 ps a voxel.
+// The
 // form before (rows of a 32 x 8 tile staged in LDS from bucket-sorted rows,
 // each voxel reading its 16 positions and looping over further patches of a
 // position) issued 1,197 vector instructions per 64 voxels, at 4 cycles each
