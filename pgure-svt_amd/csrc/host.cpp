@@ -1938,11 +1938,15 @@ int run_core(const void* X, int dtype, uint32_t nr, uint32_t nc, uint32_t nf, co
             // are the same
             (void)hipGetLastError();
             std::atomic<size_t> next{done};
+            auto work = [&] {
+              for (size_t j; (j = next.fetch_add(1)) < leaf_jobs.size();) host_leaves(*leaf_jobs[j]);
+            };
             std::vector<std::thread> th;
-            for (uint32_t k = 0; k < threads; ++k)
-              th.emplace_back([&] {
-                for (size_t j; (j = next.fetch_add(1)) < leaf_jobs.size();) host_leaves(*leaf_jobs[j]);
-              });
+            try {
+              for (uint32_t k = 1; k < threads; ++k) th.emplace_back(work);
+            } catch (...) {  // no more threads: those there are enough
+            }
+            work();
             for (auto& x : th) x.join();
           }
           queued->set();
